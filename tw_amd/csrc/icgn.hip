@@ -11,8 +11,9 @@
 // FP32 dp with the norm evaluated in FP64 as the reference's pow() does.
 //
 // Per-iteration work stays in registers:
-//   * each lane of a POI's group of L lanes walks pixels l, l+L, ...
-//     (l = lane % L) of the (2Sy+1)x(2Sx+1) subset;
+//   * the lanes of a POI's group walk down columns of the (2Sy+1)x(2Sx+1)
+//     subset (StripPlan), so what depends on the column alone is formed once
+//     per column and the x and y weights of the sums come at no cost per pixel;
 //   * one pass forms sum T, sum T^2 and the six sums SD_k T in FP64 (every
 //     FP32 product SD_k T is exact in FP64), so the residual vector is
 //       RHS_k = (R_s/T_s) (sum SD_k T - mean(T) A_k) - B_k
@@ -68,15 +69,6 @@ __device__ __forceinline__ bool group_any(bool pred, int lane)
     const unsigned long long b = __ballot(pred);
     if constexpr (L == 64) return b != 0ull;
     return (uint32_t)((lane & 32) ? (b >> 32) : b) != 0u;
-}
-
-// Warp coordinate exactly as the CPU path evaluates it (:618-619, :761-762):
-// ((POI + W0*dx) + W1*dy) + W2, every product and sum rounded to FP32 (the
-// pragma keeps the compiler from fusing a product into the following sum).
-__device__ __forceinline__ float warp_coord(float poi, float w0, float w1, float w2, float dx, float dy)
-{
-#pragma clang fp contract(off)
-    return ((poi + w0 * dx) + w1 * dy) + w2;
 }
 
 // Bicubic value from the materialised LUT cell (16 floats, 4k+l ~ y^k x^l).
@@ -331,28 +323,34 @@ __device__ __forceinline__ void kahan_pixel(float ks[8], float kc[8], float T, u
     }
 }
 
-// The subset's pixels in row-major order, p = l * Wsub + m: the exact float
-// offsets dx = m - Sx, dy = l - Sy and the byte offset 4 (l * rw + m) into
-// the gradient plane from the subset's corner.  Every POI of a launch has the
-// same subset and ROI width, so one table in LDS serves a workgroup's eight
-// POIs, and a lane's step to its next pixel is an LDS read instead of
-// float compares and selects.  The three arrays have the same 4-byte stride,
-// so one address register reaches all of them (the array offsets are
-// immediates of the LDS reads).
-constexpr int kStepTable = 2048;          // pixels: subsets up to 45 x 45
-struct StepTable {
-    float dx[kStepTable];
-    float dy[kStepTable];
-    uint32_t go[kStepTable];
+// A lane's share of a strip (StripPlan): the exact float offsets of its first
+// pixel from the POI, that pixel's byte offset in the gradient plane from the
+// subset's corner, and its row count (low half; 0: the lane has no share) with
+// the rows that every share of the strip has at least (high half).  Every POI
+// of a launch has the same subset and ROI width, so one table in LDS serves a
+// workgroup.
+struct StripLane {
+    float dx, dy;
+    uint32_t go;
+    uint32_t rows;
 };
 
-__device__ __forceinline__ void fill_step_table(StepTable& t, const IcgnParams& P)
+template <int L>
+__device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P, int t0, int tstride)
 {
-    for (int p = threadIdx.x; p < P.s; p += blockDim.x) {
-        const int l = p / P.Wsub, m = p - l * P.Wsub;
-        t.dx[p] = (float)(m - P.Sx);
-        t.dy[p] = (float)(l - P.Sy);
-        t.go[p] = 4u * (uint32_t)(l * P.rw + m);
+    // constant strip indices: a run-time index would move the plan to scratch
+#pragma unroll
+    for (int k = 0; k < kMaxStrips; ++k) {
+        if (k >= P.strips.count) break;
+        const Strip s = P.strips.s[k];
+        const int base = P.Hsub / s.segs, rem = P.Hsub - base * s.segs;
+        for (int l = t0; l < L; l += tstride) {
+            const int seg = l / s.ncol, m = s.col + l - seg * s.ncol;
+            const int y = seg * base + min(seg, rem);
+            const int rows = seg < s.segs ? base + (seg < rem ? 1 : 0) : 0;
+            tab[k * L + l] = {(float)(m - P.Sx), (float)(y - P.Sy), 4u * (uint32_t)(y * P.rw + m),
+                              (uint32_t)rows | ((uint32_t)base << 16)};
+        }
     }
 }
 
@@ -361,21 +359,33 @@ __device__ __forceinline__ void fill_step_table(StepTable& t, const IcgnParams& 
 // first pass at integer target pixels (:610-637); otherwise bicubic
 // (:757-792).  Returns false when a warped pixel of the group's POI leaves the
 // ROI.  Accumulates sum T, sum T^2 and the six sum SD_k T / 2 (the gradient
-// plane stores 2 Rx, 2 Ry) in FP64.  With a step table (tab != null) the lanes
-// take pixels hl + L k from it: s / L full rounds, then the s % L remaining pixels;
-// without one they step their offsets in registers.  Each lane visits the
-// same pixels in the same order either way, so the sums are identical.  RP:
-// the fused bicubic passes evaluate the target's row polynomials (P.rp)
-// instead of the image bytes.  UNR: pixels per trip of the step-table loop.
-template <int L, int INTERP, bool INT, bool CHECK, bool TABLE, bool RP, bool K32 = false, int UNR = 1>
+// plane stores 2 Rx, 2 Ry) in FP64.  RP: the fused bicubic passes evaluate the
+// target's row polynomials (P.rp) instead of the image bytes.
+//
+// Each lane walks down one column at a time.  Along a column dx is constant,
+// so POI + W0 dx is formed once, the gradient offset of the next row is a
+// scalar add, and of the sums only S = sum g T needs a product per pixel: the
+// dx-weighted sum is dx S, and the dy-weighted one follows from the running
+// sums, sum_i i g_i T_i = m S - sum_i S_i over m rows (S_i the running sum
+// after row i: Abel's summation by parts).  S runs on from strip to strip;
+// what it held when a strip began is taken out again (a1, a2 below).  Where T
+// is integer-valued every term is an integer below 2^53, so these sums stay
+// exact there, as direct ones would be.
+//
+// Bound by VALU issue (79 % of the slots on the 2048^2 frame, 157,609 POIs of
+// 41x41) with the texture-address unit close behind (74 %).  Against a walk in
+// row-major order from a table of pixel offsets: 47 VALU instructions per
+// bicubic pixel (58) and 16 per integer one (26), 1.20 ms (1.35 ms); 14k POIs
+// on whole wavefronts 0.139 ms (0.153).  One row per trip: two or four took
+// 1.27 and 1.28 ms.
+template <int L, int INTERP, bool INT, bool CHECK, bool RP, bool K32 = false>
 __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py, const float Wm[6], int lane,
-                                            double acc[8], const StepTable* tab)
+                                            double acc[8], const StripLane* tab)
 {
     const int hl = lane & (L - 1);
     // the fused interpolation from the bytes returns T 2^-24 (interp_rows_s);
     // the sums are scaled back at the end, exactly
     constexpr bool SCALED = !INT && INTERP == TWDIC_INTERP_FUSED && !RP;
-    const int Sx = P.Sx, Sy = P.Sy, Wsub = P.Wsub, s = P.s;
     const int sx0 = P.sx0, sy0 = P.sy0, rw = P.rw, rh = P.rh;
     const TargetBuf tb = target_buf(P);
     const __amdgpu_buffer_rsrc_t g2r =
@@ -385,18 +395,27 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     double st = 0.0, stt = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0, b0 = 0.0, b1 = 0.0, b2 = 0.0;
     float ks[8] = {}, kc[8] = {};
     bool out = false;
-    auto pixel = [&](float dx, float dy, uint32_t go, int goff) {
+    // byte offset of the subset's corner pixel in the gradient plane
+    const uint32_t gcorner = 4u * (uint32_t)((py - P.Sy - sy0) * rw + (px - P.Sx - sx0));
+    // cx, cy: the column's share of the warped coordinates; go + so: the
+    // pixel's byte offset in the gradient plane (so is wave-uniform)
+    auto pixel = [&](float cx, float cy, float dx, float dy, uint32_t go, int so) {
         float wx, wy;
-        if constexpr (INT) {
-            // the first pass's warp is W = [[1, 0, u], [0, 1, v]] exactly, where
-            // ((POI + 1 dx) + 0 dy) + u = (POI + dx) + u bit for bit (POI + dx
-            // is a non-zero integer, so adding the zero product changes nothing)
+        {
 #pragma clang fp contract(off)
-            wx = (fpx + dx) + Wm[2];
-            wy = (fpy + dy) + Wm[5];
-        } else {
-            wx = warp_coord(fpx, Wm[0], Wm[1], Wm[2], dx, dy);
-            wy = warp_coord(fpy, Wm[3], Wm[4], Wm[5], dx, dy);
+            if constexpr (INT) {
+                // the first pass's warp is W = [[1, 0, u], [0, 1, v]] exactly, where
+                // ((POI + 1 dx) + 0 dy) + u = (POI + dx) + u bit for bit (POI + dx
+                // is a non-zero integer, so adding the zero product changes nothing)
+                wx = cx + Wm[2];
+                wy = (fpy + dy) + Wm[5];
+            } else {
+                // as the CPU path evaluates it (:618-619, :761-762): ((POI + W0*dx) +
+                // W1*dy) + W2, every product and sum rounded to FP32 (the pragma keeps
+                // the compiler from fusing a product into the following sum)
+                wx = (cx + Wm[1] * dy) + Wm[2];
+                wy = (cy + Wm[4] * dy) + Wm[5];
+            }
         }
         const int ix = (int)wx, iy = (int)wy;          // truncation, as int()
         float T = 0.f;
@@ -420,65 +439,55 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                 T = interp_lut(P.lut, (uint32_t)((iy - sy0) * rw + (ix - sx0)), tx, ty);
             }
         }
-        const uint32_t g = __builtin_amdgcn_raw_buffer_load_b32(g2r, (int)go + goff, 0, 0);
+        const uint32_t g = __builtin_amdgcn_raw_buffer_load_b32(g2r, (int)go, so, 0);
         if constexpr (K32) {
             kahan_pixel(ks, kc, T, g, dx, dy);
             return;
         }
-        // FP64: every product SD_k T is exact, and where T takes integer values
+        // FP64: every product g T is exact, and where T takes integer values
         // (the integer pass, uniform target regions) the sums are exact, so
         // T = R gives an exactly zero update and near-flat subsets, whose
         // residual is scaled by the large R_s / T_s, see no rounding there
         const double gx = (double)(int16_t)(g & 0xffffu), gy = (double)(int16_t)(g >> 16);
-        const double Td = T, ddx = dx, ddy = dy;
+        const double Td = T;
         st += Td;
         stt = fma(Td, Td, stt);
-        const double a = gx * Td, b = gy * Td;
-        a0 += a;
-        a1 = fma(a, ddx, a1);
-        a2 = fma(a, ddy, a2);
-        b0 += b;
-        b1 = fma(b, ddx, b1);
-        b2 = fma(b, ddy, b2);
+        a0 = fma(gx, Td, a0);
+        a2 -= a0;
+        b0 = fma(gy, Td, b0);
+        b2 -= b0;
     };
-    // byte offset of the subset's corner pixel in the gradient plane
-    const int gcorner = 4 * ((py - Sy - sy0) * rw + (px - Sx - sx0));
-    if constexpr (TABLE) {
-        const int full = s / L;
-        // with UNR = 2 two pixels' loads are in flight together
-#pragma unroll UNR
-        for (int k = 0; k < full; ++k) {
-            const int p = hl + L * k;
-            pixel(tab->dx[p], tab->dy[p], tab->go[p], gcorner);
-        }
-        const int p = hl + L * full;
-        if (p < s) {
-            pixel(tab->dx[p], tab->dy[p], tab->go[p], gcorner);
-        }
-    } else {
-        // lane walks pixels p = hl, hl + L, ...: column
-        // m = p % Wsub, row l = p / Wsub, kept as the exact float offsets
-        // dx = m - Sx, dy = l - Sy and the 32-bit byte offset into the
-        // gradient plane
-        const int qL = L / Wsub, rL = L - qL * Wsub;
-        // recomputed per pass: kept live across the iteration loop, this start
-        // state is what the register allocator spills
-        int lane_v = hl;
-        asm volatile("" : "+v"(lane_v));
-        const int l0 = lane_v / Wsub, m0 = lane_v - l0 * Wsub;
-        float dx = (float)(m0 - Sx), dy = (float)(l0 - Sy);
-        uint32_t go = (uint32_t)gcorner + 4u * (uint32_t)(l0 * rw + m0);
-        const float fSx = (float)Sx, fWsub = (float)Wsub, frL = (float)rL, fqL = (float)qL;
-        const uint32_t gstep = 4u * (uint32_t)(qL * rw + rL), gwrap = 4u * (uint32_t)(rw - Wsub);
+    const int nstrips = P.strips.count;
 #pragma unroll 1
-        for (int p = hl; p < s; p += L) {
-            pixel(dx, dy, go, 0);
-            // next pixel of this lane: L further in row-major subset order
-            dx += frL;
-            const bool wrap = dx > fSx;
-            dx = wrap ? dx - fWsub : dx;
-            dy += wrap ? fqL + 1.f : fqL;
-            go += wrap ? gstep + gwrap : gstep;
+    for (int k = 0; k < nstrips; ++k) {
+        const StripLane e = tab[k * L + hl];
+        const int full = __builtin_amdgcn_readfirstlane((int)(e.rows >> 16)), rows = (int)(e.rows & 0xffffu);
+        if (rows > 0) {
+            const uint32_t go = gcorner + e.go;
+            const double ddx = (double)e.dx, ddy = (double)e.dy;
+            a1 = fma(-ddx, a0, a1);
+            a2 = fma(-ddy, a0, a2);
+            b1 = fma(-ddx, b0, b1);
+            b2 = fma(-ddy, b0, b2);
+            float cx, cy, dy = e.dy;
+            {
+#pragma clang fp contract(off)
+                cx = INT ? fpx + e.dx : fpx + Wm[0] * e.dx;
+                cy = INT ? 0.f : fpy + Wm[3] * e.dx;
+            }
+            int so = 0;
+#pragma unroll 1
+            for (int r = 0; r < full; ++r) {
+                pixel(cx, cy, e.dx, dy, go, so);
+                dy += 1.f;
+                so += 4 * rw;
+            }
+            if (rows > full) pixel(cx, cy, e.dx, dy, go, so);
+            const double end = ddy + (double)rows;
+            a1 = fma(ddx, a0, a1);
+            a2 = fma(end, a0, a2);
+            b1 = fma(ddx, b0, b1);
+            b2 = fma(end, b0, b2);
         }
     }
     // 2^24 and 2^48 scale the sums of T 2^-24 back exactly (FP64, far from
@@ -505,9 +514,9 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
 // per-pixel test can fire (the margin covers the FP32 rounding of the
 // per-pixel warp and of the range, both below 1e-2 px), the pass runs
 // without the per-pixel tests; the results are identical either way.
-template <int L, int INTERP, bool INT, bool TABLE, bool RP, bool K32 = false, int UNR = 1>
+template <int L, int INTERP, bool INT, bool RP, bool K32 = false>
 __device__ __forceinline__ bool subset_pass(const IcgnParams& P, int px, int py, const float Wm[6], int lane,
-                                            double acc[8], const StepTable* tab)
+                                            double acc[8], const StripLane* tab)
 {
     const float ex = (float)P.Sx, ey = (float)P.Sy;
     const float cx = (float)px + Wm[2], cy = (float)py + Wm[5];
@@ -516,8 +525,8 @@ __device__ __forceinline__ bool subset_pass(const IcgnParams& P, int px, int py,
                       cy - ry >= (float)(P.sy0 + 1) && cy + ry < (float)(P.sy0 + P.rh - 2);
     // both halves take the same loop: the per-pixel tests run unless every
     // active lane's POI is safe
-    if (__all(safe)) return subset_loop<L, INTERP, INT, false, TABLE, RP, K32, UNR>(P, px, py, Wm, lane, acc, tab);
-    return subset_loop<L, INTERP, INT, true, TABLE, RP, K32, UNR>(P, px, py, Wm, lane, acc, tab);
+    if (__all(safe)) return subset_loop<L, INTERP, INT, false, RP, K32>(P, px, py, Wm, lane, acc, tab);
+    return subset_loop<L, INTERP, INT, true, RP, K32>(P, px, py, Wm, lane, acc, tab);
 }
 
 // IC-GN for one POI by a group of L lanes: a whole wavefront (L = 64) or
@@ -527,8 +536,8 @@ __device__ __forceinline__ bool subset_pass(const IcgnParams& P, int px, int py,
 // per-POI values, so with halves the two POIs' solves and warp updates issue
 // as one instruction stream; with whole wavefronts they are wave-uniform and
 // kept in SGPRs.
-template <int L, int INTERP, bool TABLE, bool RP, bool K32 = false, int UNR = 1>
-__device__ __forceinline__ void icgn_poi_t(const IcgnParams& P, int poi, int lane, const StepTable* tab,
+template <int L, int INTERP, bool RP, bool K32 = false>
+__device__ __forceinline__ void icgn_poi_t(const IcgnParams& P, int poi, int lane, const StripLane* tab,
                                            const double* rs)
 {
     int py = P.poi[2 * poi];
@@ -553,8 +562,8 @@ __device__ __forceinline__ void icgn_poi_t(const IcgnParams& P, int poi, int lan
         for (int it = 0;; ++it) {
             if (it >= 1) iters = it + 1;                       // ++iNumIterations (:753)
             double acc[8];
-            const bool inside = it == 0 ? subset_pass<L, INTERP, true, TABLE, RP, K32, UNR>(P, px, py, Wm, lane, acc, tab)
-                                        : subset_pass<L, INTERP, false, TABLE, RP, K32, UNR>(P, px, py, Wm, lane, acc, tab);
+            const bool inside = it == 0 ? subset_pass<L, INTERP, true, RP, K32>(P, px, py, Wm, lane, acc, tab)
+                                        : subset_pass<L, INTERP, false, RP, K32>(P, px, py, Wm, lane, acc, tab);
             if (!inside) { flag = TWDIC_ICGN_OUT_OF_ROI; break; }         // :632-635, :787-790
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[i] = group_sum<L>(acc[i]);
@@ -629,14 +638,14 @@ __device__ __forceinline__ void icgn_poi_t(const IcgnParams& P, int poi, int lan
 // The fused mode reads the target's row polynomials when the caller built
 // them (P.rp, the same for every wave of a launch), else the image bytes;
 // both evaluate the same Catmull-Rom spline.
-template <int L, int INTERP, bool TABLE>
-__device__ __forceinline__ void icgn_poi(const IcgnParams& P, int poi, int lane, const StepTable* tab,
+template <int L, int INTERP>
+__device__ __forceinline__ void icgn_poi(const IcgnParams& P, int poi, int lane, const StripLane* tab,
                                          const double* rs)
 {
     if (INTERP == TWDIC_INTERP_FUSED && P.rp != nullptr)
-        icgn_poi_t<L, INTERP, TABLE, INTERP == TWDIC_INTERP_FUSED>(P, poi, lane, tab, rs);
+        icgn_poi_t<L, INTERP, INTERP == TWDIC_INTERP_FUSED>(P, poi, lane, tab, rs);
     else
-        icgn_poi_t<L, INTERP, TABLE, false>(P, poi, lane, tab, rs);
+        icgn_poi_t<L, INTERP, false>(P, poi, lane, tab, rs);
 }
 
 // The reference state of the POIs first .. first + count - 1 (those below n)
@@ -655,8 +664,7 @@ __device__ __forceinline__ void copy_ref_state(double (*slots)[kRefStateUsed], c
 
 // MINW: occupancy target (waves per SIMD) the register budget is fitted to;
 // 0 leaves the choice to the compiler.
-// TABLE: the subset has at most kStepTable pixels; the workgroup builds the
-// step table in LDS first.
+// The workgroup builds its strips' lane table in LDS first.
 // L lanes per POI, 256 / L POIs per workgroup (POI (256 / L) b' + t / L for
 // thread t); consecutive workgroups go to the 8 XCDs round-robin, so block b
 // is remapped to b' = the next block of XCD b % 8's contiguous share and each
@@ -667,39 +675,31 @@ __device__ __forceinline__ int xcd_block(int b, int nb)
     return x * q + min(x, r) + slot;
 }
 
-template <int INTERP, int MINW, bool TABLE, bool RP, int L, bool K32 = false>
+template <int INTERP, int MINW, bool RP, int L, bool K32 = false>
 __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_icgn(IcgnParams P)
 {
     constexpr int G = 256 / L;                   // POIs per workgroup
     __shared__ double rs[G][kRefStateUsed];
+    __shared__ StripLane tab[kMaxStrips * L];
     const int first = xcd_block(blockIdx.x, gridDim.x) * G;
     const int slot = threadIdx.x / L, poi = first + slot;
     copy_ref_state(rs, P.refstate, first, G, P.n, threadIdx.x, 256);
-    if constexpr (TABLE) {
-        __shared__ StepTable tab;
-        fill_step_table(tab, P);
-        __syncthreads();
-        if (poi >= P.n) return;
-        // two pixels per table-loop trip with halves (0.6 % faster on the
-        // 2048^2 frame); the batched kernel keeps one, which was 5 % faster there
-        icgn_poi_t<L, INTERP, true, RP, K32, L == 32 ? 2 : 1>(P, poi, threadIdx.x & 63, &tab, rs[slot]);
-    } else {
-        __syncthreads();
-        if (poi >= P.n) return;
-        icgn_poi_t<L, INTERP, false, RP, K32>(P, poi, threadIdx.x & 63, nullptr, rs[slot]);
-    }
+    fill_strips<L>(tab, P, threadIdx.x, 256);
+    __syncthreads();
+    if (poi >= P.n) return;
+    icgn_poi_t<L, INTERP, RP, K32>(P, poi, threadIdx.x & 63, tab, rs[slot]);
 }
 
 // Batched form, one launch over many image pairs: workgroup item w =
 // (pair, first POI) holds up to 256 / L POIs of one pair (every listed pair
 // takes L lanes per POI, icgn_lanes_for of its POI count), so the
-// workgroup's step table is that pair's.  XCD: items in contiguous per-XCD ranges as in
+// workgroup's strip table is that pair's.  XCD: items in contiguous per-XCD ranges as in
 // k_icgn (one band of the work per L2); otherwise dealt out in block order,
 // which balances the XCDs when the work per item differs from pair to pair.
 // ALL_RP: every pair has its row-polynomial plane (the usual case), so only
 // that form is compiled in and gets the register budget; otherwise each pair
 // takes its form at run time.
-template <int INTERP, int MINW, bool TABLE, bool XCD, bool ALL_RP, int L>
+template <int INTERP, int MINW, bool XCD, bool ALL_RP, int L>
 __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_batch_icgn_wg(const PairDesc* __restrict__ pairs,
                                                                            const int2* __restrict__ wg)
 {
@@ -707,71 +707,52 @@ __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_batch_icgn_wg(cons
     const int2 it = wg[XCD ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x];
     const IcgnParams P = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(it.x)].icgn;
     __shared__ double rs[G][kRefStateUsed];
+    __shared__ StripLane tab[kMaxStrips * L];
     const int first = __builtin_amdgcn_readfirstlane(it.y);
     const int slot = threadIdx.x / L, poi = first + slot;
     copy_ref_state(rs, P.refstate, first, G, P.n, threadIdx.x, 256);
-    if constexpr (TABLE) {
-        __shared__ StepTable tab;
-        fill_step_table(tab, P);
-        __syncthreads();
-        if (poi >= P.n) return;
-        if constexpr (ALL_RP)
-            icgn_poi_t<L, INTERP, true, true>(P, poi, threadIdx.x & 63, &tab, rs[slot]);
-        else
-            icgn_poi<L, INTERP, true>(P, poi, threadIdx.x & 63, &tab, rs[slot]);
-    } else {
-        __syncthreads();
-        if (poi >= P.n) return;
-        if constexpr (ALL_RP)
-            icgn_poi_t<L, INTERP, false, true>(P, poi, threadIdx.x & 63, nullptr, rs[slot]);
-        else
-            icgn_poi<L, INTERP, false>(P, poi, threadIdx.x & 63, nullptr, rs[slot]);
-    }
+    fill_strips<L>(tab, P, threadIdx.x, 256);
+    __syncthreads();
+    if (poi >= P.n) return;
+    if constexpr (ALL_RP)
+        icgn_poi_t<L, INTERP, true>(P, poi, threadIdx.x & 63, tab, rs[slot]);
+    else
+        icgn_poi<L, INTERP>(P, poi, threadIdx.x & 63, tab, rs[slot]);
 }
 
-bool step_table_fits(int wsub, int hsub)
-{
-    return wsub * hsub <= kStepTable;
-}
-
-template <int MINW, bool TABLE, bool XCD, bool ALL_RP, int L>
+template <int MINW, bool XCD, bool ALL_RP, int L>
 static void launch_wg(const PairDesc* pairs, const int2* wg, int count, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_batch_icgn_wg<TWDIC_INTERP_FUSED, MINW, TABLE, XCD, ALL_RP, L>), dim3(count), dim3(256), 0,
-                       st, pairs, wg);
+    hipLaunchKernelGGL((k_batch_icgn_wg<TWDIC_INTERP_FUSED, MINW, XCD, ALL_RP, L>), dim3(count), dim3(256), 0, st,
+                       pairs, wg);
 }
 
 template <int MINW, bool ALL_RP, int L>
-static void launch_wg_w(const PairDesc* pairs, const int2* wg, int count, bool table, bool xcd, hipStream_t st)
+static void launch_wg_w(const PairDesc* pairs, const int2* wg, int count, bool xcd, hipStream_t st)
 {
-    if (table)
-        xcd ? launch_wg<MINW, true, true, ALL_RP, L>(pairs, wg, count, st)
-            : launch_wg<MINW, true, false, ALL_RP, L>(pairs, wg, count, st);
-    else
-        xcd ? launch_wg<MINW, false, true, ALL_RP, L>(pairs, wg, count, st)
-            : launch_wg<MINW, false, false, ALL_RP, L>(pairs, wg, count, st);
+    xcd ? launch_wg<MINW, true, ALL_RP, L>(pairs, wg, count, st) : launch_wg<MINW, false, ALL_RP, L>(pairs, wg, count, st);
 }
 
 template <int L>
-static void launch_wg_l(const PairDesc* pairs, const int2* wg, int count, bool table, int waves, bool xcd_ranges,
-                        bool all_rp, hipStream_t st)
+static void launch_wg_l(const PairDesc* pairs, const int2* wg, int count, int waves, bool xcd_ranges, bool all_rp,
+                        hipStream_t st)
 {
     if (all_rp)
-        waves == 6 ? launch_wg_w<6, true, L>(pairs, wg, count, table, xcd_ranges, st)
-                   : launch_wg_w<5, true, L>(pairs, wg, count, table, xcd_ranges, st);
+        waves == 6 ? launch_wg_w<6, true, L>(pairs, wg, count, xcd_ranges, st)
+                   : launch_wg_w<5, true, L>(pairs, wg, count, xcd_ranges, st);
     else
-        waves == 6 ? launch_wg_w<6, false, L>(pairs, wg, count, table, xcd_ranges, st)
-                   : launch_wg_w<5, false, L>(pairs, wg, count, table, xcd_ranges, st);
+        waves == 6 ? launch_wg_w<6, false, L>(pairs, wg, count, xcd_ranges, st)
+                   : launch_wg_w<5, false, L>(pairs, wg, count, xcd_ranges, st);
 }
 
-hipError_t launch_batch_icgn_wg(const PairDesc* pairs, const int2* wg, int count, bool table, int lanes, int waves,
+hipError_t launch_batch_icgn_wg(const PairDesc* pairs, const int2* wg, int count, int lanes, int waves,
                                 bool xcd_ranges, bool all_rp, hipStream_t st)
 {
     if (count <= 0) return hipSuccess;
     if (lanes == 64)
-        launch_wg_l<64>(pairs, wg, count, table, waves, xcd_ranges, all_rp, st);
+        launch_wg_l<64>(pairs, wg, count, waves, xcd_ranges, all_rp, st);
     else
-        launch_wg_l<32>(pairs, wg, count, table, waves, xcd_ranges, all_rp, st);
+        launch_wg_l<32>(pairs, wg, count, waves, xcd_ranges, all_rp, st);
     return hipGetLastError();
 }
 
@@ -785,7 +766,9 @@ __global__ __launch_bounds__(256) void k_batch_icgn(const PairDesc* __restrict__
                                                     int total, int* counter, int chunk)
 {
     __shared__ double rs[4][1][kRefStateUsed];
+    __shared__ StripLane tabs[4][kMaxStrips * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    StripLane* tab = tabs[wave];
     for (;;) {
         int base = 0;
         if (lane == 0) base = atomicAdd(counter, chunk);
@@ -796,15 +779,19 @@ __global__ __launch_bounds__(256) void k_batch_icgn(const PairDesc* __restrict__
             const int2 it = items[i];
             const int pair = __builtin_amdgcn_readfirstlane(it.x), poi = __builtin_amdgcn_readfirstlane(it.y);
             const IcgnParams P = const_pairs(pairs)[pair].icgn;
-            // the wave's LDS slot: written and read by this wavefront only
+            // the wave's LDS slots: written and read by this wavefront only
             __builtin_amdgcn_wave_barrier();
             copy_ref_state(rs[wave], P.refstate, poi, 1, P.n, lane, 64);
+            if (P.lanes == 64)
+                fill_strips<64>(tab, P, lane, 64);
+            else
+                fill_strips<32>(tab, P, lane, 64);
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
             if (P.lanes == 64)
-                icgn_poi<64, TWDIC_INTERP_FUSED, false>(P, poi, lane, nullptr, rs[wave][0]);
+                icgn_poi<64, TWDIC_INTERP_FUSED>(P, poi, lane, tab, rs[wave][0]);
             else if (lane < 32)
-                icgn_poi<32, TWDIC_INTERP_FUSED, false>(P, poi, lane, nullptr, rs[wave][0]);
+                icgn_poi<32, TWDIC_INTERP_FUSED>(P, poi, lane, tab, rs[wave][0]);
         }
     }
 }
@@ -827,24 +814,23 @@ hipError_t launch_batch_icgn(const PairDesc* pairs, const int2* items, int total
 
 // variant: the occupancy target of the half-wavefront form (5 or 6 waves per
 // SIMD, or 0, the compiler's choice), or 20, the compensated FP32 sums; the
-// whole-wavefront form is built for 5 waves per SIMD.  (Seven waves do not
-// fit: the workgroup's LDS caps a CU at five.)
-template <int INTERP, bool TABLE, bool RP, int L>
+// whole-wavefront form is built for 5 waves per SIMD.
+template <int INTERP, bool RP, int L>
 static void launch_icgn_v(const IcgnParams& p, int variant, hipStream_t st)
 {
     constexpr int G = 256 / L;
     const dim3 grid((p.n + G - 1) / G);
     if (variant == 20) {
-        hipLaunchKernelGGL((k_icgn<INTERP, 5, TABLE, RP, L, true>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((k_icgn<INTERP, 5, RP, L, true>), grid, dim3(256), 0, st, p);
         return;
     }
     if constexpr (L == 64) {
-        hipLaunchKernelGGL((k_icgn<INTERP, 5, TABLE, RP, 64>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((k_icgn<INTERP, 5, RP, 64>), grid, dim3(256), 0, st, p);
     } else {
         switch (variant) {
-        case 5: hipLaunchKernelGGL((k_icgn<INTERP, 5, TABLE, RP, L>), grid, dim3(256), 0, st, p); break;
-        case 6: hipLaunchKernelGGL((k_icgn<INTERP, 6, TABLE, RP, L>), grid, dim3(256), 0, st, p); break;
-        default: hipLaunchKernelGGL((k_icgn<INTERP, 0, TABLE, RP, L>), grid, dim3(256), 0, st, p); break;
+        case 5: hipLaunchKernelGGL((k_icgn<INTERP, 5, RP, L>), grid, dim3(256), 0, st, p); break;
+        case 6: hipLaunchKernelGGL((k_icgn<INTERP, 6, RP, L>), grid, dim3(256), 0, st, p); break;
+        default: hipLaunchKernelGGL((k_icgn<INTERP, 0, RP, L>), grid, dim3(256), 0, st, p); break;
         }
     }
 }
@@ -852,11 +838,7 @@ static void launch_icgn_v(const IcgnParams& p, int variant, hipStream_t st)
 template <int INTERP, bool RP>
 static void launch_icgn_r(const IcgnParams& p, int variant, hipStream_t st)
 {
-    const bool table = p.s <= kStepTable;
-    if (p.lanes == 64)
-        table ? launch_icgn_v<INTERP, true, RP, 64>(p, variant, st) : launch_icgn_v<INTERP, false, RP, 64>(p, variant, st);
-    else
-        table ? launch_icgn_v<INTERP, true, RP, 32>(p, variant, st) : launch_icgn_v<INTERP, false, RP, 32>(p, variant, st);
+    p.lanes == 64 ? launch_icgn_v<INTERP, RP, 64>(p, variant, st) : launch_icgn_v<INTERP, RP, 32>(p, variant, st);
 }
 
 template <int INTERP>

@@ -38,6 +38,53 @@ constexpr int kRefStateUsed = 42;     // the doubles above that the iteration ke
 constexpr int kIcgnHalfWaveMin = 32768;
 inline int icgn_lanes_for(int n) { return n >= kIcgnHalfWaveMin ? 32 : 64; }
 
+// How the L lanes of a POI's group walk its subset: strips of `ncol` columns
+// from column `col`, each column cut into `segs` row ranges of equal length
+// (the first ones a row longer where they do not divide), one lane per column
+// and range, ncol segs <= L.
+constexpr int kMaxStrips = 6;
+struct Strip {
+    int16_t col, ncol, segs;
+};
+struct StripPlan {
+    int count;
+    Strip s[kMaxStrips];
+};
+
+// The strips of a W x H subset (1 <= W, H <= 121; L = 32 or 64) with the
+// fewest rounds, a strip costing one round besides its longest row range.
+inline StripPlan strip_plan(int W, int H, int L)
+{
+    constexpr int kMaxW = 128;
+    int cost[kMaxW], take[kMaxW];
+    cost[0] = 0;
+    auto segs = [&](int c) { return L / c < H ? L / c : H; };
+    for (int w = 1; w <= W; ++w) {
+        cost[w] = 1 << 30;
+        for (int c = w < L ? w : L; c >= 1; --c) {
+            const int sg = segs(c), v = cost[w - c] + (H + sg - 1) / sg + 1;
+            if (v < cost[w]) {
+                cost[w] = v;
+                take[w] = c;
+            }
+        }
+    }
+    StripPlan p{};
+    int col = 0, w = W;
+    for (; w > 0 && p.count < kMaxStrips; w -= take[w]) {
+        p.s[p.count++] = {(int16_t)col, (int16_t)take[w], (int16_t)segs(take[w])};
+        col += take[w];
+    }
+    if (w > 0) {                       // more strips than the table holds: whole widths instead
+        p.count = 0;
+        for (col = 0; col < W; col += L) {
+            const int c = W - col < L ? W - col : L;
+            p.s[p.count++] = {(int16_t)col, (int16_t)c, (int16_t)segs(c)};
+        }
+    }
+    return p;
+}
+
 // Mean and L2 spread of n samples from their exact-or-FP64 sums s1 = sum x,
 // s2 = sum x^2.  Shared by the reference-state and iteration kernels so that
 // identical subsets give bit-identical statistics.
@@ -78,6 +125,7 @@ struct IcgnParams {
     int Sx, Sy, Wsub, Hsub, s;
     int max_iter;
     int lanes;                // lanes per POI: 32 or 64 (icgn_lanes_for of the set's POI count)
+    StripPlan strips;         // how those lanes walk the subset
     double delta_p;           // the caller's float, widened: the loop test compares in FP64
     const uint32_t* g2;       // reference gradients (2Rx, 2Ry) as int16 pairs, ROI-relative
     const float* lut;         // target LUT [rh][rw][16]
@@ -99,6 +147,13 @@ struct PairDesc {
     IcgnParams icgn;
     FftccParams fftcc;
 };
+
+// The lanes per POI and the walk of a set of n POIs, from its subset size.
+inline void set_icgn_layout(IcgnParams& p, int n)
+{
+    p.lanes = icgn_lanes_for(n);
+    p.strips = strip_plan(p.Wsub, p.Hsub, p.lanes);
+}
 
 // Descriptors are never written while a batch kernel runs: reading them
 // through the constant address space lets the compiler use scalar loads and
@@ -146,9 +201,7 @@ int mma_form(int N);
 hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int form, hipStream_t st);
 // batched form: IC-GN (fused interpolation) over workgroup items (pair, first
 // POI), 256 / lanes POIs of one pair per workgroup, every listed pair with
-// that many lanes per POI; `table` when every listed pair's
-// subset fits the step table (step_table_fits).
-bool step_table_fits(int wsub, int hsub);
+// that many lanes per POI.
 // The row-polynomial plane of an ROI is addressed with 32-bit byte offsets
 // 16 (iy rw + ix) from entry -(sy0 rw + sx0); true when they all fit.
 inline bool row_poly_fits(int sx0, int sy0, int rw, int rh)
@@ -162,7 +215,7 @@ inline size_t row_poly_bytes(int rw, int rh)
 }
 // waves: occupancy target 5 or 6; xcd_ranges: contiguous per-XCD item ranges;
 // all_rp: every pair's descriptor has its row-polynomial plane
-hipError_t launch_batch_icgn_wg(const PairDesc* pairs, const int2* wg, int count, bool table, int lanes, int waves,
+hipError_t launch_batch_icgn_wg(const PairDesc* pairs, const int2* wg, int count, int lanes, int waves,
                                 bool xcd_ranges, bool all_rp, hipStream_t st);
 hipError_t launch_ref_state(const IcgnParams& p, hipStream_t st);
 hipError_t launch_icgn(const IcgnParams& p, int interp, int variant, hipStream_t st);
