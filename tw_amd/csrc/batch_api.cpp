@@ -39,7 +39,7 @@ struct twdic_batch {
     int64_t nf[3] = {};
     int64_t total = 0;
     uint32_t* d_g2 = nullptr;         // reference gradient planes of all pairs
-    uint4* d_rp = nullptr;            // target row polynomials of all pairs (rebuilt every step)
+    float4* d_rp = nullptr;            // target row polynomials of all pairs (rebuilt every step)
     int max_rh = 0;                   // largest ROI height among the pairs with a plane
     bool all_rp = false;              // every pair has a plane
     double* d_state = nullptr;        // per-POI reference state of all pairs
@@ -348,7 +348,7 @@ twdic_status set_pairs_impl(twdic_batch* b, const twdic_pair* pairs, int npairs)
         return e;
     };
     TB_HIP(b, alloc((void**)&b->d_g2, g2_elems * sizeof(uint32_t)));
-    TB_HIP(b, alloc((void**)&b->d_rp, rp_elems * sizeof(uint4)));
+    TB_HIP(b, alloc((void**)&b->d_rp, rp_elems * sizeof(float4)));
     TB_HIP(b, alloc((void**)&b->d_state, state_elems * sizeof(double)));
     TB_HIP(b, alloc((void**)&b->d_zncc_scratch, zn * sizeof(float)));
     TB_HIP(b, alloc((void**)&b->d_desc, sizeof(PairDesc) * std::max(1, npairs)));

@@ -32,6 +32,7 @@
 #include "twdic_internal.h"
 
 #include <cfloat>
+#include <type_traits>
 
 namespace twdic {
 
@@ -186,49 +187,57 @@ __device__ __forceinline__ float interp_fused_s(const TargetBuf& B, int ix, int 
 }
 
 // The target's row polynomials (launch_row_poly) as a buffer resource whose
-// base is entry -(sy0 rw + sx0): cell (ix, iy) reads the 16-byte entries at
-// byte offsets 16 (iy rw + ix) (rows iy - 1, iy) and that plus 32 rw (rows
-// iy + 1, iy + 2).  The host passes the plane only when every such offset is
-// below 2^32.
+// base is the entry of row -1, column 0: row iy - 1 of cell (ix, iy) is at
+// byte offset 16 (iy rw + ix), the rows below it 16 rw further each.  The
+// host passes the plane only when every such offset is below 2^32.
 struct RowPolyBuf {
     __amdgpu_buffer_rsrc_t r;
-    int rw16;      // 16 rw: bytes per entry row
+    int pitch;     // 16 rw: bytes per plane row
 };
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ RowPolyBuf row_poly_buf(const IcgnParams& P)
 {
     const uint32_t lead = 16u * ((uint32_t)P.sy0 * (uint32_t)P.rw + (uint32_t)P.sx0);
     const uint8_t* base = reinterpret_cast<const uint8_t*>(P.rp) - lead;
-    const int records = (int)(lead + 16u * (uint32_t)(P.rh + 1) * (uint32_t)P.rw);
+    const int records = (int)(lead + 16u * (uint32_t)(P.rh + 2) * (uint32_t)P.rw);
     return {__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, records, 0x00020000), 16 * P.rw};
 }
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-// One row's cubic at t: c0 + t (c1/2 + t (c2/2 + t c3/2)), the fp16
-// coefficients (stored halved, exactly) taken as exact f32 operands by the
-// mixed-precision FMA.  Every intermediate is exactly half the one of
-// c0 + (t/2) (c1 + t (c2 + t c3)) evaluated in the same order, so the two
-// forms round identically.
-__device__ __forceinline__ float row_poly(uint32_t c01, uint32_t c23, float t)
+__device__ __forceinline__ int row_poly_offset(const RowPolyBuf& B, int ix, int iy)
 {
-    const half2_t a = __builtin_bit_cast(half2_t, c01), b = __builtin_bit_cast(half2_t, c23);
-    return fmaf(t, fmaf(t, fmaf(t, (float)b.y, (float)b.x), (float)a.y), (float)a.x);
+    return (int)__umul24((uint32_t)iy, (uint32_t)B.pitch) + 16 * ix;
 }
 
-// Bicubic value at (ix + tx, iy + ty): the four rows' cubics at tx, then the
-// Catmull-Rom cubic through them at ty in the same form.  Its coefficients
-// are formed from the row values with exact small-integer weights, so a
-// uniform neighbourhood gives back its value exactly (every higher
-// coefficient is an exact zero), as the LUT does: uniform target regions keep
-// the reference's DarkSubset behaviour without a test.
-__device__ __forceinline__ float interp_row_poly(const RowPolyBuf& B, int ix, int iy, float tx, float ty)
+// the row polynomial at byte offset o, `rows` rows further down
+__device__ __forceinline__ f32x4 load_row_poly(const RowPolyBuf& B, int o, int rows)
 {
-    const int o = (int)__umul24((uint32_t)iy, (uint32_t)B.rw16) + 16 * ix;
-    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(B.r, o, 0, 0);
-    const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(B.r, o, 2 * B.rw16, 0);
-    const float R0 = row_poly(a.x, a.y, tx), R1 = row_poly(a.z, a.w, tx);
-    const float R2 = row_poly(b.x, b.y, tx), R3 = row_poly(b.z, b.w, tx);
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(B.r, o, rows * B.pitch, 0));
+}
+
+// One row's cubic at t from its stored coefficients c0, c1/2, c2/2, c3/2:
+// c0 + t (c1/2 + t (c2/2 + t c3/2)).  Every intermediate is exactly half the
+// one of c0 + (t/2) (c1 + t (c2 + t c3)) evaluated in the same order, so the
+// two forms round identically.
+__device__ __forceinline__ float row_poly(f32x4 c, float t)
+{
+    // the last step as a three-address instruction: the compiler's choice is a
+    // move and a two-address one
+    float r;
+    const float s = fmaf(t, fmaf(t, c.w, c.z), c.y);
+    asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r) : "v"(t), "v"(s), "v"(c.x));
+    return r;
+}
+
+// Bicubic value from the cubics of the four rows iy - 1 .. iy + 2 at tx: the
+// Catmull-Rom cubic through them at ty in the same form.  Its coefficients are formed from the row values with exact
+// small-integer weights, so a uniform neighbourhood gives back its value
+// exactly (every higher coefficient is an exact zero), as the LUT does:
+// uniform target regions keep the reference's DarkSubset behaviour without a
+// test.
+__device__ __forceinline__ float column_cubic(float R0, float R1, float R2, float R3, float ty)
+{
     const float d1 = R2 - R0;
     const float d2 = fmaf(4.f, R2, fmaf(-5.f, R1, fmaf(2.f, R0, -R3)));
     const float d3 = fmaf(3.f, R1 - R2, R3 - R0);
@@ -372,12 +381,20 @@ __device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P,
 // is integer-valued every term is an integer below 2^53, so these sums stay
 // exact there, as direct ones would be.
 //
-// Bound by VALU issue (79 % of the slots on the 2048^2 frame, 157,609 POIs of
-// 41x41) with the texture-address unit close behind (74 %).  Against a walk in
-// row-major order from a table of pixel offsets: 47 VALU instructions per
-// bicubic pixel (58) and 16 per integer one (26), 1.20 ms (1.35 ms); 14k POIs
-// on whole wavefronts 0.139 ms (0.153).  One row per trip: two or four took
-// 1.27 and 1.28 ms.
+// The bicubic passes over the row polynomials (ROLL) also keep the four rows
+// of the current cell in registers: in a column the next pixel's cell is the
+// one below unless a cell border runs between them, so a pixel loads one row
+// instead of four, and as its place is known beforehand, a pixel ahead.  The
+// fractional parts are then the coordinates less the expected cell's corner,
+// and one unsigned compare of both tells whether the pixel lies in it.
+//
+// Bound by VALU issue: 84 % of the slots on the 2048^2 frame (157,609 POIs of
+// 41x41).  There a walk in row-major order from a table of pixel offsets took
+// 1.35 ms (58 VALU instructions per bicubic pixel, of them 12 mixed-precision
+// ones of 1.5 slots, 26 per integer pixel), walking columns 1.20 ms (47 and
+// 16; two rows per trip 1.27 ms), keeping the rows 1.07 ms (48, all of one
+// slot); 14k POIs on whole wavefronts 0.153, 0.139, 0.123 ms.  W1 dy and W4 dy
+// from an LDS table (45 instructions) changed nothing.
 template <int L, int INTERP, bool INT, bool CHECK, bool RP, bool K32 = false>
 __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py, const float Wm[6], int lane,
                                             double acc[8], const StripLane* tab)
@@ -386,6 +403,7 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     // the fused interpolation from the bytes returns T 2^-24 (interp_rows_s);
     // the sums are scaled back at the end, exactly
     constexpr bool SCALED = !INT && INTERP == TWDIC_INTERP_FUSED && !RP;
+    constexpr bool ROLL = RP && !INT && !CHECK && !K32;
     const int sx0 = P.sx0, sy0 = P.sy0, rw = P.rw, rh = P.rh;
     const TargetBuf tb = target_buf(P);
     const __amdgpu_buffer_rsrc_t g2r =
@@ -397,49 +415,27 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     bool out = false;
     // byte offset of the subset's corner pixel in the gradient plane
     const uint32_t gcorner = 4u * (uint32_t)((py - P.Sy - sy0) * rw + (px - P.Sx - sx0));
-    // cx, cy: the column's share of the warped coordinates; go + so: the
-    // pixel's byte offset in the gradient plane (so is wave-uniform)
-    auto pixel = [&](float cx, float cy, float dx, float dy, uint32_t go, int so) {
-        float wx, wy;
-        {
+    // the warped coordinates of the pixel at (dx, dy) of a column whose share
+    // of them is cx, cy
+    auto warp = [&](float cx, float cy, float dy, float& wx, float& wy) {
 #pragma clang fp contract(off)
-            if constexpr (INT) {
-                // the first pass's warp is W = [[1, 0, u], [0, 1, v]] exactly, where
-                // ((POI + 1 dx) + 0 dy) + u = (POI + dx) + u bit for bit (POI + dx
-                // is a non-zero integer, so adding the zero product changes nothing)
-                wx = cx + Wm[2];
-                wy = (fpy + dy) + Wm[5];
-            } else {
-                // as the CPU path evaluates it (:618-619, :761-762): ((POI + W0*dx) +
-                // W1*dy) + W2, every product and sum rounded to FP32 (the pragma keeps
-                // the compiler from fusing a product into the following sum)
-                wx = (cx + Wm[1] * dy) + Wm[2];
-                wy = (cy + Wm[4] * dy) + Wm[5];
-            }
+        if constexpr (INT) {
+            // the first pass's warp is W = [[1, 0, u], [0, 1, v]] exactly, where
+            // ((POI + 1 dx) + 0 dy) + u = (POI + dx) + u bit for bit (POI + dx
+            // is a non-zero integer, so adding the zero product changes nothing)
+            wx = cx + Wm[2];
+            wy = (fpy + dy) + Wm[5];
+        } else {
+            // as the CPU path evaluates it (:618-619, :761-762): ((POI + W0*dx) +
+            // W1*dy) + W2, every product and sum rounded to FP32 (the pragma keeps
+            // the compiler from fusing a product into the following sum)
+            wx = (cx + Wm[1] * dy) + Wm[2];
+            wy = (cy + Wm[4] * dy) + Wm[5];
         }
-        const int ix = (int)wx, iy = (int)wy;          // truncation, as int()
-        float T = 0.f;
-        bool in = true, interior = true;
-        if (CHECK) {
-            in = ix >= sx0 && iy >= sy0 && ix < sx0 + rw && iy < sy0 + rh;
-            // the CPU bicubic LUT's last row/column is zero; the B-spline LUT covers it
-            interior = in && (INTERP == TWDIC_INTERP_BSPLINE || (ix != sx0 + rw - 1 && iy != sy0 + rh - 1));
-            out |= !in;
-        }
-        if (INT) {
-            if (in) T = (float)__builtin_amdgcn_raw_buffer_load_b8(tb.r, target_offset(tb, ix, iy), tb.stride + 1, 0); // :629
-        } else if (interior) {
-            // :771-772; wx, wy >= 1 here, so x - (float)(int)x is fract(x), exactly
-            const float tx = __builtin_amdgcn_fractf(wx), ty = __builtin_amdgcn_fractf(wy);
-            if constexpr (RP) {
-                T = interp_row_poly(rb, ix, iy, tx, ty);
-            } else if (INTERP == TWDIC_INTERP_FUSED) {
-                T = interp_fused_s(tb, ix, iy, tx, ty);
-            } else {
-                T = interp_lut(P.lut, (uint32_t)((iy - sy0) * rw + (ix - sx0)), tx, ty);
-            }
-        }
-        const uint32_t g = __builtin_amdgcn_raw_buffer_load_b32(g2r, (int)go, so, 0);
+    };
+    // so (wave-uniform) is the pixel's row offset in the gradient plane
+    auto gradient = [&](uint32_t go, int so) { return __builtin_amdgcn_raw_buffer_load_b32(g2r, (int)go, so, 0); };
+    auto accumulate = [&](float T, uint32_t g, float dx, float dy) {
         if constexpr (K32) {
             kahan_pixel(ks, kc, T, g, dx, dy);
             return;
@@ -456,6 +452,36 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
         a2 -= a0;
         b0 = fma(gy, Td, b0);
         b2 -= b0;
+    };
+    // one pixel on its own
+    auto pixel = [&](float cx, float cy, float dx, float dy, uint32_t go, int so) {
+        float wx, wy;
+        warp(cx, cy, dy, wx, wy);
+        const int ix = (int)wx, iy = (int)wy;          // truncation, as int()
+        float T = 0.f;
+        bool in = true, interior = true;
+        if (CHECK) {
+            in = ix >= sx0 && iy >= sy0 && ix < sx0 + rw && iy < sy0 + rh;
+            // the CPU bicubic LUT's last row/column is zero; the B-spline LUT covers it
+            interior = in && (INTERP == TWDIC_INTERP_BSPLINE || (ix != sx0 + rw - 1 && iy != sy0 + rh - 1));
+            out |= !in;
+        }
+        if (INT) {
+            if (in) T = (float)__builtin_amdgcn_raw_buffer_load_b8(tb.r, target_offset(tb, ix, iy), tb.stride + 1, 0); // :629
+        } else if (interior) {
+            // :771-772; wx, wy >= 1 here, so x - (float)(int)x is fract(x), exactly
+            const float tx = __builtin_amdgcn_fractf(wx), ty = __builtin_amdgcn_fractf(wy);
+            if constexpr (RP) {
+                const int o = row_poly_offset(rb, ix, iy);
+                T = column_cubic(row_poly(load_row_poly(rb, o, 0), tx), row_poly(load_row_poly(rb, o, 1), tx),
+                                 row_poly(load_row_poly(rb, o, 2), tx), row_poly(load_row_poly(rb, o, 3), tx), ty);
+            } else if (INTERP == TWDIC_INTERP_FUSED) {
+                T = interp_fused_s(tb, ix, iy, tx, ty);
+            } else {
+                T = interp_lut(P.lut, (uint32_t)((iy - sy0) * rw + (ix - sx0)), tx, ty);
+            }
+        }
+        accumulate(T, gradient(go, so), dx, dy);
     };
     const int nstrips = P.strips.count;
 #pragma unroll 1
@@ -476,13 +502,77 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                 cy = INT ? 0.f : fpy + Wm[3] * e.dx;
             }
             int so = 0;
+            if constexpr (ROLL) {
+                // the expected cell of the next pixel: column fx and row fy as
+                // floats, its first row at byte offset o; rows[] holds its four
+                // rows from index K on (mod 4).  A pixel's first row is done with
+                // once its cubic is evaluated, and the row the next cell adds is
+                // loaded in its place, a pixel ahead of its use.
+                float wx, wy;
+                warp(cx, cy, dy, wx, wy);
+                int o = row_poly_offset(rb, (int)wx, (int)wy);
+                float fx = (float)(int)wx, fy = (float)(int)wy;
+                f32x4 q[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q[i] = load_row_poly(rb, o, i);
+                uint32_t g = gradient(go, 0);
+                auto step = [&](auto k) {
+                    constexpr int K = decltype(k)::value;
+                    warp(cx, cy, dy, wx, wy);
+                    float tx = wx - fx, ty = wy - fy;       // exact; in [0, 1) in the expected cell
+                    if (max(__float_as_uint(tx), __float_as_uint(ty)) >= 0x3f800000u) {
+                        // another cell: its rows anew, in this lane
+                        const int ix = (int)wx, iy = (int)wy;
+                        fx = (float)ix;
+                        fy = (float)iy;
+                        tx = wx - fx;
+                        ty = wy - fy;
+                        o = row_poly_offset(rb, ix, iy);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) q[(K + i) & 3] = load_row_poly(rb, o, i);
+                    }
+                    const float R0 = row_poly(q[K], tx);
+                    q[K] = load_row_poly(rb, o, 4);
+                    so += 4 * rw;
+                    const uint32_t gn = gradient(go, so);
+                    const float R1 = row_poly(q[(K + 1) & 3], tx), R2 = row_poly(q[(K + 2) & 3], tx),
+                                R3 = row_poly(q[(K + 3) & 3], tx);
+                    accumulate(column_cubic(R0, R1, R2, R3, ty), g, e.dx, dy);
+                    // keep the compiler from sinking this pixel's arithmetic below the next ones' loads
+                    asm volatile("" : "+v"(st), "+v"(stt), "+v"(a0), "+v"(a2), "+v"(b0), "+v"(b2));
+                    g = gn;
+                    dy += 1.f;
+                    fy += 1.f;
+                    o += rb.pitch;
+                };
+                using std::integral_constant;
+                const int quads = full >> 2, left = rows - 4 * quads;
 #pragma unroll 1
-            for (int r = 0; r < full; ++r) {
-                pixel(cx, cy, e.dx, dy, go, so);
-                dy += 1.f;
-                so += 4 * rw;
+                for (int r = 0; r < quads; ++r) {
+                    step(integral_constant<int, 0>{});
+                    step(integral_constant<int, 1>{});
+                    step(integral_constant<int, 2>{});
+                    step(integral_constant<int, 3>{});
+                }
+                if (left > 0) {
+                    step(integral_constant<int, 0>{});
+                    if (left > 1) {
+                        step(integral_constant<int, 1>{});
+                        if (left > 2) {
+                            step(integral_constant<int, 2>{});
+                            if (left > 3) step(integral_constant<int, 3>{});
+                        }
+                    }
+                }
+            } else {
+#pragma unroll 1
+                for (int r = 0; r < full; ++r) {
+                    pixel(cx, cy, e.dx, dy, go, so);
+                    dy += 1.f;
+                    so += 4 * rw;
+                }
+                if (rows > full) pixel(cx, cy, e.dx, dy, go, so);
             }
-            if (rows > full) pixel(cx, cy, e.dx, dy, go, so);
             const double end = ddy + (double)rows;
             a1 = fma(ddx, a0, a1);
             a2 = fma(end, a0, a2);

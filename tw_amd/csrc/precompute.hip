@@ -224,41 +224,25 @@ hipError_t launch_bicubic_lut(const uint8_t* tar, int stride, int sx0, int sy0, 
 // and x + 1, its cubic through p0..p3 = T(y, x-1 .. x+2) is
 //   R(t) = c0 + t/2 (c1 + t (c2 + t c3)),
 //   c0 = p1, c1 = p2 - p0, c2 = 2 p0 - 5 p1 + 4 p2 - p3, c3 = 3 (p1 - p2) + p3 - p0,
-// integers of magnitude at most 1530.  Stored as c0, c1/2, c2/2, c3/2 (the
-// halves are multiples of 1/2 below 766 in magnitude, so exact in fp16), the
-// cubic is c0 + t (c1/2 + t (c2/2 + t c3/2)).  Entry (x, j) holds the four
-// coefficients of rows y = sy0 - 1 + j and y + 1 (fp16, row y, then row y + 1:
-// 16 bytes) for cell column sx0 + x, x < rw, j <= rh; the last column (never
-// an interior cell) is zero.  A cell's four neighbourhood rows are then two
-// 16-byte entries, (x, j) and (x, j + 2).
+// integers of magnitude at most 1530.  Stored as c0, c1/2, c2/2, c3/2 in FP32
+// (exactly), the cubic is c0 + t (c1/2 + t (c2/2 + t c3/2)).  Entry (x, j) holds
+// the four coefficients (16 bytes) of row y = sy0 - 1 + j for cell column
+// sx0 + x, x < rw, j <= rh + 1; the last column (never an interior cell) is
+// zero.  A cell's four neighbourhood rows are the entries (x, j) .. (x, j + 3).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t h2bits(float lo, float hi)
-{
-    const uint32_t a = __builtin_bit_cast(uint16_t, (_Float16)lo);
-    const uint32_t b = __builtin_bit_cast(uint16_t, (_Float16)hi);
-    return a | (b << 16);
-}
-
-// Entry (x, j) from the two target rows' dwords at columns sx0 + x - 1 ..
-// sx0 + x + 2: for x < rw - 1 they lie in the image (the ROI keeps a one-pixel
+// Entry (x, j) from the target row's dword at columns sx0 + x - 1 ..
+// sx0 + x + 2: for x < rw - 1 it lies in the image (the ROI keeps a one-pixel
 // frame); the buffer's range check would read anything past its last row as
 // zero.  The target resource's base is the image, records (sy0 + rh + 1) rows.
 __device__ __forceinline__ void row_poly_entry(__amdgpu_buffer_rsrc_t img, int stride, int sx0, int sy0, int rw,
-                                               int x, int j, uint4* __restrict__ rp)
+                                               int x, int j, float4* __restrict__ rp)
 {
-    uint4 e = make_uint4(0u, 0u, 0u, 0u);
+    float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
     if (x < rw - 1) {
-        const int o = (sy0 - 1 + j) * stride + (sx0 - 1 + x);
-        uint32_t h[4];
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(img, o, r * stride, 0);
-            const int p0 = (int)(w & 255u), p1 = (int)((w >> 8) & 255u), p2 = (int)((w >> 16) & 255u),
-                      p3 = (int)(w >> 24);
-            h[2 * r] = h2bits((float)p1, 0.5f * (float)(p2 - p0));
-            h[2 * r + 1] = h2bits(0.5f * (float)(2 * p0 - 5 * p1 + 4 * p2 - p3), 0.5f * (float)(3 * (p1 - p2) + p3 - p0));
-        }
-        e = make_uint4(h[0], h[1], h[2], h[3]);
+        const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(img, (sy0 - 1 + j) * stride + (sx0 - 1 + x), 0, 0);
+        const int p0 = (int)(w & 255u), p1 = (int)((w >> 8) & 255u), p2 = (int)((w >> 16) & 255u), p3 = (int)(w >> 24);
+        e = make_float4((float)p1, 0.5f * (float)(p2 - p0), 0.5f * (float)(2 * p0 - 5 * p1 + 4 * p2 - p3),
+                        0.5f * (float)(3 * (p1 - p2) + p3 - p0));
     }
     rp[(size_t)j * rw + x] = e;
 }
@@ -271,18 +255,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_poly_src(const uint8_t* ta
 // One entry per thread: x along the block's 256 threads and blockIdx.x, rows
 // j = blockIdx.y, + gridDim.y, ...
 __global__ __launch_bounds__(256) void k_row_poly(const uint8_t* __restrict__ tar, int stride, int sx0, int sy0,
-                                                  int rw, int rh, uint4* __restrict__ rp)
+                                                  int rw, int rh, float4* __restrict__ rp)
 {
     const __amdgpu_buffer_rsrc_t img = row_poly_src(tar, stride, sy0, rh);
     const int x = blockIdx.x * 256 + threadIdx.x;
     if (x >= rw) return;
-    for (int j = blockIdx.y; j <= rh; j += gridDim.y) row_poly_entry(img, stride, sx0, sy0, rw, x, j, rp);
+    for (int j = blockIdx.y; j <= rh + 1; j += gridDim.y) row_poly_entry(img, stride, sx0, sy0, rw, x, j, rp);
 }
 
-hipError_t launch_row_poly(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, uint4* rp,
+hipError_t launch_row_poly(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* rp,
                            hipStream_t st)
 {
-    const dim3 grid((rw + 255) / 256, std::min(rh + 1, 65535));
+    const dim3 grid((rw + 255) / 256, std::min(rh + 2, 65535));
     hipLaunchKernelGGL(k_row_poly, grid, dim3(256), 0, st, tar, stride, sx0, sy0, rw, rh, rp);
     return hipGetLastError();
 }
@@ -296,15 +280,15 @@ __global__ __launch_bounds__(256) void k_batch_row_poly(const PairDesc* __restri
     const IcgnParams P = const_pairs(pairs)[blockIdx.y].icgn;
     if (P.rp == nullptr) return;
     const __amdgpu_buffer_rsrc_t img = row_poly_src(P.tar, P.stride, P.sy0, P.rh);
-    for (int j = blockIdx.x; j <= P.rh; j += gridDim.x)
+    for (int j = blockIdx.x; j <= P.rh + 1; j += gridDim.x)
         for (int x = threadIdx.x; x < P.rw; x += 256)
-            row_poly_entry(img, P.stride, P.sx0, P.sy0, P.rw, x, j, const_cast<uint4*>(P.rp));
+            row_poly_entry(img, P.stride, P.sx0, P.sy0, P.rw, x, j, const_cast<float4*>(P.rp));
 }
 
 hipError_t launch_batch_row_poly(const PairDesc* pairs, int npairs, int max_rh, hipStream_t st)
 {
     if (npairs <= 0) return hipSuccess;
-    const int blocks = std::max(1, std::min(max_rh + 1, 1024));
+    const int blocks = std::max(1, std::min(max_rh + 2, 1024));
     hipLaunchKernelGGL(k_batch_row_poly, dim3(blocks, npairs), dim3(256), 0, st, pairs);
     return hipGetLastError();
 }

@@ -334,7 +334,7 @@ bool admit(twdic_server* s, Slot& sl, Job& j)
 
     char* base = s->d_arena;
     uint8_t* d_tar = (uint8_t*)(base + off);
-    uint4* d_rp = rp_fits ? (uint4*)(base + off + tar_b) : nullptr;
+    float4* d_rp = rp_fits ? (float4*)(base + off + tar_b) : nullptr;
     char* d_out = base + off + tar_b + rp_b;
     float* d_u = (float*)d_out;
     float* d_v = d_u + n;

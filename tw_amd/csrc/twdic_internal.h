@@ -129,7 +129,7 @@ struct IcgnParams {
     double delta_p;           // the caller's float, widened: the loop test compares in FP64
     const uint32_t* g2;       // reference gradients (2Rx, 2Ry) as int16 pairs, ROI-relative
     const float* lut;         // target LUT [rh][rw][16]
-    const uint4* rp;          // target row polynomials [rh + 1][rw] (fused mode; null: from the image bytes)
+    const float4* rp;         // target row polynomials [rh + 2][rw] (fused mode; null: from the image bytes)
     double* refstate;         // kRefStateStride doubles per POI
     const int32_t* poi;
     int n;
@@ -174,8 +174,8 @@ hipError_t launch_gradients(const uint8_t* img, int stride, int sx0, int sy0, in
                             float* gx, float* gy, float* gxy, uint32_t* g2, hipStream_t st);
 hipError_t launch_bspline_lut(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float* lut,
                               hipStream_t st);
-// fp16 Catmull-Rom row polynomials of the target, (rh + 1) x rw entries of 16 bytes
-hipError_t launch_row_poly(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, uint4* rp,
+// Catmull-Rom row polynomials of the target, (rh + 2) x rw entries of 16 bytes
+hipError_t launch_row_poly(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* rp,
                            hipStream_t st);
 // the same for every pair of a batch with a plane (descriptor icgn.rp set);
 // max_rh: the largest ROI height among them
@@ -211,7 +211,7 @@ inline bool row_poly_fits(int sx0, int sy0, int rw, int rh)
 }
 inline size_t row_poly_bytes(int rw, int rh)
 {
-    return 16ull * (size_t)rw * (size_t)(rh + 1);
+    return 16ull * (size_t)rw * (size_t)(rh + 2);
 }
 // waves: occupancy target 5 or 6; xcd_ranges: contiguous per-XCD item ranges;
 // all_rp: every pair's descriptor has its row-polynomial plane
@@ -258,7 +258,7 @@ struct twdic_ctx {
     float* d_ty = nullptr;
     float* d_txy = nullptr;
     float* d_lut = nullptr;
-    uint4* d_rp = nullptr;            // target row polynomials (fused interpolation)
+    float4* d_rp = nullptr;           // target row polynomials (fused interpolation)
     uint32_t* d_g2 = nullptr;         // packed (2Rx, 2Ry) int16 pairs
     float2* d_fft_tw = nullptr;
     bool ref_loaded = false, tar_loaded = false;
