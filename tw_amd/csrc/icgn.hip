@@ -244,6 +244,26 @@ __device__ __forceinline__ float column_cubic(float R0, float R1, float R2, floa
     return fmaf(0.5f * ty, fmaf(fmaf(d3, ty, d2), ty, d1), R1);
 }
 
+// The same from the same rows as the materialised LUT gives it (interp_lut):
+// the cell's coefficients a[k][l] of y^k x^l are small-integer combinations of
+// the row coefficients, exact in FP32 (multiples of 1/4 below 2^14), and the
+// polynomial is evaluated in the LUT's order.  The rows k >= 1 are formed
+// doubled, which changes no rounding, and halved in the last product.
+__device__ __forceinline__ float lut_cubic(f32x4 q0, f32x4 q1, f32x4 q2, f32x4 q3, float tx, float ty)
+{
+    float a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll
+    for (int l = 3; l >= 0; --l) {
+        const float b1 = q2[l] - q0[l];
+        const float b2 = fmaf(4.f, q2[l], fmaf(-5.f, q1[l], fmaf(2.f, q0[l], -q3[l])));
+        const float b3 = fmaf(3.f, q1[l] - q2[l], q3[l] - q0[l]);
+        a1 = l == 3 ? b1 : fmaf(a1, tx, b1);
+        a2 = l == 3 ? b2 : fmaf(a2, tx, b2);
+        a3 = l == 3 ? b3 : fmaf(a3, tx, b3);
+    }
+    return fmaf(fmaf(fmaf(a3, ty, a2), ty, a1), 0.5f * ty, row_poly(q1, tx));
+}
+
 // p from W, as the update sets it (TW_paDIC_ICGN2D_CPU.cpp:902-907): p0 = W02,
 // p1 = W00 - 1, p2 = W01, p3 = W12, p4 = W10, p5 = W11 - 1.  For the initial
 // W = [[1 + 0, 0, u], [0, 1 + 0, v]] (:605-607) this gives back (u, 0, 0, v,
@@ -334,10 +354,14 @@ __device__ __forceinline__ void kahan_pixel(float ks[8], float kc[8], float T, u
 
 // A lane's share of a strip (StripPlan): the exact float offsets of its first
 // pixel from the POI, that pixel's byte offset in the gradient plane from the
-// subset's corner, and its row count (low half; 0: the lane has no share) with
-// the rows that every share of the strip has at least (high half).  Every POI
-// of a launch has the same subset and ROI width, so one table in LDS serves a
-// workgroup.
+// subset's corner, and, a byte each, its row count (0: the lane has no share),
+// the rows that every share of the strip has at least, and the strip's row
+// shares per column.  Every POI of a launch has the same subset and ROI width,
+// so one table in LDS serves a workgroup.
+//
+// The shares of a column are ranges of rows where the lane keeps a cell's rows
+// (RP), which needs consecutive ones; otherwise the rows are dealt out in
+// turn, so that a wavefront reads neighbouring rows of the LUT or the image.
 struct StripLane {
     float dx, dy;
     uint32_t go;
@@ -345,7 +369,7 @@ struct StripLane {
 };
 
 template <int L>
-__device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P, int t0, int tstride)
+__device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P, bool ranges, int t0, int tstride)
 {
     // constant strip indices: a run-time index would move the plan to scratch
 #pragma unroll
@@ -355,10 +379,10 @@ __device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P,
         const int base = P.Hsub / s.segs, rem = P.Hsub - base * s.segs;
         for (int l = t0; l < L; l += tstride) {
             const int seg = l / s.ncol, m = s.col + l - seg * s.ncol;
-            const int y = seg * base + min(seg, rem);
+            const int y = ranges ? seg * base + min(seg, rem) : seg;
             const int rows = seg < s.segs ? base + (seg < rem ? 1 : 0) : 0;
             tab[k * L + l] = {(float)(m - P.Sx), (float)(y - P.Sy), 4u * (uint32_t)(y * P.rw + m),
-                              (uint32_t)rows | ((uint32_t)base << 16)};
+                              (uint32_t)(rows | (base << 8) | (s.segs << 16))};
         }
     }
 }
@@ -376,7 +400,7 @@ __device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P,
 // scalar add, and of the sums only S = sum g T needs a product per pixel: the
 // dx-weighted sum is dx S, and the dy-weighted one follows from the running
 // sums, sum_i i g_i T_i = m S - sum_i S_i over m rows (S_i the running sum
-// after row i: Abel's summation by parts).  S runs on from strip to strip;
+// after row i: Abel's summation by parts; rows that are STEP apart scale it).  S runs on from strip to strip;
 // what it held when a strip began is taken out again (a1, a2 below).  Where T
 // is integer-valued every term is an integer below 2^53, so these sums stay
 // exact there, as direct ones would be.
@@ -433,6 +457,7 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
             wy = (cy + Wm[4] * dy) + Wm[5];
         }
     };
+    double step_d = 1.0;       // rows from a lane's pixel to its next one
     // so (wave-uniform) is the pixel's row offset in the gradient plane
     auto gradient = [&](uint32_t go, int so) { return __builtin_amdgcn_raw_buffer_load_b32(g2r, (int)go, so, 0); };
     auto accumulate = [&](float T, uint32_t g, float dx, float dy) {
@@ -449,9 +474,9 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
         st += Td;
         stt = fma(Td, Td, stt);
         a0 = fma(gx, Td, a0);
-        a2 -= a0;
+        a2 = fma(-step_d, a0, a2);
         b0 = fma(gy, Td, b0);
-        b2 -= b0;
+        b2 = fma(-step_d, b0, b2);
     };
     // one pixel on its own
     auto pixel = [&](float cx, float cy, float dx, float dy, uint32_t go, int so) {
@@ -473,8 +498,12 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
             const float tx = __builtin_amdgcn_fractf(wx), ty = __builtin_amdgcn_fractf(wy);
             if constexpr (RP) {
                 const int o = row_poly_offset(rb, ix, iy);
-                T = column_cubic(row_poly(load_row_poly(rb, o, 0), tx), row_poly(load_row_poly(rb, o, 1), tx),
-                                 row_poly(load_row_poly(rb, o, 2), tx), row_poly(load_row_poly(rb, o, 3), tx), ty);
+                const f32x4 q0 = load_row_poly(rb, o, 0), q1 = load_row_poly(rb, o, 1), q2 = load_row_poly(rb, o, 2),
+                            q3 = load_row_poly(rb, o, 3);
+                if constexpr (INTERP == TWDIC_INTERP_LUT)
+                    T = lut_cubic(q0, q1, q2, q3, tx, ty);
+                else
+                    T = column_cubic(row_poly(q0, tx), row_poly(q1, tx), row_poly(q2, tx), row_poly(q3, tx), ty);
             } else if (INTERP == TWDIC_INTERP_FUSED) {
                 T = interp_fused_s(tb, ix, iy, tx, ty);
             } else {
@@ -487,7 +516,9 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
 #pragma unroll 1
     for (int k = 0; k < nstrips; ++k) {
         const StripLane e = tab[k * L + hl];
-        const int full = __builtin_amdgcn_readfirstlane((int)(e.rows >> 16)), rows = (int)(e.rows & 0xffffu);
+        const int shares = __builtin_amdgcn_readfirstlane((int)e.rows);       // but for the lane's row count
+        const int full = (shares >> 8) & 0xff, step = RP ? 1 : shares >> 16, rows = (int)(e.rows & 0xffu);
+        step_d = (double)step;
         if (rows > 0) {
             const uint32_t go = gcorner + e.go;
             const double ddx = (double)e.dx, ddy = (double)e.dy;
@@ -516,7 +547,7 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
 #pragma unroll
                 for (int i = 0; i < 4; ++i) q[i] = load_row_poly(rb, o, i);
                 uint32_t g = gradient(go, 0);
-                auto step = [&](auto k) {
+                auto next = [&](auto k) {
                     constexpr int K = decltype(k)::value;
                     warp(cx, cy, dy, wx, wy);
                     float tx = wx - fx, ty = wy - fy;       // exact; in [0, 1) in the expected cell
@@ -531,13 +562,19 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
 #pragma unroll
                         for (int i = 0; i < 4; ++i) q[(K + i) & 3] = load_row_poly(rb, o, i);
                     }
-                    const float R0 = row_poly(q[K], tx);
-                    q[K] = load_row_poly(rb, o, 4);
                     so += 4 * rw;
                     const uint32_t gn = gradient(go, so);
-                    const float R1 = row_poly(q[(K + 1) & 3], tx), R2 = row_poly(q[(K + 2) & 3], tx),
-                                R3 = row_poly(q[(K + 3) & 3], tx);
-                    accumulate(column_cubic(R0, R1, R2, R3, ty), g, e.dx, dy);
+                    float T;
+                    if constexpr (INTERP == TWDIC_INTERP_LUT) {
+                        T = lut_cubic(q[K], q[(K + 1) & 3], q[(K + 2) & 3], q[(K + 3) & 3], tx, ty);
+                        q[K] = load_row_poly(rb, o, 4);
+                    } else {
+                        const float R0 = row_poly(q[K], tx);
+                        q[K] = load_row_poly(rb, o, 4);
+                        T = column_cubic(R0, row_poly(q[(K + 1) & 3], tx), row_poly(q[(K + 2) & 3], tx),
+                                         row_poly(q[(K + 3) & 3], tx), ty);
+                    }
+                    accumulate(T, g, e.dx, dy);
                     // keep the compiler from sinking this pixel's arithmetic below the next ones' loads
                     asm volatile("" : "+v"(st), "+v"(stt), "+v"(a0), "+v"(a2), "+v"(b0), "+v"(b2));
                     g = gn;
@@ -549,18 +586,18 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                 const int quads = full >> 2, left = rows - 4 * quads;
 #pragma unroll 1
                 for (int r = 0; r < quads; ++r) {
-                    step(integral_constant<int, 0>{});
-                    step(integral_constant<int, 1>{});
-                    step(integral_constant<int, 2>{});
-                    step(integral_constant<int, 3>{});
+                    next(integral_constant<int, 0>{});
+                    next(integral_constant<int, 1>{});
+                    next(integral_constant<int, 2>{});
+                    next(integral_constant<int, 3>{});
                 }
                 if (left > 0) {
-                    step(integral_constant<int, 0>{});
+                    next(integral_constant<int, 0>{});
                     if (left > 1) {
-                        step(integral_constant<int, 1>{});
+                        next(integral_constant<int, 1>{});
                         if (left > 2) {
-                            step(integral_constant<int, 2>{});
-                            if (left > 3) step(integral_constant<int, 3>{});
+                            next(integral_constant<int, 2>{});
+                            if (left > 3) next(integral_constant<int, 3>{});
                         }
                     }
                 }
@@ -568,12 +605,12 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
 #pragma unroll 1
                 for (int r = 0; r < full; ++r) {
                     pixel(cx, cy, e.dx, dy, go, so);
-                    dy += 1.f;
-                    so += 4 * rw;
+                    dy += (float)step;
+                    so += 4 * rw * step;
                 }
                 if (rows > full) pixel(cx, cy, e.dx, dy, go, so);
             }
-            const double end = ddy + (double)rows;
+            const double end = ddy + step_d * (double)rows;
             a1 = fma(ddx, a0, a1);
             a2 = fma(end, a0, a2);
             b1 = fma(ddx, b0, b1);
@@ -774,7 +811,7 @@ __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_icgn(IcgnParams P)
     const int first = xcd_block(blockIdx.x, gridDim.x) * G;
     const int slot = threadIdx.x / L, poi = first + slot;
     copy_ref_state(rs, P.refstate, first, G, P.n, threadIdx.x, 256);
-    fill_strips<L>(tab, P, threadIdx.x, 256);
+    fill_strips<L>(tab, P, RP, threadIdx.x, 256);
     __syncthreads();
     if (poi >= P.n) return;
     icgn_poi_t<L, INTERP, RP, K32>(P, poi, threadIdx.x & 63, tab, rs[slot]);
@@ -801,7 +838,7 @@ __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_batch_icgn_wg(cons
     const int first = __builtin_amdgcn_readfirstlane(it.y);
     const int slot = threadIdx.x / L, poi = first + slot;
     copy_ref_state(rs, P.refstate, first, G, P.n, threadIdx.x, 256);
-    fill_strips<L>(tab, P, threadIdx.x, 256);
+    fill_strips<L>(tab, P, ALL_RP || P.rp != nullptr, threadIdx.x, 256);
     __syncthreads();
     if (poi >= P.n) return;
     if constexpr (ALL_RP)
@@ -873,9 +910,9 @@ __global__ __launch_bounds__(256) void k_batch_icgn(const PairDesc* __restrict__
             __builtin_amdgcn_wave_barrier();
             copy_ref_state(rs[wave], P.refstate, poi, 1, P.n, lane, 64);
             if (P.lanes == 64)
-                fill_strips<64>(tab, P, lane, 64);
+                fill_strips<64>(tab, P, P.rp != nullptr, lane, 64);
             else
-                fill_strips<32>(tab, P, lane, 64);
+                fill_strips<32>(tab, P, P.rp != nullptr, lane, 64);
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
             if (P.lanes == 64)
@@ -934,8 +971,8 @@ static void launch_icgn_r(const IcgnParams& p, int variant, hipStream_t st)
 template <int INTERP>
 static void launch_icgn_t(const IcgnParams& p, int variant, hipStream_t st)
 {
-    if (INTERP == TWDIC_INTERP_FUSED && p.rp != nullptr)
-        launch_icgn_r<INTERP, INTERP == TWDIC_INTERP_FUSED>(p, variant, st);
+    if (INTERP != TWDIC_INTERP_BSPLINE && p.rp != nullptr)
+        launch_icgn_r<INTERP, INTERP != TWDIC_INTERP_BSPLINE>(p, variant, st);
     else
         launch_icgn_r<INTERP, false>(p, variant, st);
 }

@@ -179,6 +179,15 @@ twdic_status ensure_ref_grads(twdic_ctx* c)
     return TWDIC_OK;
 }
 
+// Whether the bicubic passes read the target's row polynomials: in the fused
+// mode, and in the LUT mode as long as nobody can see the LUT itself (its cells
+// follow exactly from the rows, icgn.hip lut_cubic).  No plane: ROIs past
+// 2^28 pixels.
+bool uses_plane(const twdic_ctx* c)
+{
+    return c->d_rp && (c->cfg.interp == TWDIC_INTERP_FUSED || !c->lut_exposed);
+}
+
 IcgnParams icgn_params(twdic_ctx* c, const int32_t* poi, int n, float* u, float* v, float* p6,
                        int32_t* iters, uint8_t* flags, float* dpnorm)
 {
@@ -189,7 +198,7 @@ IcgnParams icgn_params(twdic_ctx* c, const int32_t* poi, int n, float* u, float*
     p.Sx = g.sx; p.Sy = g.sy; p.Wsub = 2 * g.sx + 1; p.Hsub = 2 * g.sy + 1; p.s = p.Wsub * p.Hsub;
     p.max_iter = g.max_iter; p.delta_p = g.delta_p;
     p.g2 = c->d_g2; p.lut = c->d_lut;
-    p.rp = g.interp == TWDIC_INTERP_FUSED ? c->d_rp : nullptr;    // null when the plane does not fit
+    p.rp = uses_plane(c) ? c->d_rp : nullptr;
     p.refstate = c->d_refstate;
     p.poi = poi; p.n = n;
     set_icgn_layout(p, n);
@@ -202,34 +211,33 @@ IcgnParams icgn_params(twdic_ctx* c, const int32_t* poi, int n, float* u, float*
 namespace {
 
 // The per-target interpolation data of the context's mode, on the context
-// stream: the LUT (LUT, B-spline modes) or the row polynomials (fused mode).
+// stream: the row polynomials (uses_plane) or the LUT.
 // Built once per target; every call rebuilds it once the target buffer has
 // been handed out, since the caller may then write it directly.
 hipError_t launch_target_interp(twdic_ctx* c, hipStream_t st)
 {
     const twdic_config& g = c->cfg;
+    if (uses_plane(c)) return launch_row_poly(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_rp, st);
     if (g.interp == TWDIC_INTERP_LUT)
         // cuBicubicCoefficients, TW_paDIC_cuICGN2D.cu:844-851
         return launch_bicubic_lut(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_lut, st);
     if (g.interp == TWDIC_INTERP_BSPLINE)
         // BicubicSplineCoefficients_s, TW_paDIC_ICGN2D_CPU.cpp:333-340
         return launch_bspline_lut(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_lut, st);
-    if (c->d_rp) return launch_row_poly(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_rp, st);
     return hipSuccess;
 }
 
 twdic_status target_interp_prepare(twdic_ctx* c)
 {
-    bool& valid = c->cfg.interp == TWDIC_INTERP_FUSED ? c->tar_rp_valid : c->tar_pre_valid;
+    bool& valid = c->cfg.interp == TWDIC_INTERP_FUSED || uses_plane(c) ? c->tar_rp_valid : c->tar_pre_valid;
     if (valid && !c->tar_exposed) return TWDIC_OK;
     TW_HIP(c, launch_target_interp(c, c->stream));
     valid = true;
     return TWDIC_OK;
 }
 
-// Everything IC-GN needs before its kernel: reference gradients, the target
-// LUT in the LUT/B-spline modes or the row polynomials in the fused mode, and
-// the per-POI reference state, all on the context stream.
+// Everything IC-GN needs before its kernel: reference gradients, the target's
+// row polynomials or LUT (launch_target_interp), and the per-POI reference state, all on the context stream.
 twdic_status icgn_prepare(twdic_ctx* c, const int32_t* d_poi, int n, float* d_u, float* d_v, float* d_p6,
                           int32_t* d_iters, uint8_t* d_flags, float* d_dpnorm, IcgnParams& p)
 {
@@ -363,9 +371,9 @@ twdic_status twdic_create(const twdic_config* cfg, int device, twdic_ctx** out)
         if ((e = hipMalloc(a.p, a.b)) != hipSuccess) bail(e, "hipMalloc");
         else if ((e = hipMemset(*a.p, 0, a.b)) != hipSuccess) bail(e, "hipMemset");
     }
-    // fused mode: the target's row polynomials (16 bytes per ROI pixel);
-    // without them (ROIs past 2^28 pixels) IC-GN reads the image bytes
-    if (st == TWDIC_OK && cfg->interp == TWDIC_INTERP_FUSED &&
+    // fused and LUT modes: the target's row polynomials (16 bytes per ROI pixel);
+    // without them (ROIs past 2^28 pixels) IC-GN reads the image bytes or the LUT
+    if (st == TWDIC_OK && cfg->interp != TWDIC_INTERP_BSPLINE &&
         row_poly_fits(cfg->roi_x, cfg->roi_y, cfg->roi_w, cfg->roi_h)) {
         if ((e = hipMalloc((void**)&c->d_rp, row_poly_bytes(cfg->roi_w, cfg->roi_h))) != hipSuccess)
             bail(e, "hipMalloc");
@@ -674,9 +682,16 @@ twdic_status twdic_frame_replay(twdic_ctx* c)
         c->refstate_poi = ip.poi;
         c->refstate_n = ip.n;
     }
+    // a graph captured before the LUT was handed out builds the row polynomials:
+    // the LUT is kept up beside it
+    const bool plane = ip.rp != nullptr;
+    if (plane && c->cfg.interp == TWDIC_INTERP_LUT && c->lut_exposed) {
+        TW_HIP(c, launch_target_interp(c, c->stream));
+        c->tar_pre_valid = true;
+    }
     TW_HIP(c, hipGraphLaunch(c->graph_exec, c->stream));
     // the graph rebuilt the LUT or the row polynomials
-    (c->cfg.interp == TWDIC_INTERP_FUSED ? c->tar_rp_valid : c->tar_pre_valid) = true;
+    (c->cfg.interp == TWDIC_INTERP_FUSED || plane ? c->tar_rp_valid : c->tar_pre_valid) = true;
     return TWDIC_OK;
 }
 
@@ -697,6 +712,14 @@ twdic_status twdic_get_buffer(twdic_ctx* c, int which, void** d_ptr, size_t* byt
     case TWDIC_BUF_REF: p = c->d_ref; b = img; break;
     case TWDIC_BUF_TAR: p = c->d_tar; b = img; c->tar_exposed = true; break;
     default: return fail(c, TWDIC_EINVAL, "unknown buffer");
+    }
+    if (which == TWDIC_BUF_LUT && c->cfg.interp == TWDIC_INTERP_LUT && !c->lut_exposed) {
+        c->lut_exposed = true;
+        // the LUT of the target IC-GN last ran on, if that is still the current one
+        if (c->tar_rp_valid && !c->tar_pre_valid) {
+            TW_HIP(c, launch_target_interp(c, c->stream));
+            c->tar_pre_valid = true;
+        }
     }
     if (which == TWDIC_BUF_RX || which == TWDIC_BUF_RY) {
         twdic_status st = ensure_ref_grads(c);

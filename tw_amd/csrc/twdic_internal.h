@@ -129,7 +129,7 @@ struct IcgnParams {
     double delta_p;           // the caller's float, widened: the loop test compares in FP64
     const uint32_t* g2;       // reference gradients (2Rx, 2Ry) as int16 pairs, ROI-relative
     const float* lut;         // target LUT [rh][rw][16]
-    const float4* rp;         // target row polynomials [rh + 2][rw] (fused mode; null: from the image bytes)
+    const float4* rp;         // target row polynomials [rh + 2][rw] (fused and LUT modes; null: from the image bytes or the LUT)
     double* refstate;         // kRefStateStride doubles per POI
     const int32_t* poi;
     int n;
@@ -266,6 +266,7 @@ struct twdic_ctx {
     bool tar_pre_valid = false;       // Tx/Ty/Txy/LUT match d_tar
     bool tar_rp_valid = false;        // d_rp matches d_tar
     bool tar_exposed = false;         // d_tar was handed out: it may change without twdic_set_target
+    bool lut_exposed = false;         // d_lut was handed out: the LUT mode keeps it up and reads it
     uint64_t ref_version = 0;
     // per-reference POI state cache key
     double* d_refstate = nullptr;
