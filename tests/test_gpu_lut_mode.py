@@ -1,7 +1,8 @@
-"""The LUT interpolation mode reads the target's row polynomials as long as the
-LUT buffer has not been handed out (twdic_get_buffer), and the LUT itself from
-then on.  Both evaluate the same cell polynomials in the same order from exact
-coefficients, so every output must be equal bit for bit; the LUT handed out
+"""The LUT and B-spline interpolation modes read layouts of their own (the
+target's row polynomials, and planes of coefficients) as long as the LUT buffer
+has not been handed out (twdic_get_buffer), and the LUT itself from then on.
+Both evaluate the same cell polynomials in the same order from the same or
+exact coefficients, so every output must be equal bit for bit; the LUT handed out
 must be the current target's, from the calls that ran before and after, eager
 and through a captured frame."""
 import numpy as np
@@ -36,13 +37,17 @@ def _lut(ctx, c):
 
 
 @pytest.mark.parametrize("S", [10, 15, 24])
-def test_plane_and_table_agree_bitwise(S):
+@pytest.mark.parametrize("interp", [api.INTERP_LUT, api.INTERP_BSPLINE])
+def test_own_layout_and_table_agree_bitwise(interp, S):
     c = cases.speckle_512()
-    c.S = S
+    c.S, c.margin = S, 0
+    table_of = oracle.bicubic_lut
+    if interp == api.INTERP_BSPLINE:
+        c.roi, table_of = (1, 1, 508, 508), oracle.bspline_lut
     tar2 = np.ascontiguousarray(np.roll(c.tar, 1, axis=1))
     poi = np.random.default_rng(S).integers(60, 452, (700, 2)).astype(np.int32)
-    print(f"[gpu-test] LUT mode S {S}", flush=True)
-    with ctx_for(c, interp=api.INTERP_LUT) as plane, ctx_for(c, interp=api.INTERP_LUT) as table:
+    print(f"[gpu-test] interpolation mode {interp} S {S}", flush=True)
+    with ctx_for(c, interp=interp) as plane, ctx_for(c, interp=interp) as table:
         table.buffer(api.BUF_LUT)                                   # handed out before the first call
         pd, td = (x.array(poi.shape, np.int32).upload(poi) for x in (plane, table))
         for k, tar in enumerate((c.tar, tar2)):
@@ -53,17 +58,17 @@ def test_plane_and_table_agree_bitwise(S):
             assert (b["flags"] == 0).mean() > 0.9
             for f in OUT:
                 assert np.array_equal(a[f], b[f]), (k, f)
-            assert np.array_equal(_lut(table, c), oracle.bicubic_lut(tar, *c.roi))
+            assert np.array_equal(_lut(table, c), table_of(tar, *c.roi))
         plane.frame_capture(*args)
         plane.set_target(c.tar)
         table.set_target(c.tar)
         b, _ = _frame(table, td, len(poi))
         for handed in (False, True):
             if handed:                                              # the replay's target, then kept up
-                assert np.array_equal(_lut(plane, c), oracle.bicubic_lut(c.tar, *c.roi))
+                assert np.array_equal(_lut(plane, c), table_of(c.tar, *c.roi))
                 plane.set_target(tar2)
                 _frame(plane, pd, len(poi), replay=True)
-                assert np.array_equal(_lut(plane, c), oracle.bicubic_lut(tar2, *c.roi))
+                assert np.array_equal(_lut(plane, c), table_of(tar2, *c.roi))
                 plane.set_target(c.tar)
             a, _ = _frame(plane, pd, len(poi), replay=True)
             for f in OUT:

@@ -73,15 +73,31 @@ __device__ __forceinline__ bool group_any(bool pred, int lane)
 }
 
 // Bicubic value from the materialised LUT cell (16 floats, 4k+l ~ y^k x^l).
-__device__ __forceinline__ float interp_lut(const float* __restrict__ lut, uint32_t cell, float tx, float ty)
+__device__ __forceinline__ float lut_poly(float4 r0, float4 r1, float4 r2, float4 r3, float tx, float ty)
 {
-    const float4* c = reinterpret_cast<const float4*>(lut) + (size_t)cell * 4;
-    float4 r0 = c[0], r1 = c[1], r2 = c[2], r3 = c[3];
     float a0 = fmaf(fmaf(fmaf(r0.w, tx, r0.z), tx, r0.y), tx, r0.x);
     float a1 = fmaf(fmaf(fmaf(r1.w, tx, r1.z), tx, r1.y), tx, r1.x);
     float a2 = fmaf(fmaf(fmaf(r2.w, tx, r2.z), tx, r2.y), tx, r2.x);
     float a3 = fmaf(fmaf(fmaf(r3.w, tx, r3.z), tx, r3.y), tx, r3.x);
     return fmaf(fmaf(fmaf(a3, ty, a2), ty, a1), ty, a0);
+}
+
+__device__ __forceinline__ float interp_lut(const float* __restrict__ lut, uint32_t cell, float tx, float ty)
+{
+    const float4* c = reinterpret_cast<const float4*>(lut) + (size_t)cell * 4;
+    return lut_poly(c[0], c[1], c[2], c[3], tx, ty);
+}
+
+// The same from four planes, plane k holding every cell's coefficients of y^k:
+// neighbouring lanes' 16 bytes are then neighbours in memory, where the
+// 64-byte cells put two of them in a cache line, four times over (the L1 then
+// looked up a line in every cycle).  28k POIs of 33x33: 0.45 ms from cells,
+// 0.39 ms from planes, where the L2 serves 23 TB/s; ranges or dealt rows, two
+// rows per trip and three instead of five waves per SIMD take the same.
+__device__ __forceinline__ float interp_planes(const float4* __restrict__ planes, size_t cells, uint32_t cell, float tx,
+                                               float ty)
+{
+    return lut_poly(planes[cell], planes[cells + cell], planes[2 * cells + cell], planes[3 * cells + cell], tx, ty);
 }
 
 // The same bicubic interpolant evaluated from the 4x4 pixel neighbourhood:
@@ -360,7 +376,7 @@ __device__ __forceinline__ void kahan_pixel(float ks[8], float kc[8], float T, u
 // so one table in LDS serves a workgroup.
 //
 // The shares of a column are ranges of rows where the lane keeps a cell's rows
-// (RP), which needs consecutive ones; otherwise the rows are dealt out in
+// (row polynomials), which needs consecutive ones; otherwise the rows are dealt out in
 // turn, so that a wavefront reads neighbouring rows of the LUT or the image.
 struct StripLane {
     float dx, dy;
@@ -392,8 +408,9 @@ __device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P,
 // first pass at integer target pixels (:610-637); otherwise bicubic
 // (:757-792).  Returns false when a warped pixel of the group's POI leaves the
 // ROI.  Accumulates sum T, sum T^2 and the six sum SD_k T / 2 (the gradient
-// plane stores 2 Rx, 2 Ry) in FP64.  RP: the fused bicubic passes evaluate the
-// target's row polynomials (P.rp) instead of the image bytes.
+// plane stores 2 Rx, 2 Ry) in FP64.  RP: the later passes read P.rp, the
+// target's row polynomials or B-spline planes, instead of the image bytes or
+// the LUT.
 //
 // Each lane walks down one column at a time.  Along a column dx is constant,
 // so POI + W0 dx is formed once, the gradient offset of the next row is a
@@ -427,12 +444,13 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     // the fused interpolation from the bytes returns T 2^-24 (interp_rows_s);
     // the sums are scaled back at the end, exactly
     constexpr bool SCALED = !INT && INTERP == TWDIC_INTERP_FUSED && !RP;
-    constexpr bool ROLL = RP && !INT && !CHECK && !K32;
+    constexpr bool ROWS = RP && INTERP != TWDIC_INTERP_BSPLINE;      // the target's rows as polynomials
+    constexpr bool ROLL = ROWS && !INT && !CHECK && !K32;
     const int sx0 = P.sx0, sy0 = P.sy0, rw = P.rw, rh = P.rh;
     const TargetBuf tb = target_buf(P);
     const __amdgpu_buffer_rsrc_t g2r =
         __builtin_amdgcn_make_buffer_rsrc((void*)P.g2, (short)0, 4 * rw * rh, 0x00020000);
-    const RowPolyBuf rb = RP ? row_poly_buf(P) : RowPolyBuf{};
+    const RowPolyBuf rb = ROWS ? row_poly_buf(P) : RowPolyBuf{};
     const float fpx = (float)px, fpy = (float)py;
     double st = 0.0, stt = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0, b0 = 0.0, b1 = 0.0, b2 = 0.0;
     float ks[8] = {}, kc[8] = {};
@@ -496,7 +514,9 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
         } else if (interior) {
             // :771-772; wx, wy >= 1 here, so x - (float)(int)x is fract(x), exactly
             const float tx = __builtin_amdgcn_fractf(wx), ty = __builtin_amdgcn_fractf(wy);
-            if constexpr (RP) {
+            if constexpr (RP && INTERP == TWDIC_INTERP_BSPLINE) {
+                T = interp_planes(P.rp, (size_t)rw * rh, (uint32_t)((iy - sy0) * rw + (ix - sx0)), tx, ty);
+            } else if constexpr (RP) {
                 const int o = row_poly_offset(rb, ix, iy);
                 const f32x4 q0 = load_row_poly(rb, o, 0), q1 = load_row_poly(rb, o, 1), q2 = load_row_poly(rb, o, 2),
                             q3 = load_row_poly(rb, o, 3);
@@ -517,7 +537,7 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     for (int k = 0; k < nstrips; ++k) {
         const StripLane e = tab[k * L + hl];
         const int shares = __builtin_amdgcn_readfirstlane((int)e.rows);       // but for the lane's row count
-        const int full = (shares >> 8) & 0xff, step = RP ? 1 : shares >> 16, rows = (int)(e.rows & 0xffu);
+        const int full = (shares >> 8) & 0xff, step = ROWS ? 1 : shares >> 16, rows = (int)(e.rows & 0xffu);
         step_d = (double)step;
         if (rows > 0) {
             const uint32_t go = gcorner + e.go;
@@ -811,7 +831,7 @@ __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_icgn(IcgnParams P)
     const int first = xcd_block(blockIdx.x, gridDim.x) * G;
     const int slot = threadIdx.x / L, poi = first + slot;
     copy_ref_state(rs, P.refstate, first, G, P.n, threadIdx.x, 256);
-    fill_strips<L>(tab, P, RP, threadIdx.x, 256);
+    fill_strips<L>(tab, P, RP && INTERP != TWDIC_INTERP_BSPLINE, threadIdx.x, 256);
     __syncthreads();
     if (poi >= P.n) return;
     icgn_poi_t<L, INTERP, RP, K32>(P, poi, threadIdx.x & 63, tab, rs[slot]);
@@ -971,8 +991,8 @@ static void launch_icgn_r(const IcgnParams& p, int variant, hipStream_t st)
 template <int INTERP>
 static void launch_icgn_t(const IcgnParams& p, int variant, hipStream_t st)
 {
-    if (INTERP != TWDIC_INTERP_BSPLINE && p.rp != nullptr)
-        launch_icgn_r<INTERP, INTERP != TWDIC_INTERP_BSPLINE>(p, variant, st);
+    if (p.rp != nullptr)
+        launch_icgn_r<INTERP, true>(p, variant, st);
     else
         launch_icgn_r<INTERP, false>(p, variant, st);
 }

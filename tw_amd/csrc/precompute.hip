@@ -74,6 +74,8 @@ hipError_t launch_gradients(const uint8_t* img, int stride, int sx0, int sy0, in
 // B-spline basis B, rotated by 180 degrees.  FP32, every product and sum
 // rounded separately in the reference's order.  Every ROI pixel gets
 // coefficients (the caller guarantees a 2-pixel frame right and below).
+// PLANES: the y^k coefficients of all cells in plane k (float4[4][rh][rw])
+// instead of 16 floats per cell.
 // ---------------------------------------------------------------------------
 namespace {
 __device__ __forceinline__ float bsp_cp(int k, int l)
@@ -94,6 +96,7 @@ __device__ __forceinline__ float bsp_base(int k, int l)
 }
 }  // namespace
 
+template <bool PLANES>
 __global__ __launch_bounds__(256) void k_bspline_lut(const uint8_t* __restrict__ img, int stride, int sx0, int sy0,
                                                      int rw, int rh, float* __restrict__ lut)
 {
@@ -129,17 +132,27 @@ __global__ __launch_bounds__(256) void k_bspline_lut(const uint8_t* __restrict__
                 for (int n = 0; n < 4; ++n) a = a + bsp_base(k, m) * bsp_base(l, n) * beta[n][m];
             c[k][l] = a;
         }
-    float4* out = reinterpret_cast<float4*>(lut + ((size_t)y * rw + x) * 16);
+    const size_t cell = (size_t)y * rw + x, at = PLANES ? cell : 4 * cell, step = PLANES ? (size_t)rw * rh : 1;
+    float4* out = reinterpret_cast<float4*>(lut);
 #pragma unroll
     for (int k = 0; k < 4; ++k)      // rotated by 180 degrees (:591-599)
-        out[k] = make_float4(c[3 - k][3], c[3 - k][2], c[3 - k][1], c[3 - k][0]);
+        out[at + k * step] = make_float4(c[3 - k][3], c[3 - k][2], c[3 - k][1], c[3 - k][0]);
 }
 
 hipError_t launch_bspline_lut(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float* lut,
                               hipStream_t st)
 {
     dim3 grid((rw + 63) / 64, (rh + 3) / 4);
-    hipLaunchKernelGGL(k_bspline_lut, grid, dim3(256), 0, st, tar, stride, sx0, sy0, rw, rh, lut);
+    hipLaunchKernelGGL(k_bspline_lut<false>, grid, dim3(256), 0, st, tar, stride, sx0, sy0, rw, rh, lut);
+    return hipGetLastError();
+}
+
+hipError_t launch_bspline_planes(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* planes,
+                                 hipStream_t st)
+{
+    dim3 grid((rw + 63) / 64, (rh + 3) / 4);
+    hipLaunchKernelGGL(k_bspline_lut<true>, grid, dim3(256), 0, st, tar, stride, sx0, sy0, rw, rh,
+                       reinterpret_cast<float*>(planes));
     return hipGetLastError();
 }
 

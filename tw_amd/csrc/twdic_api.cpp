@@ -179,10 +179,11 @@ twdic_status ensure_ref_grads(twdic_ctx* c)
     return TWDIC_OK;
 }
 
-// Whether the bicubic passes read the target's row polynomials: in the fused
-// mode, and in the LUT mode as long as nobody can see the LUT itself (its cells
-// follow exactly from the rows, icgn.hip lut_cubic).  No plane: ROIs past
-// 2^28 pixels.
+// Whether IC-GN reads the target from d_rp: always in the fused mode (row
+// polynomials), in the LUT and B-spline modes as long as nobody can see the
+// LUT itself (bicubic cells follow exactly from the row polynomials, icgn.hip
+// lut_cubic; the B-spline coefficients are kept as planes).  No row
+// polynomials: ROIs past 2^28 pixels.
 bool uses_plane(const twdic_ctx* c)
 {
     return c->d_rp && (c->cfg.interp == TWDIC_INTERP_FUSED || !c->lut_exposed);
@@ -211,12 +212,14 @@ IcgnParams icgn_params(twdic_ctx* c, const int32_t* poi, int n, float* u, float*
 namespace {
 
 // The per-target interpolation data of the context's mode, on the context
-// stream: the row polynomials (uses_plane) or the LUT.
+// stream: the row polynomials or planes (uses_plane), or the LUT.
 // Built once per target; every call rebuilds it once the target buffer has
 // been handed out, since the caller may then write it directly.
 hipError_t launch_target_interp(twdic_ctx* c, hipStream_t st)
 {
     const twdic_config& g = c->cfg;
+    if (uses_plane(c) && g.interp == TWDIC_INTERP_BSPLINE)
+        return launch_bspline_planes(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_rp, st);
     if (uses_plane(c)) return launch_row_poly(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_rp, st);
     if (g.interp == TWDIC_INTERP_LUT)
         // cuBicubicCoefficients, TW_paDIC_cuICGN2D.cu:844-851
@@ -372,12 +375,12 @@ twdic_status twdic_create(const twdic_config* cfg, int device, twdic_ctx** out)
         else if ((e = hipMemset(*a.p, 0, a.b)) != hipSuccess) bail(e, "hipMemset");
     }
     // fused and LUT modes: the target's row polynomials (16 bytes per ROI pixel);
-    // without them (ROIs past 2^28 pixels) IC-GN reads the image bytes or the LUT
-    if (st == TWDIC_OK && cfg->interp != TWDIC_INTERP_BSPLINE &&
-        row_poly_fits(cfg->roi_x, cfg->roi_y, cfg->roi_w, cfg->roi_h)) {
-        if ((e = hipMalloc((void**)&c->d_rp, row_poly_bytes(cfg->roi_w, cfg->roi_h))) != hipSuccess)
-            bail(e, "hipMalloc");
-    }
+    // without them (ROIs past 2^28 pixels) IC-GN reads the image bytes or the LUT.
+    // B-spline mode: the coefficient planes (64 bytes per ROI pixel).
+    const size_t rp = cfg->interp == TWDIC_INTERP_BSPLINE ? roi * 64
+                      : row_poly_fits(cfg->roi_x, cfg->roi_y, cfg->roi_w, cfg->roi_h)
+                          ? row_poly_bytes(cfg->roi_w, cfg->roi_h) : 0;
+    if (st == TWDIC_OK && rp && (e = hipMalloc((void**)&c->d_rp, rp)) != hipSuccess) bail(e, "hipMalloc");
     for (int i = 0; i < 16 && st == TWDIC_OK; ++i)
         if ((e = hipEventCreate(&c->ev[i])) != hipSuccess) bail(e, "hipEventCreate");
     for (int i = 0; i <= twdic_ctx::kMaxFrameChunks && st == TWDIC_OK; ++i)
@@ -682,15 +685,15 @@ twdic_status twdic_frame_replay(twdic_ctx* c)
         c->refstate_poi = ip.poi;
         c->refstate_n = ip.n;
     }
-    // a graph captured before the LUT was handed out builds the row polynomials:
+    // a graph captured before the LUT was handed out builds the rows or planes:
     // the LUT is kept up beside it
     const bool plane = ip.rp != nullptr;
-    if (plane && c->cfg.interp == TWDIC_INTERP_LUT && c->lut_exposed) {
+    if (plane && c->cfg.interp != TWDIC_INTERP_FUSED && c->lut_exposed) {
         TW_HIP(c, launch_target_interp(c, c->stream));
         c->tar_pre_valid = true;
     }
     TW_HIP(c, hipGraphLaunch(c->graph_exec, c->stream));
-    // the graph rebuilt the LUT or the row polynomials
+    // the graph rebuilt the LUT, or the rows or planes
     (c->cfg.interp == TWDIC_INTERP_FUSED || plane ? c->tar_rp_valid : c->tar_pre_valid) = true;
     return TWDIC_OK;
 }
@@ -713,7 +716,7 @@ twdic_status twdic_get_buffer(twdic_ctx* c, int which, void** d_ptr, size_t* byt
     case TWDIC_BUF_TAR: p = c->d_tar; b = img; c->tar_exposed = true; break;
     default: return fail(c, TWDIC_EINVAL, "unknown buffer");
     }
-    if (which == TWDIC_BUF_LUT && c->cfg.interp == TWDIC_INTERP_LUT && !c->lut_exposed) {
+    if (which == TWDIC_BUF_LUT && c->cfg.interp != TWDIC_INTERP_FUSED && !c->lut_exposed) {
         c->lut_exposed = true;
         // the LUT of the target IC-GN last ran on, if that is still the current one
         if (c->tar_rp_valid && !c->tar_pre_valid) {

@@ -129,7 +129,8 @@ struct IcgnParams {
     double delta_p;           // the caller's float, widened: the loop test compares in FP64
     const uint32_t* g2;       // reference gradients (2Rx, 2Ry) as int16 pairs, ROI-relative
     const float* lut;         // target LUT [rh][rw][16]
-    const float4* rp;         // target row polynomials [rh + 2][rw] (fused and LUT modes; null: from the image bytes or the LUT)
+    const float4* rp;         // target row polynomials [rh + 2][rw] (fused, LUT modes) or B-spline planes
+                              // [4][rh][rw]; null: from the image bytes or the LUT
     double* refstate;         // kRefStateStride doubles per POI
     const int32_t* poi;
     int n;
@@ -174,6 +175,9 @@ hipError_t launch_gradients(const uint8_t* img, int stride, int sx0, int sy0, in
                             float* gx, float* gy, float* gxy, uint32_t* g2, hipStream_t st);
 hipError_t launch_bspline_lut(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float* lut,
                               hipStream_t st);
+// the same coefficients as planes, float4[4][rh][rw]
+hipError_t launch_bspline_planes(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* planes,
+                                 hipStream_t st);
 // Catmull-Rom row polynomials of the target, (rh + 2) x rw entries of 16 bytes
 hipError_t launch_row_poly(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* rp,
                            hipStream_t st);
@@ -266,7 +270,7 @@ struct twdic_ctx {
     bool tar_pre_valid = false;       // Tx/Ty/Txy/LUT match d_tar
     bool tar_rp_valid = false;        // d_rp matches d_tar
     bool tar_exposed = false;         // d_tar was handed out: it may change without twdic_set_target
-    bool lut_exposed = false;         // d_lut was handed out: the LUT mode keeps it up and reads it
+    bool lut_exposed = false;         // d_lut was handed out: the LUT modes keep it up and read it
     uint64_t ref_version = 0;
     // per-reference POI state cache key
     double* d_refstate = nullptr;
