@@ -61,8 +61,12 @@ struct twdic_batch {
     int lanes = 4;                    // TWDIC_BATCH_STREAMS (1..4)
     // flat form: one launch per stage and kernel form over all pairs
     bool flat = true;                 // TWDIC_BATCH_FORM=direct selects the direct form
-    int2* d_mitems[4] = {};           // FFT-CC items (pair, POI) per matrix-core kernel form (mma_form)
-    int64_t nm[4] = {};
+    struct WindowItems {              // FFT-CC items (pair, POI) of the pairs with window edge N
+        int N;
+        int2* d;
+        int64_t n;
+    };
+    std::vector<WindowItems> mitems;
     // IC-GN workgroup items (pair, first POI): half-wavefront (list 0) or whole
     // wavefront (list 1) per POI, by the pair's POI count (icgn_lanes_for)
     int2* d_wg[2] = {};
@@ -109,11 +113,12 @@ void release(twdic_batch* b)
     b->graph_exec = nullptr;
     b->graph = nullptr;
     void* bufs[] = {b->d_desc, b->d_items, b->d_fitems[0], b->d_fitems[1], b->d_fitems[2], b->d_g2, b->d_state,
-                    b->d_zncc_scratch, b->d_counters, b->d_mitems[0], b->d_mitems[1], b->d_mitems[2],
-                    b->d_mitems[3], b->d_wg[0], b->d_wg[1], b->d_rp};
+                    b->d_zncc_scratch, b->d_counters, b->d_wg[0], b->d_wg[1], b->d_rp};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
-    for (int f = 0; f < 4; ++f) { b->d_mitems[f] = nullptr; b->nm[f] = 0; }
+    for (auto& m : b->mitems)
+        if (m.d) (void)hipFree(m.d);
+    b->mitems.clear();
     for (int t = 0; t < 2; ++t) { b->d_wg[t] = nullptr; b->nwg[t] = 0; }
     for (int c = 0; c < 3; ++c) b->nf[c] = 0;
     for (auto& kv : b->tw) (void)hipFree(kv.second);
@@ -260,14 +265,13 @@ twdic_status run_direct(twdic_batch* b, bool fftcc, bool icgn)
     return TWDIC_OK;
 }
 
-// Flat form: FFT-CC per matrix-core kernel form, then IC-GN per lane
+// Flat form: FFT-CC per window edge, then IC-GN per lane
 // count, each one launch over the items of every pair on the batch stream.  The
 // same per-POI device code as the single-context kernels.
 twdic_status enqueue_flat(twdic_batch* b, bool fftcc, bool icgn)
 {
     if (fftcc)
-        for (int f = 0; f < 4; ++f)
-            if (b->nm[f]) TB_HIP(b, launch_batch_fftcc_mma(b->d_desc, b->d_mitems[f], (int)b->nm[f], f, b->stream));
+        for (const auto& m : b->mitems) TB_HIP(b, launch_batch_fftcc_mma(b->d_desc, m.d, (int)m.n, m.N, b->stream));
     if (icgn) TB_HIP(b, launch_batch_row_poly(b->d_desc, (int)b->pairs.size(), b->max_rh, b->stream));
     if (icgn)
         for (int t = 0; t < 2; ++t)
@@ -405,22 +409,25 @@ twdic_status set_pairs_impl(twdic_batch* b, const twdic_pair* pairs, int npairs)
         }
     }
     if (total) TB_HIP(b, hipMemcpy(b->d_items, items.data(), sizeof(int2) * total, hipMemcpyHostToDevice));
-    // flat form: FFT-CC items per kernel form, IC-GN items of 256 / lanes POIs of one pair
-    std::vector<int2> mitems[4], wg[2];
+    // flat form: FFT-CC items per window edge, IC-GN items of 256 / lanes POIs of one pair
+    std::map<int, std::vector<int2>> mitems;
+    std::vector<int2> wg[2];
     for (int i = 0; i < npairs; ++i) {
         const twdic_pair& p = b->pairs[i];
-        auto& mi = mitems[mma_form(p.fft_n)];
+        auto& mi = mitems[p.fft_n];
         for (int k = 0; k < p.n; ++k) mi.push_back(make_int2(i, k));
         const int lanes = icgn_lanes_for(p.n), per_wg = 256 / lanes;
         auto& w = wg[lanes == 64 ? 1 : 0];
         for (int k = 0; k < p.n; k += per_wg) w.push_back(make_int2(i, k));
     }
-    for (int f = 0; f < 4; ++f) {
-        b->nm[f] = (int64_t)mitems[f].size();
-        if (b->nm[f] > INT32_MAX) return bfail(b, TWDIC_EINVAL, "more than 2^31 - 1 POIs in one FFT-CC kernel form");
-        if (!b->nm[f]) continue;
-        TB_HIP(b, alloc((void**)&b->d_mitems[f], sizeof(int2) * mitems[f].size()));
-        TB_HIP(b, hipMemcpy(b->d_mitems[f], mitems[f].data(), sizeof(int2) * mitems[f].size(), hipMemcpyHostToDevice));
+    for (const auto& [N, list] : mitems) {
+        if (list.empty()) continue;
+        if (list.size() > (size_t)INT32_MAX)
+            return bfail(b, TWDIC_EINVAL, "more than 2^31 - 1 POIs in one FFT-CC window edge");
+        b->mitems.push_back({N, nullptr, (int64_t)list.size()});
+        int2*& d = b->mitems.back().d;
+        TB_HIP(b, alloc((void**)&d, sizeof(int2) * list.size()));
+        TB_HIP(b, hipMemcpy(d, list.data(), sizeof(int2) * list.size(), hipMemcpyHostToDevice));
     }
     for (int t = 0; t < 2; ++t) {
         b->nwg[t] = (int64_t)wg[t].size();
@@ -442,7 +449,7 @@ twdic_status set_pairs_impl(twdic_batch* b, const twdic_pair* pairs, int npairs)
         return false;
     };
     bool bad = bad_item(items, 1) || bad_item(wg[0], 4) || bad_item(wg[1], 4);
-    for (int f = 0; f < 4 && !bad; ++f) bad = bad_item(mitems[f], 1);
+    for (const auto& kv : mitems) bad = bad || bad_item(kv.second, 1);
     for (int c = 0; c < 3 && !bad; ++c) bad = bad_item(fitems[c], 1);
     if (bad) return bfail(b, TWDIC_EINVAL, "internal: a work item names no POI of its pair");
     if (kPersistent) {

@@ -15,7 +15,11 @@
 // on the engine, batching or pairing.
 //
 // Engines:
-//   * k_fftcc_mma<NT, N64, TILE> (default, any even N <= 64): the whole
+//   * k_fftcc_dft_mfma<CH, FULL> (default for N = 64 and most sets with 32 < N
+//     <= 60, dft_takes): the surface from fp16 DFTs on the matrix cores, within
+//     a proven error, then the exact integer correlation at the shifts it
+//     leaves in question.
+//   * k_fftcc_mma<NT, N64, TILE> (the other sets; any even N <= 64): the whole
 //     integer correlation surface on the int8 matrix cores, one wavefront per
 //     POI (32 x 32 x 32 tiles; 16 x 16 x 64 tiles for 32 < N <= 48).
 //   * k_fftcc_fft<P> (N = 4P = 32 or 64): FP32 FFTs.  One workgroup of 4N
@@ -1125,10 +1129,11 @@ __global__ __launch_bounds__(64) void k_batch_fftcc_mma(const PairDesc* __restri
 }
 
 // ===========================================================================
-// Matrix-core DFT engine, N = 64: the correlation surface from fp16 2-D DFTs
-// on v_mfma_f32_32x32x16_f16, then the exact integer correlation at every
-// shift the surface leaves within its proven error of the maximum.
+// Matrix-core DFT engine, N = 64 and 32 < N <= 60: the correlation surface from
+// fp16 2-D DFTs on v_mfma_f32_32x32x16_f16, then the exact integer correlation
+// at every shift the surface leaves within its proven error of the maximum.
 //
+// For N = 64:
 //   r = R - a, t = T - b with a, b the rounded window means: integers in
 //   [-255, 255], exact in fp16; the correlation of r and t differs from I[k]
 //   = sum R T(k) by a constant, so it has the same argmax.
@@ -1169,16 +1174,40 @@ __global__ __launch_bounds__(64) void k_batch_fftcc_mma(const PairDesc* __restri
 //   window of pure noise a handful; the count is not capped.)
 //   A workgroup of eight wavefronts, one POI each, shares the fp16 tables in
 //   LDS; the window bytes stay in LDS for the exact stage.
+//
+// For 32 < N <= 60 the same passes run on N x N tables padded with zeros, which
+// also silence the window rows and columns beyond N.  The half spectrum k = 0 ..
+// N / 2 fits the 32 columns, so no column is packed; columns 0 and N / 2, their
+// own conjugates, count once.  Row k = 31 is empty: it carries the mask that
+// keeps rows b >= N from being candidates.  N <= 48 needs three K chunks instead
+// of four (112 MFMAs instead of 144) and 160 registers, so twelve wavefronts, three
+// per SIMD, hide each other's chains of dependent MFMAs and conversions, which
+// bound the engine: .53 ms for 155k POIs at N = 40, .75 ms at N = 56 (188
+// registers, two wavefronts per SIMD).
 // ===========================================================================
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f16x __attribute__((ext_vector_type(16)));
 
-constexpr double kDftBound = 22.0;        // N^2 |C^ - C| / (||r|| ||t||), see above
-// LDS pitch of the R rows (64 B) and the doubled T rows (128 B): 18 and 34
-// dwords put the 8-byte operand reads of 16 consecutive rows on distinct banks
-constexpr int kExR = 72, kExT = 136;
-constexpr int kDftWaves = 8;              // POIs in flight per workgroup (one per wavefront)
+constexpr double kDftBound = 22.0;        // N^2 |C^ - C| / (||r|| ||t||) at N = 64, see above
+// the same over N^2 / 4096 for every even 32 < N <= 60 (largest at N = 54: 25.9)
+constexpr double kDftBoundN = 26.0;
+
+// The POI sets the engine takes (both engines give the same results): N = 64,
+// the even 48 < N <= 60, and 32 < N <= 48 from the count on at which it is the
+// faster one: it starts with its tables, 3 us more than the integer engine for
+// one POI.  (N = 62 leaves the spectrum no free row, see fftcc_dft_mfma_poi.)
+// Against the integer engine, 2048^2 speckle, ms:
+//   N       34         40         48         50         56         60
+//   25      .013/.011  .014/.012  .015/.013  .015/.016  .015/.017  .015/.018
+//   800     .016/.012  .016/.013  .016/.015  .016/.018  .016/.020  .016/.021
+//   1,200   .016/.014  .016/.016  .016/.019  .016/.024  .017/.026  .016/.027
+//   5,000   .025/.034  .023/.038  .025/.044  .03 /.065  .031/.072  .03 /.076
+//   155k    .53 /.69   .53 /.82   .56 /1.00  .73 /1.61  .75 /1.86  .77 /1.96
+inline bool dft_takes(int N, int n)
+{
+    return N == 64 || (N > 48 && N <= 60) || (N > 32 && N <= 48 && n >= 1280);
+}
 
 // F in fp16 as MFMA operands, [table][part][tile][K chunk][lane], lane = 32 h + m,
 // parts re, im, -im:
@@ -1193,16 +1222,22 @@ __device__ h8 g_dft_tab[2][3][2][4][64];
 __device__ h8 g_dft_nyq[2][64];
 int g_dft_cus[64] = {};                        // compute units per device, set by dft_tables_init
 
-// One workgroup: the tables (32 KB, read by all its wavefronts) and, per
-// wavefront, its POI's R rows and doubled T rows as bytes and the second
-// pass's spectrum column 0 (for the j <-> -j unpacking).
+// One workgroup: the tables (read by all its wavefronts) and, per wavefront,
+// its POI's R rows and doubled T rows as bytes and, at N = 64, the second
+// pass's spectrum column 0 (for the j <-> -j unpacking).  CH: K chunks of 16
+// that hold a window edge, 3 for 32 < N <= 48, else 4.  FULL: N = 64.
+// Row pitches of R (16 CH bytes) and T (32 CH): 14 and 26, or 18 and 34,
+// dwords put the 8-byte operand reads of 16 consecutive rows on distinct banks.
+template <int CH, bool FULL>
 struct DftWgSmem {
-    h8 ta[2][4][64];
-    h8 tb[3][2][4][64];
+    static constexpr int WAVES = CH == 3 ? 12 : 8;       // POIs in flight, one per wavefront
+    static constexpr int ROWS = 16 * CH, RP = CH == 3 ? 56 : 72, TP = CH == 3 ? 104 : 136;
+    h8 ta[2][CH][64];
+    h8 tb[3][2][CH][64];
     h8 tn[2][64];
-    uint8_t ex[kDftWaves][64 * kExR + 64 * kExT];
-    float col0[kDftWaves][4][64];               // Re R^, Im R^, Re T^, Im T^ of column 0, by row j
-    uint32_t xcol[kDftWaves][64];
+    uint8_t ex[WAVES][ROWS * (RP + TP)];
+    float col0[FULL ? WAVES : 1][4][64];                // Re R^, Im R^, Re T^, Im T^ of column 0, by row j
+    uint32_t xcol[FULL ? WAVES : 1][64];
 };
 
 __device__ __forceinline__ f16x mfma16(h8 a, h8 b, f16x c)
@@ -1290,9 +1325,13 @@ __device__ __forceinline__ h8 centred_h8(uint2 w, h2v off)
     return r;
 }
 
-__device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const FftccParams& p, int poi)
+template <int CH, bool FULL>
+__device__ __forceinline__ void fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int wave, int lane, const FftccParams& p,
+                                                   int poi)
 {
-    constexpr int N = 64, NN = 4096;
+    using Sm = DftWgSmem<CH, FULL>;
+    constexpr int WORDS = 4 * CH;
+    const int N = FULL ? 64 : p.N, NN = N * N;
     const int m = lane & 31, h = lane >> 5;
     const int py = p.poi[2 * poi], px = p.poi[2 * poi + 1];
     if (py - N / 2 < 0 || px - N / 2 < 0 || py + N / 2 > p.img_h || px + N / 2 > p.img_w) {
@@ -1300,13 +1339,11 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
         return;
     }
     uint8_t* ex = sm.ex[wave];
-    const uint8_t* erows = ex;                 // R row y at y kExR
-    const uint8_t* etrows = ex + 64 * kExR;    // T row y at y kExT, twice
-    float (*col0)[64] = sm.col0[wave];
-    uint32_t* xcol = sm.xcol[wave];
+    const uint8_t* erows = ex;                     // R row y at y RP, zero beyond N
+    const uint8_t* etrows = ex + Sm::ROWS * Sm::RP;    // T row y at y TP, and again N bytes on
     // -- window rows (lane = row) to LDS, exact integer sums -------------------
     int sr = 0, st = 0, srr = 0, stt = 0;
-    {
+    if constexpr (FULL) {
         const size_t o = (size_t)(py - N / 2 + lane) * p.stride + (px - N / 2);
         uint32_t rw[16], tw[16];
         __builtin_memcpy(rw, p.ref + o, 64);
@@ -1319,8 +1356,8 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
             stt = (int)__builtin_amdgcn_udot4(tw[k], tw[k], (uint32_t)stt, false);
         }
         wave_lds_sync();                       // the previous POI's reads of this region are done
-        uint2* er = reinterpret_cast<uint2*>(ex + lane * kExR);
-        uint2* et = reinterpret_cast<uint2*>(ex + 64 * kExR + lane * kExT);
+        uint2* er = reinterpret_cast<uint2*>(ex + lane * Sm::RP);
+        uint2* et = reinterpret_cast<uint2*>(ex + Sm::ROWS * Sm::RP + lane * Sm::TP);
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const uint2 a = make_uint2(rw[2 * k], rw[2 * k + 1]);
@@ -1329,6 +1366,45 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
             et[k] = b;
             et[8 + k] = b;
         }
+    } else {
+        uint32_t rw[WORDS] = {}, tw[WORDS] = {};
+        if (lane < N) {
+            const size_t o = (size_t)(py - N / 2 + lane) * p.stride + (px - N / 2);
+            load_row<WORDS>(p.ref + o, N, rw);
+            load_row<WORDS>(p.tar + o, N, tw);
+        }
+#pragma unroll
+        for (int k = 0; k < WORDS; ++k) {
+            const int x = 4 * k;
+            const uint32_t keep = x + 4 <= N ? ~0u : x >= N ? 0u : 0xffffu;   // N is even
+            rw[k] &= keep;
+            tw[k] &= keep;
+            sr = (int)__builtin_amdgcn_udot4(rw[k], 0x01010101u, (uint32_t)sr, false);
+            st = (int)__builtin_amdgcn_udot4(tw[k], 0x01010101u, (uint32_t)st, false);
+            srr = (int)__builtin_amdgcn_udot4(rw[k], rw[k], (uint32_t)srr, false);
+            stt = (int)__builtin_amdgcn_udot4(tw[k], tw[k], (uint32_t)stt, false);
+        }
+        wave_lds_sync();                       // the previous POI's reads of this region are done
+        if (lane < N) {
+            uint2* er = reinterpret_cast<uint2*>(ex + lane * Sm::RP);
+            uint8_t* trow = ex + Sm::ROWS * Sm::RP + lane * Sm::TP;
+            uint2* et = reinterpret_cast<uint2*>(trow);
+#pragma unroll
+            for (int k = 0; k < WORDS / 2; ++k) {
+                er[k] = make_uint2(rw[2 * k], rw[2 * k + 1]);
+                et[k] = make_uint2(tw[2 * k], tw[2 * k + 1]);
+            }
+            // the T row again from byte N on (up to byte 2 N - 1 it is read)
+            uint32_t* t32 = reinterpret_cast<uint32_t*>(trow) + (N >> 2);
+            if ((N & 2) == 0) {
+#pragma unroll
+                for (int e = 0; e < WORDS; ++e) t32[e] = tw[e];
+            } else {                                       // N = 4 n + 2: bytes 0, 1 at N, then shifted words
+                *reinterpret_cast<uint16_t*>(trow + N) = (uint16_t)tw[0];
+#pragma unroll
+                for (int e = 0; e + 1 < WORDS; ++e) t32[1 + e] = __builtin_amdgcn_alignbyte(tw[e + 1], tw[e], 2);
+            }
+        }
     }
     sr = dpp_sum(sr); st = dpp_sum(st); srr = dpp_sum(srr); stt = dpp_sum(stt);
     const long long Sr = sr, St = st, Srr = srr, Stt = stt;
@@ -1336,36 +1412,38 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
         if (lane == 0 && p.status) p.status[poi] = TWDIC_FFTCC_FLAT;
         return;
     }
-    const int a = (sr + NN / 2) >> 12, b = (st + NN / 2) >> 12;    // rounded means
+    const int a = (int)((uint32_t)(sr + NN / 2) / (uint32_t)NN), b = (int)((uint32_t)(st + NN / 2) / (uint32_t)NN);   // rounded means
     const h2v oa = {(_Float16)(1024 + a), (_Float16)(1024 + a)};
     const h2v ob = {(_Float16)(1024 + b), (_Float16)(1024 + b)};
     const double nr2 = (double)(Srr - 2LL * a * Sr + (long long)a * a * NN);     // ||r||^2, exact
     const double nt2 = (double)(Stt - 2LL * b * St + (long long)b * b * NN);
     const double rho = sqrt(nr2 * nt2);
     int ex2;
-    (void)frexp(4096.0 * rho, &ex2);
-    const float s = ldexpf(1.0f, 14 - ex2);                                      // s 4096 rho in [2^13, 2^14)
-    const float tol = (float)(2.0 * 1.25 * kDftBound * rho * (double)s / 65536.0); // in C^ units (s 2^-16 N^2 C)
+    (void)frexp((double)NN * rho, &ex2);
+    const float s = ldexpf(1.0f, 14 - ex2);                                      // s N^2 rho in [2^13, 2^14)
+    const double bound = FULL ? kDftBound : kDftBoundN * (double)NN / 4096.0;
+    const float tol = (float)(2.0 * 1.25 * bound * rho * (double)s / 65536.0);     // in C^ units (s 2^-16 N^2 C)
     wave_lds_sync();
 
+    const int wave_f = FULL ? wave : 0;
     // -- first pass, columns k = 0 .. 31 (column 0 = Y[.][0] + i Y[.][32]) -------
-    h8 Yrr[4], Yri[4], Ytr[4], Yti[4];         // B operands, K chunk c = rows 16 c .. 16 c + 15 (accumulator order)
+    h8 Yrr[CH], Yri[CH], Ytr[CH], Yti[CH];     // B operands, K chunk c = rows 16 c .. 16 c + 15 (accumulator order)
 #pragma unroll
     for (int Mt = 0; Mt < 2; ++Mt) {
         f16x yrr = {}, yri = {}, ytr = {}, yti = {};
-        const int y = 32 * Mt + m;
+        const int y = FULL ? 32 * Mt + m : min(32 * Mt + m, N - 1);    // rows from N on meet zeros of the table
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < CH; ++c) {
             const h8 Fr = sm.ta[0][c][lane], Fi = sm.ta[1][c][lane];
-            const h8 Ar = centred_h8(*reinterpret_cast<const uint2*>(erows + y * kExR + 16 * c + 8 * h), oa);
-            const h8 At = centred_h8(*reinterpret_cast<const uint2*>(etrows + y * kExT + 16 * c + 8 * h), ob);
+            const h8 Ar = centred_h8(*reinterpret_cast<const uint2*>(erows + y * Sm::RP + 16 * c + 8 * h), oa);
+            const h8 At = centred_h8(*reinterpret_cast<const uint2*>(etrows + y * Sm::TP + 16 * c + 8 * h), ob);
             yrr = mfma16(Ar, Fr, yrr);
             yri = mfma16(Ar, Fi, yri);
             ytr = mfma16(At, Fr, ytr);
             yti = mfma16(At, Fi, yti);
         }
 #pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
+        for (int hf = 0; hf < 2 && 2 * Mt + hf < CH; ++hf) {
             Yrr[2 * Mt + hf] = to_h8(yrr, hf, 1.f);
             Yri[2 * Mt + hf] = to_h8(yri, hf, 1.f);
             Ytr[2 * Mt + hf] = to_h8(ytr, hf, 1.f);
@@ -1374,12 +1452,12 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
         __builtin_amdgcn_sched_barrier(0);
     }
     // -- second pass: R^, T^ for k = 0 .. 31 and P = conj(R^) T^ s ----------------
-    h8 Pre[4], Pim[4];                         // A operands of the first inverse pass [j chunk]
+    h8 Pre[CH], Pim[CH];                       // A operands of the first inverse pass [j chunk]
 #pragma unroll
     for (int Mj = 0; Mj < 2; ++Mj) {
         f16x Rr = {}, Ri = {}, Tr = {}, Ti = {};
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < CH; ++c) {
             const h8 Fr = sm.tb[0][Mj][c][lane], Fi = sm.tb[1][Mj][c][lane], nFi = sm.tb[2][Mj][c][lane];
             Rr = mfma16(Fr, Yrr[c], Rr);
             Ri = mfma16(Fr, Yri[c], Ri);
@@ -1390,14 +1468,14 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
             Tr = mfma16(nFi, Yti[c], Tr);
             Ti = mfma16(Fi, Ytr[c], Ti);
         }
-        if (m == 0) {                          // column 0: W_R = R^[j][0] + i R^[j][32], W_T likewise
+        if (FULL && m == 0) {                  // column 0: W_R = R^[j][0] + i R^[j][32], W_T likewise
 #pragma unroll
             for (int g = 0; g < 4; ++g) {      // registers 4 g .. 4 g + 3 hold rows j0 .. j0 + 3
                 const int j0 = 32 * Mj + 8 * g + 4 * h;
-                *reinterpret_cast<float4*>(&col0[0][j0]) = make_float4(Rr[4 * g], Rr[4 * g + 1], Rr[4 * g + 2], Rr[4 * g + 3]);
-                *reinterpret_cast<float4*>(&col0[1][j0]) = make_float4(Ri[4 * g], Ri[4 * g + 1], Ri[4 * g + 2], Ri[4 * g + 3]);
-                *reinterpret_cast<float4*>(&col0[2][j0]) = make_float4(Tr[4 * g], Tr[4 * g + 1], Tr[4 * g + 2], Tr[4 * g + 3]);
-                *reinterpret_cast<float4*>(&col0[3][j0]) = make_float4(Ti[4 * g], Ti[4 * g + 1], Ti[4 * g + 2], Ti[4 * g + 3]);
+                *reinterpret_cast<float4*>(&sm.col0[wave_f][0][j0]) = make_float4(Rr[4 * g], Rr[4 * g + 1], Rr[4 * g + 2], Rr[4 * g + 3]);
+                *reinterpret_cast<float4*>(&sm.col0[wave_f][1][j0]) = make_float4(Ri[4 * g], Ri[4 * g + 1], Ri[4 * g + 2], Ri[4 * g + 3]);
+                *reinterpret_cast<float4*>(&sm.col0[wave_f][2][j0]) = make_float4(Tr[4 * g], Tr[4 * g + 1], Tr[4 * g + 2], Tr[4 * g + 3]);
+                *reinterpret_cast<float4*>(&sm.col0[wave_f][3][j0]) = make_float4(Ti[4 * g], Ti[4 * g + 1], Ti[4 * g + 2], Ti[4 * g + 3]);
             }
         }
         f16x pr, pi;
@@ -1406,43 +1484,49 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
             pr[i] = fmaf(Rr[i], Tr[i], Ri[i] * Ti[i]);
             pi[i] = fmaf(Rr[i], Ti[i], -(Ri[i] * Tr[i]));
         }
-        // columns k >= 1 doubled for their conjugates 64 - k (column 0 is
-        // rewritten below); 2^16 undoes the two 2^-8 of the table
+        // columns k >= 1 doubled for their conjugates N - k (at N = 64 column 0 is
+        // rewritten below; otherwise 0 and N / 2, their own conjugates, count
+        // once); 2^16 undoes the two 2^-8 of the table
+        const float weight = !FULL && (m == 0 || 2 * m == N) ? 65536.f * s : 131072.f * s;
 #pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-            Pre[2 * Mj + hf] = to_h8(pr, hf, 131072.f * s);
-            Pim[2 * Mj + hf] = to_h8(pi, hf, 131072.f * s);
+        for (int hf = 0; hf < 2 && 2 * Mj + hf < CH; ++hf) {
+            Pre[2 * Mj + hf] = to_h8(pr, hf, weight);
+            Pim[2 * Mj + hf] = to_h8(pi, hf, weight);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    // column 0 of P becomes P[j][0] + i P[j][32]: unpack R^[j][0] = (W[j] +
-    // conj W[-j]) / 2, R^[j][32] = (W[j] - conj W[-j]) / 2i, likewise T^; lane
-    // j does row j (the results for j and -j are exact conjugates), lanes m = 0
-    // collect theirs
-    wave_lds_sync();
-    {
-        const int jm = (64 - lane) & 63;
-        const float4 w = make_float4(col0[0][lane], col0[1][lane], col0[2][lane], col0[3][lane]);
-        const float4 wm = make_float4(col0[0][jm], col0[1][jm], col0[2][jm], col0[3][jm]);
-        const float ar = 0.5f * (w.x + wm.x), ai = 0.5f * (w.y - wm.y);    // R^[j][0]
-        const float br = 0.5f * (w.y + wm.y), bi = 0.5f * (wm.x - w.x);    // R^[j][32]
-        const float cr = 0.5f * (w.z + wm.z), ci = 0.5f * (w.w - wm.w);    // T^[j][0]
-        const float dr = 0.5f * (w.w + wm.w), di = 0.5f * (wm.z - w.z);    // T^[j][32]
-        const float p0r = fmaf(ar, cr, ai * ci), p0i = fmaf(ar, ci, -(ai * cr));   // conj(R^0) T^0
-        const float p1r = fmaf(br, dr, bi * di), p1i = fmaf(br, di, -(bi * dr));   // conj(R^32) T^32
-        const h2v x = {(_Float16)((p0r - p1i) * (65536.f * s)), (_Float16)((p0i + p1r) * (65536.f * s))};
-        xcol[lane] = __builtin_bit_cast(uint32_t, x);
-    }
-    wave_lds_sync();
-    if (m == 0) {
+    if constexpr (FULL) {
+        float (*col0)[64] = sm.col0[wave_f];
+        uint32_t* xcol = sm.xcol[wave_f];
+        // column 0 of P becomes P[j][0] + i P[j][32]: unpack R^[j][0] = (W[j] +
+        // conj W[-j]) / 2, R^[j][32] = (W[j] - conj W[-j]) / 2i, likewise T^; lane
+        // j does row j (the results for j and -j are exact conjugates), lanes m = 0
+        // collect theirs
+        wave_lds_sync();
+        {
+            const int jm = (64 - lane) & 63;
+            const float4 w = make_float4(col0[0][lane], col0[1][lane], col0[2][lane], col0[3][lane]);
+            const float4 wm = make_float4(col0[0][jm], col0[1][jm], col0[2][jm], col0[3][jm]);
+            const float ar = 0.5f * (w.x + wm.x), ai = 0.5f * (w.y - wm.y);    // R^[j][0]
+            const float br = 0.5f * (w.y + wm.y), bi = 0.5f * (wm.x - w.x);    // R^[j][32]
+            const float cr = 0.5f * (w.z + wm.z), ci = 0.5f * (w.w - wm.w);    // T^[j][0]
+            const float dr = 0.5f * (w.w + wm.w), di = 0.5f * (wm.z - w.z);    // T^[j][32]
+            const float p0r = fmaf(ar, cr, ai * ci), p0i = fmaf(ar, ci, -(ai * cr));   // conj(R^0) T^0
+            const float p1r = fmaf(br, dr, bi * di), p1i = fmaf(br, di, -(bi * dr));   // conj(R^32) T^32
+            const h2v x = {(_Float16)((p0r - p1i) * (65536.f * s)), (_Float16)((p0i + p1r) * (65536.f * s))};
+            xcol[lane] = __builtin_bit_cast(uint32_t, x);
+        }
+        wave_lds_sync();
+        if (m == 0) {
 #pragma unroll
-        for (int Mj = 0; Mj < 2; ++Mj)
+            for (int Mj = 0; Mj < 2; ++Mj)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const h2v x = __builtin_bit_cast(h2v, xcol[32 * Mj + 8 * (r >> 2) + 4 * h + (r & 3)]);
-                Pre[2 * Mj + (r >> 3)][r & 7] = x[0];
-                Pim[2 * Mj + (r >> 3)][r & 7] = x[1];
-            }
+                for (int r = 0; r < 16; ++r) {
+                    const h2v x = __builtin_bit_cast(h2v, xcol[32 * Mj + 8 * (r >> 2) + 4 * h + (r & 3)]);
+                    Pre[2 * Mj + (r >> 3)][r & 7] = x[0];
+                    Pim[2 * Mj + (r >> 3)][r & 7] = x[1];
+                }
+        }
     }
     // -- first inverse pass, rows k = 0 .. 31: Q[k][a] = sum_j P[j][k] conj(F[j][a])
     //    (row 0 comes out as Q[0][a] + i Q[32][a], both real) -----------------------
@@ -1450,7 +1534,7 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
     {
         f16x qr[2] = {}, qi[2] = {};
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < CH; ++c) {
 #pragma unroll
             for (int Nc = 0; Nc < 2; ++Nc) {
                 const h8 Fr = sm.tb[0][Nc][c][lane], Fi = sm.tb[1][Nc][c][lane], nFi = sm.tb[2][Nc][c][lane];
@@ -1468,6 +1552,9 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
                 Qi[hf][Nc] = to_h8(qi[Nc], hf, 1.f);
             }
         }
+        // N <= 60: row k = 31 is empty; a one in it lets the last pass's table
+        // push the rows b >= N below every candidate
+        if (!FULL && h == 1) Qr[1][0][7] = Qr[1][1][7] = (_Float16)1.f;
         __builtin_amdgcn_sched_barrier(0);
     }
     // -- last pass: C^T = Re(F* Q) + (-1)^b Q[32][a], lane -> a, register -> b ------
@@ -1476,7 +1563,8 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
     for (int c = 0; c < 2; ++c) {
 #pragma unroll
         for (int Md = 0; Md < 2; ++Md) {
-            const h8 Fr = sm.tb[0][Md][c][lane], Fi = c == 0 ? sm.tn[Md][lane] : sm.tb[1][Md][c][lane];
+            const h8 Fr = !FULL && c == 1 ? sm.tn[Md][lane] : sm.tb[0][Md][c][lane];
+            const h8 Fi = FULL && c == 0 ? sm.tn[Md][lane] : sm.tb[1][Md][c][lane];
 #pragma unroll
             for (int Nd = 0; Nd < 2; ++Nd) {
                 Cd[Md][Nd] = mfma16(Fr, Qr[c][Nd], Cd[Md][Nd]);
@@ -1494,12 +1582,12 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
             float g = Cd[Md][Nd][0];
 #pragma unroll
             for (int r = 1; r < 16; ++r) g = fmaxf(g, Cd[Md][Nd][r]);
-            gmx[Nd][Md] = g;
+            gmx[Nd][Md] = !FULL && 32 * Nd + m >= N ? -FLT_MAX : g;    // columns a >= N are none
         }
     const float mx = dpp_max(fmaxf(fmaxf(gmx[0][0], gmx[0][1]), fmaxf(gmx[1][0], gmx[1][1])));
     const float thr = mx - tol;
-    // bit 16 (2 Nd + Md) + r: this lane's shifts in increasing row-major index a
-    // N + b (shifted in from the top bit down); a group no lane has a candidate
+    // bit 16 (2 Nd + Md) + r: this lane's shifts in increasing row-major index (a,
+    // then b, kept as 64 a + b) (shifted in from the top bit down); a group no lane has a candidate
     // in is skipped
     uint32_t mw[2] = {0u, 0u};
 #pragma unroll
@@ -1516,28 +1604,33 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
     uint64_t mask = ((uint64_t)mw[1] << 32) | mw[0];
 
     // -- exact integer correlation at the candidates, in increasing index order ---
-    const uint32_t* rrow = reinterpret_cast<const uint32_t*>(erows + lane * kExR);
+    const uint32_t* rrow = reinterpret_cast<const uint32_t*>(erows + (FULL || lane < N ? lane : 0) * Sm::RP);
     int bestI = -1, peak = -1;
     for (;;) {
         int mine = INT_MAX;
         if (mask) {
             const int bit = __builtin_ctzll(mask);
             const int Nd = bit >> 5, Md = (bit >> 4) & 1, r = bit & 15;
-            mine = (32 * Nd + m) * N + 32 * Md + 8 * (r >> 2) + 4 * h + (r & 3);
+            mine = (32 * Nd + m) * 64 + 32 * Md + 8 * (r >> 2) + 4 * h + (r & 3);
         }
         const int k = dpp_min(mine);
         if (k == INT_MAX) break;
         const int kv = k >> 6, ku = k & 63, d = ku >> 2, sh = ku & 3;
-        const uint32_t* trow = reinterpret_cast<const uint32_t*>(etrows + ((lane + kv) & 63) * kExT);
+        int ty = lane + kv;                    // row (lane + kv) mod N
+        if constexpr (FULL)
+            ty &= 63;
+        else
+            ty = lane >= N ? 0 : ty >= N ? ty - N : ty;
+        const uint32_t* trow = reinterpret_cast<const uint32_t*>(etrows + ty * Sm::TP);
         uint32_t acc = 0;
         uint32_t w0 = trow[d];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
+        for (int j = 0; j < WORDS; ++j) {
             const uint32_t w1 = trow[d + j + 1];
             acc = __builtin_amdgcn_udot4(rrow[j], __builtin_amdgcn_alignbyte(w1, w0, sh), acc, false);
             w0 = w1;
         }
-        const int I = dpp_sum((int)acc);
+        const int I = dpp_sum(FULL || lane < N ? (int)acc : 0);
         if (I > bestI) {
             bestI = I;
             peak = k;
@@ -1547,8 +1640,9 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
     if (lane == 0) {
         const double nr = (double)Srr - (double)Sr * (double)Sr / (double)NN;
         const double nt = (double)Stt - (double)St * (double)St / (double)NN;
-        int iu, iv;
-        wrap_peak(peak, N, iu, iv);
+        int iu = peak & 63, iv = peak >> 6;    // wrapped to the reference's (u, v) (:316-322)
+        if (iu > N / 2) iu -= N;
+        if (iv > N / 2) iv -= N;
         p.u[poi] = (float)iu;
         p.v[poi] = (float)iv;
         p.zncc[poi] = (float)(((double)bestI - (double)Sr * (double)St / (double)NN) / sqrt(nr * nt));
@@ -1556,12 +1650,12 @@ __device__ void fftcc_dft_mfma_poi(DftWgSmem& sm, int wave, int lane, const Fftc
     }
 }
 
-// Workgroups of kDftWaves wavefronts share the DFT tables in LDS; workgroup
-// b takes the contiguous POI range [g n / G, (g + 1) n / G) (G workgroups),
-// its wavefronts every kDftWaves-th POI of it.  Workgroups go to the 8 XCDs
+// A workgroup's wavefronts share the DFT tables in LDS; workgroup b takes the
+// contiguous POI range [g n / G, (g + 1) n / G) (G workgroups), its wavefronts
+// every WAVES-th POI of it.  Workgroups go to the 8 XCDs
 // round-robin, so g = (b mod 8) G / 8 + b / 8 when 8 divides G: each XCD
 // (and its L2) then covers one contiguous eighth of the POIs, a band of rows.
-__device__ __forceinline__ void dft_tables_to_lds(DftWgSmem& sm)
+__device__ __forceinline__ void dft_tables_to_lds(DftWgSmem<4, true>& sm, const float2*, int)
 {
     const h8* gb = &g_dft_tab[1][0][0][0][0];
     h8* la = &sm.ta[0][0][0];
@@ -1573,35 +1667,83 @@ __device__ __forceinline__ void dft_tables_to_lds(DftWgSmem& sm)
     __syncthreads();
 }
 
+// N < 64: from the N twiddles exp(-2 pi i e / N), each rounded to fp16, zero
+// where a row or column is beyond the window (or, in table 0, beyond the half
+// spectrum k <= N / 2).  The upper half of the circle mirrors the lower one,
+// so F[-j][y] = conj F[j][y] holds exactly, as the half spectrum needs.  tn:
+// the last pass's real part of K chunk 1 with -1 at k = 31 in the rows b >= N.
+template <int CH>
+__device__ __forceinline__ void dft_tables_to_lds(DftWgSmem<CH, false>& sm, const float2* __restrict__ tw, int N)
+{
+    const uint32_t inv = (1u << 18) / (uint32_t)N + 1u;       // x / N = (x inv) >> 18 for x < 4096, N <= 64
+    auto entry = [&](int row, int col, _Float16& re, _Float16& im) {
+        const uint32_t x = (uint32_t)(row * col);
+        const int e = (int)(x - ((x * inv) >> 18) * (uint32_t)N);
+        const bool up = 2 * e > N;
+        const float2 w = tw[up ? N - e : e];
+        re = (_Float16)w.x;
+        im = (_Float16)(up ? -w.y : w.y);
+    };
+    _Float16* la = reinterpret_cast<_Float16*>(&sm.ta[0][0][0]);
+    _Float16* lb = reinterpret_cast<_Float16*>(&sm.tb[0][0][0][0]);
+    _Float16* ln = reinterpret_cast<_Float16*>(&sm.tn[0][0]);
+    const _Float16 zero = (_Float16)0.f, down = (_Float16)0.00390625f;
+    constexpr int A = CH * 64 * 8, B = 2 * A;                  // entries of one part
+    for (int i = threadIdx.x; i < A; i += blockDim.x) {
+        const int q = i & 7, lane = (i >> 3) & 63, c = i >> 9;
+        const int x = 16 * c + 8 * (lane >> 5) + q, k = lane & 31;
+        _Float16 re = zero, im = zero;
+        if (x < N && 2 * k <= N) entry(x, k, re, im);
+        la[i] = re;
+        la[A + i] = im;
+    }
+    for (int i = threadIdx.x; i < B; i += blockDim.x) {
+        const int q = i & 7, lane = (i >> 3) & 63, c = (i >> 9) % CH, tile = (i >> 9) / CH;
+        const int row = 32 * tile + (lane & 31), col = 16 * c + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+        _Float16 re = zero, im = zero;
+        if (row < N && col < N) entry(row, col, re, im);
+        lb[i] = re * down;
+        lb[B + i] = im * down;
+        lb[2 * B + i] = -im * down;
+        if (c == 1) ln[((tile << 6) + lane) * 8 + q] = col == 31 ? (row < N ? zero : (_Float16)-1.f) : re * down;
+    }
+    __syncthreads();
+}
+
 __device__ __forceinline__ int dft_range_index()
 {
     const int G = gridDim.x, b = blockIdx.x;
     return (G & 7) == 0 ? (b & 7) * (G >> 3) + (b >> 3) : b;
 }
 
-__global__ __launch_bounds__(64 * kDftWaves, 1) void k_fftcc_dft_mfma(FftccParams p)
+template <int CH, bool FULL>
+__global__ __launch_bounds__((64 * DftWgSmem<CH, FULL>::WAVES), 1) void k_fftcc_dft_mfma(FftccParams p)
 {
-    __shared__ DftWgSmem sm;
-    dft_tables_to_lds(sm);
+    __shared__ DftWgSmem<CH, FULL> sm;
+    dft_tables_to_lds(sm, p.tw, p.N);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = dft_range_index();
     const int lo = (int)((long long)g * p.n / gridDim.x);
     const int hi = (int)((long long)(g + 1) * p.n / gridDim.x);
-    for (int poi = lo + wave; poi < hi; poi += kDftWaves) fftcc_dft_mfma_poi(sm, wave, lane, p, poi);
+    for (int poi = lo + wave; poi < hi; poi += DftWgSmem<CH, FULL>::WAVES) fftcc_dft_mfma_poi(sm, wave, lane, p, poi);
 }
 
-// Batched form over items (pair, POI) of pairs with N = 64: the same ranges
+// Batched form over items (pair, POI) of pairs that share N: the same ranges
 // per workgroup, each wavefront reading its item's pair descriptor.
-__global__ __launch_bounds__(64 * kDftWaves, 1) void k_batch_fftcc_dft_mfma(const PairDesc* __restrict__ pairs,
-                                                                         const int2* __restrict__ items, int count)
+template <int CH, bool FULL>
+__global__ __launch_bounds__((64 * DftWgSmem<CH, FULL>::WAVES), 1) void k_batch_fftcc_dft_mfma(
+    const PairDesc* __restrict__ pairs, const int2* __restrict__ items, int count)
 {
-    __shared__ DftWgSmem sm;
-    dft_tables_to_lds(sm);
+    __shared__ DftWgSmem<CH, FULL> sm;
+    {
+        const FftccParams p = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(items[0].x)].fftcc;
+        dft_tables_to_lds(sm, p.tw, p.N);
+    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = dft_range_index();
     const int lo = (int)((long long)g * count / gridDim.x);
     const int hi = (int)((long long)(g + 1) * count / gridDim.x);
-    for (int i = lo + wave; i < hi; i += kDftWaves) {
+    for (int i = lo + wave; i < hi; i += DftWgSmem<CH, FULL>::WAVES) {
         const int2 it = items[i];
         const FftccParams p = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(it.x)].fftcc;
         fftcc_dft_mfma_poi(sm, wave, lane, p, __builtin_amdgcn_readfirstlane(it.y));
@@ -1610,33 +1752,46 @@ __global__ __launch_bounds__(64 * kDftWaves, 1) void k_batch_fftcc_dft_mfma(cons
 
 // workgroups for n POIs: one per compute unit (each holds one), fewer for
 // small n
-int dft_blocks(int n)
+int dft_blocks(int n, int waves)
 {
     int dev = 0;
     (void)hipGetDevice(&dev);
     const int cus = dev >= 0 && dev < 64 && g_dft_cus[dev] > 0 ? g_dft_cus[dev] : 256;
-    return std::max(1, std::min(cus, (n + kDftWaves - 1) / kDftWaves));
+    return std::max(1, std::min(cus, (n + waves - 1) / waves));
+}
+
+template <int CH, bool FULL>
+void launch_dft(const FftccParams& p, hipStream_t st)
+{
+    constexpr int W = DftWgSmem<CH, FULL>::WAVES;
+    hipLaunchKernelGGL((k_fftcc_dft_mfma<CH, FULL>), dim3(dft_blocks(p.n, W)), dim3(64 * W), 0, st, p);
+}
+
+template <int CH, bool FULL>
+void launch_batch_dft(const PairDesc* pairs, const int2* items, int count, hipStream_t st)
+{
+    constexpr int W = DftWgSmem<CH, FULL>::WAVES;
+    hipLaunchKernelGGL((k_batch_fftcc_dft_mfma<CH, FULL>), dim3(dft_blocks(count, W)), dim3(64 * W), 0, st, pairs, items,
+                       count);
 }
 
 }  // namespace
 
-int mma_form(int N)
-{
-    return N == 64 ? 0 : N > 48 ? 1 : N > 32 ? 2 : 3;
-}
-
-hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int form, hipStream_t st)
+hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int N, hipStream_t st)
 {
     if (count <= 0) return hipSuccess;
-    switch (form) {
-    case 0:
-        hipLaunchKernelGGL(k_batch_fftcc_dft_mfma, dim3(dft_blocks(count)), dim3(64 * kDftWaves), 0, st, pairs, items,
-                           count);
-        break;
-    case 1: hipLaunchKernelGGL((k_batch_fftcc_mma<64, false, 32>), dim3(count), dim3(64), 0, st, pairs, items); break;
-    case 2: hipLaunchKernelGGL((k_batch_fftcc_mma<64, false, 16>), dim3(count), dim3(64), 0, st, pairs, items); break;
-    default: hipLaunchKernelGGL((k_batch_fftcc_mma<32, false, 32>), dim3(count), dim3(64), 0, st, pairs, items); break;
-    }
+    if (N == 64)
+        launch_batch_dft<4, true>(pairs, items, count, st);
+    else if (dft_takes(N, count) && N > 48)
+        launch_batch_dft<4, false>(pairs, items, count, st);
+    else if (dft_takes(N, count))
+        launch_batch_dft<3, false>(pairs, items, count, st);
+    else if (N > 48)
+        hipLaunchKernelGGL((k_batch_fftcc_mma<64, false, 32>), dim3(count), dim3(64), 0, st, pairs, items);
+    else if (N > 32)
+        hipLaunchKernelGGL((k_batch_fftcc_mma<64, false, 16>), dim3(count), dim3(64), 0, st, pairs, items);
+    else
+        hipLaunchKernelGGL((k_batch_fftcc_mma<32, false, 32>), dim3(count), dim3(64), 0, st, pairs, items);
     return hipGetLastError();
 }
 
@@ -1646,8 +1801,13 @@ hipError_t launch_fftcc(const FftccParams& p, int variant, hipStream_t st)
 {
     if (p.n <= 0) return hipSuccess;
     const int pairs = (p.n + 1) / 2;
-    if (variant == kFftccDftMfma && p.N == 64) {
-        hipLaunchKernelGGL(k_fftcc_dft_mfma, dim3(dft_blocks(p.n)), dim3(64 * kDftWaves), 0, st, p);
+    if (variant == kFftccDftMfma && dft_takes(p.N, p.n)) {
+        if (p.N == 64)
+            launch_dft<4, true>(p, st);
+        else if (p.N > 48)
+            launch_dft<4, false>(p, st);
+        else
+            launch_dft<3, false>(p, st);
     } else if (variant == kFftccMma || variant == kFftccDftMfma) {
         if (p.N == 64)
             hipLaunchKernelGGL((k_fftcc_mma<64, true, 32>), dim3(p.n), dim3(64), 0, st, p);

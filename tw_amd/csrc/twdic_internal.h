@@ -192,17 +192,15 @@ hipError_t launch_poi_grid(int32_t* poi, int start_x, int start_y, int nx, int n
 // N <= 64); 2, 3, 4: the FFT register engine's occupancy target (N = 32, 64,
 // else the direct-DFT engine)
 constexpr int kFftccMma = 8;
-// kFftccDftMfma: N = 64 on fp16 matrix-core DFTs with exact re-evaluation
-// of the near-maximal shifts (other N: the integer engine); needs
-// dft_tables_init on the device first
+// kFftccDftMfma: N = 64 and most sets with 32 < N <= 60 on fp16 matrix-core DFTs
+// with exact re-evaluation of the near-maximal shifts (the others: the integer
+// engine); needs dft_tables_init on the device first
 constexpr int kFftccDftMfma = 9;
 hipError_t dft_tables_init(int device);
 hipError_t launch_fftcc(const FftccParams& p, int variant, hipStream_t st);
-// batched form: the matrix-core kernel over items (pair, POI) of pairs that
-// share a kernel form (mma_form of their window edge N: 0 for N = 64,
-// 1 for 48 < N < 64, 2 for 32 < N <= 48, 3 for N <= 32)
-int mma_form(int N);
-hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int form, hipStream_t st);
+// batched form: the matrix-core kernels over items (pair, POI) of pairs that
+// share the window edge N
+hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int N, hipStream_t st);
 // batched form: IC-GN (fused interpolation) over workgroup items (pair, first
 // POI), 256 / lanes POIs of one pair per workgroup, every listed pair with
 // that many lanes per POI.
@@ -278,8 +276,8 @@ struct twdic_ctx {
     uint64_t refstate_version = ~0ull;
     const int32_t* refstate_poi = nullptr;
     int refstate_n = -1;
-    // FFT-CC engine (TWDIC_FFTCC_VARIANT): 9 fp16 matrix-core DFTs for N = 64 (else
-    // 8), 8 exact integer correlation on the matrix cores, 2-4 FFT registers
+    // FFT-CC engine (TWDIC_FFTCC_VARIANT): 9 fp16 matrix-core DFTs for N = 64 and
+    // most sets with 32 < N <= 60 (else 8), 8 exact integer correlation on the matrix cores, 2-4 FFT registers
     int fftcc_variant = twdic::kFftccDftMfma;
     int icgn_variant = 5;             // occupancy target of the IC-GN kernel (0: compiler's choice)
     uint8_t* h_stage = nullptr;       // pinned staging for host images
