@@ -232,7 +232,7 @@ twdic_status build_state_direct(twdic_batch* b)
         const IcgnParams& q = b->h_desc[i].icgn;
         TB_HIP(b, launch_gradients(q.ref, q.stride, q.sx0, q.sy0, q.rw, q.rh, nullptr, nullptr, nullptr,
                                    const_cast<uint32_t*>(q.g2), b->stream));
-        if (q.n > 0) TB_HIP(b, launch_ref_state(q, b->stream));
+        if (q.n > 0) TB_HIP(b, launch_ref_state(q, b->h_desc[i].ref, b->stream));
     }
     b->state_valid = true;
     return TWDIC_OK;
@@ -381,7 +381,9 @@ twdic_status set_pairs_impl(twdic_batch* b, const twdic_pair* pairs, int npairs)
         q.sx0 = p.roi_x; q.sy0 = p.roi_y; q.rw = p.roi_w; q.rh = p.roi_h;
         q.Sx = p.sx; q.Sy = p.sy; q.Wsub = 2 * p.sx + 1; q.Hsub = 2 * p.sy + 1; q.s = q.Wsub * q.Hsub;
         q.max_iter = p.max_iter; q.delta_p = p.delta_p;
-        set_icgn_layout(q, p.n);          // as a single context on this pair's POIs
+        const SubsetWalks walks = subset_walks(q.Wsub, q.Hsub);
+        set_icgn_layout(q, p.n, walks);   // as a single context on this pair's POIs
+        b->h_desc[i].ref = ref_plan(p.n, walks);
         q.g2 = b->d_g2 + g2_off; q.lut = nullptr;
         // the fused interpolation's row polynomials, as the single context
         // builds them (ROIs past 2^28 pixels read the image bytes there too)

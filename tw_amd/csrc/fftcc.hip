@@ -1254,16 +1254,6 @@ __device__ __forceinline__ h8 to_h8(const f16x& acc, int half, float scale)
     return r;
 }
 
-// LDS written by lanes of this wavefront and then read by other lanes of it:
-// its LDS accesses complete in issue order; keep the compiler from moving
-// them across this point.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Wave-uniform reductions for the DFT engine: butterflies inside each row of
 // 16 lanes by DPP (xor 1, xor 2, half-row mirror, row mirror), then the four
 // row results by readlane.  Every lane must be active.

@@ -368,41 +368,6 @@ __device__ __forceinline__ void kahan_pixel(float ks[8], float kc[8], float T, u
     }
 }
 
-// A lane's share of a strip (StripPlan): the exact float offsets of its first
-// pixel from the POI, that pixel's byte offset in the gradient plane from the
-// subset's corner, and, a byte each, its row count (0: the lane has no share),
-// the rows that every share of the strip has at least, and the strip's row
-// shares per column.  Every POI of a launch has the same subset and ROI width,
-// so one table in LDS serves a workgroup.
-//
-// The shares of a column are ranges of rows where the lane keeps a cell's rows
-// (row polynomials), which needs consecutive ones; otherwise the rows are dealt out in
-// turn, so that a wavefront reads neighbouring rows of the LUT or the image.
-struct StripLane {
-    float dx, dy;
-    uint32_t go;
-    uint32_t rows;
-};
-
-template <int L>
-__device__ __forceinline__ void fill_strips(StripLane* tab, const IcgnParams& P, bool ranges, int t0, int tstride)
-{
-    // constant strip indices: a run-time index would move the plan to scratch
-#pragma unroll
-    for (int k = 0; k < kMaxStrips; ++k) {
-        if (k >= P.strips.count) break;
-        const Strip s = P.strips.s[k];
-        const int base = P.Hsub / s.segs, rem = P.Hsub - base * s.segs;
-        for (int l = t0; l < L; l += tstride) {
-            const int seg = l / s.ncol, m = s.col + l - seg * s.ncol;
-            const int y = ranges ? seg * base + min(seg, rem) : seg;
-            const int rows = seg < s.segs ? base + (seg < rem ? 1 : 0) : 0;
-            tab[k * L + l] = {(float)(m - P.Sx), (float)(y - P.Sy), 4u * (uint32_t)(y * P.rw + m),
-                              (uint32_t)(rows | (base << 8) | (s.segs << 16))};
-        }
-    }
-}
-
 // One pass over the subset at the current warp, by the L lanes of a POI's
 // group (hl = lane % L; px, py and the warp are the group's POI's).  INT:
 // first pass at integer target pixels (:610-637); otherwise bicubic
@@ -827,11 +792,11 @@ __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_icgn(IcgnParams P)
 {
     constexpr int G = 256 / L;                   // POIs per workgroup
     __shared__ double rs[G][kRefStateUsed];
-    __shared__ StripLane tab[kMaxStrips * L];
+    __shared__ StripLane tab[IcgnPlan::kMax * L];
     const int first = xcd_block(blockIdx.x, gridDim.x) * G;
     const int slot = threadIdx.x / L, poi = first + slot;
     copy_ref_state(rs, P.refstate, first, G, P.n, threadIdx.x, 256);
-    fill_strips<L>(tab, P, RP && INTERP != TWDIC_INTERP_BSPLINE, threadIdx.x, 256);
+    fill_strips<L>(tab, P.strips, P, RP && INTERP != TWDIC_INTERP_BSPLINE, threadIdx.x, 256);
     __syncthreads();
     if (poi >= P.n) return;
     icgn_poi_t<L, INTERP, RP, K32>(P, poi, threadIdx.x & 63, tab, rs[slot]);
@@ -854,11 +819,11 @@ __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_batch_icgn_wg(cons
     const int2 it = wg[XCD ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x];
     const IcgnParams P = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(it.x)].icgn;
     __shared__ double rs[G][kRefStateUsed];
-    __shared__ StripLane tab[kMaxStrips * L];
+    __shared__ StripLane tab[IcgnPlan::kMax * L];
     const int first = __builtin_amdgcn_readfirstlane(it.y);
     const int slot = threadIdx.x / L, poi = first + slot;
     copy_ref_state(rs, P.refstate, first, G, P.n, threadIdx.x, 256);
-    fill_strips<L>(tab, P, ALL_RP || P.rp != nullptr, threadIdx.x, 256);
+    fill_strips<L>(tab, P.strips, P, ALL_RP || P.rp != nullptr, threadIdx.x, 256);
     __syncthreads();
     if (poi >= P.n) return;
     if constexpr (ALL_RP)
@@ -913,7 +878,7 @@ __global__ __launch_bounds__(256) void k_batch_icgn(const PairDesc* __restrict__
                                                     int total, int* counter, int chunk)
 {
     __shared__ double rs[4][1][kRefStateUsed];
-    __shared__ StripLane tabs[4][kMaxStrips * 64];
+    __shared__ StripLane tabs[4][IcgnPlan::kMax * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     StripLane* tab = tabs[wave];
     for (;;) {
@@ -930,9 +895,9 @@ __global__ __launch_bounds__(256) void k_batch_icgn(const PairDesc* __restrict__
             __builtin_amdgcn_wave_barrier();
             copy_ref_state(rs[wave], P.refstate, poi, 1, P.n, lane, 64);
             if (P.lanes == 64)
-                fill_strips<64>(tab, P, P.rp != nullptr, lane, 64);
+                fill_strips<64>(tab, P.strips, P, P.rp != nullptr, lane, 64);
             else
-                fill_strips<32>(tab, P, P.rp != nullptr, lane, 64);
+                fill_strips<32>(tab, P.strips, P, P.rp != nullptr, lane, 64);
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
             if (P.lanes == 64)

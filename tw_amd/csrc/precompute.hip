@@ -308,160 +308,285 @@ hipError_t launch_batch_row_poly(const PairDesc* pairs, int npairs, int max_rh, 
 
 // ---------------------------------------------------------------------------
 // Per-reference state, one POI per group of L lanes (a wavefront, or a
-// half-wavefront for large POI sets, as the iterations; built once per
-// reference and POI set; the reference rebuilds it on m_isRefImgUpdated,
-// TW_paDIC_cuICGN2D.cu:883-903).  Sums follow ICGN2D_Compute's precompute
-// (TW_paDIC_ICGN2D_CPU.cpp:516-595): SD = [Rx, Rx dx, Rx dy, Ry, Ry dx, Ry dy],
-// H = sum SD^T SD.  Every SD is a half-integer multiple and every product is
-// a multiple of 1/4 below 2^24, so the FP64 sums here are exact and
-// independent of order: the group width does not change a bit of it.  The
-// Cholesky factorisation is FP64.
+// half-wavefront for large POI sets; built once per reference and POI set; the
+// reference rebuilds it on m_isRefImgUpdated, TW_paDIC_cuICGN2D.cu:883-903).
+// Sums follow ICGN2D_Compute's precompute (TW_paDIC_ICGN2D_CPU.cpp:516-595):
+// SD = [Rx, Rx dx, Rx dy, Ry, Ry dx, Ry dy], H = sum SD^T SD.  With g = 2R the
+// 35 sums are 32 moments of eight integers per pixel (gx^2, gx gy, gy^2 with
+// 1, dx, dy, dx^2, dx dy, dy^2; gx, gy, gx R, gy R with 1, dx, dy; R, R^2),
+// exact however they are added up.  The Cholesky factorisation is FP64.
+//
+// Each lane walks down columns (StripPlan), so dx is constant and the dy
+// moments come from running sums (summation by parts, twice for dy^2): 19
+// integer accumulators and 21 integer instructions per pixel, where the sums
+// in FP64 took 35 accumulators and about 50.  A row range of at most kRefRows
+// rows keeps the largest, sum sum sum gx^2, below 2^31; the ranges' moments
+// are added in FP64, integers below 2^53.  The lanes' moments are then added
+// through LDS, eight at a time, each lane taking one moment of eight lanes; and
+// a workgroup's factorisations run side by side, one per lane, instead of once
+// in every lane of a POI's group.  157,609 POIs of 41x41: 0.79 ms with FP64 sums
+// per pixel and butterflies, 0.26 ms so (47k POIs 0.24 and 0.09 ms); bound by VALU
+// issue.  Two rows per trip instead of four: 0.305 ms, eight 0.255 ms.
 // ---------------------------------------------------------------------------
-template <int O>
-__device__ __forceinline__ double add_lane_xor_d(double v)
+namespace {
+
+// the moments' places in a POI's slot: 0, 6, 12 the six of gx^2, gx gy, gy^2;
+// 18, 21, 24, 27 the three of gx, gy, gx R, gy R; 30, 31 R and R^2
+enum { M_XX = 0, M_XY = 6, M_YY = 12, M_X = 18, M_Y = 21, M_XR = 24, M_YR = 27, M_R = 30, M_RR = 31, kMoments = 32 };
+constexpr int kMomentSlot = kRefStateUsed + 1;      // odd: the factorising lanes' reads fall on distinct banks
+
+// true when the subset at (px, py) leaves the ROI
+__device__ __forceinline__ bool subset_outside(const IcgnParams& P, int px, int py)
 {
-    // lane ^ O within 32-lane groups: ds_swizzle bit mode (and-mask 0x1f, or-mask 0, xor-mask O)
-    constexpr int pattern = 0x1f | (O << 10);
-    const int lo = __builtin_amdgcn_ds_swizzle(__double2loint(v), pattern);
-    const int hi = __builtin_amdgcn_ds_swizzle(__double2hiint(v), pattern);
-    return v + __hiloint2double(hi, lo);
+    return px - P.Sx < P.sx0 || py - P.Sy < P.sy0 || px + P.Sx >= P.sx0 + P.rw || py + P.Sy >= P.sy0 + P.rh;
 }
 
+// The moments of the POI at (px, py), whose subset lies in the ROI, by the L
+// lanes of its group (hl = lane % L).  red: the group's own LDS.
 template <int L>
-__device__ __forceinline__ double group_sum_d(double v)
+__device__ __forceinline__ void ref_moments(const IcgnParams& P, int nstrips, int px, int py, int hl, const StripLane* tab,
+                                            double (*red)[L + 1], double* mom)
 {
-    static_assert(L == 64 || L == 32, "lane groups of 64 or 32");
-    if constexpr (L == 64) v += __shfl_xor(v, 32);
-    v = add_lane_xor_d<16>(v);
-    v = add_lane_xor_d<8>(v);
-    v = add_lane_xor_d<4>(v);
-    v = add_lane_xor_d<2>(v);
-    return add_lane_xor_d<1>(v);
+    const __amdgpu_buffer_rsrc_t imgr =
+        __builtin_amdgcn_make_buffer_rsrc((void*)P.ref, (short)0, P.stride * (P.sy0 + P.rh), 0x00020000);
+    const __amdgpu_buffer_rsrc_t g2r =
+        __builtin_amdgcn_make_buffer_rsrc((void*)P.g2, (short)0, 4 * P.rw * P.rh, 0x00020000);
+    const uint32_t gcorner = 4u * (uint32_t)((py - P.Sy - P.sy0) * P.rw + (px - P.Sx - P.sx0));
+    double m[kMoments];
+#pragma unroll
+    for (int i = 0; i < kMoments; ++i) m[i] = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < nstrips; ++k) {
+        const StripLane e = tab[k * L + hl];
+        const int full = __builtin_amdgcn_readfirstlane((int)((e.rows >> 8) & 0xffu)), rows = (int)(e.rows & 0xffu);
+        if (rows == 0) continue;
+        int xx[3] = {}, xy[3] = {}, yy[3] = {}, x[2] = {}, y[2] = {}, xr[2] = {}, yr[2] = {}, r1 = 0, r2 = 0;
+        const int go = (int)(gcorner + e.go), ro = (py + (int)e.dy) * P.stride + px + (int)e.dx;
+        int gso = 0, rso = 0;
+        auto pixel = [&]() {
+            const uint32_t g = __builtin_amdgcn_raw_buffer_load_b32(g2r, go, gso, 0);
+            const int R = __builtin_amdgcn_raw_buffer_load_b8(imgr, ro, rso, 0);
+            const int gx = (int16_t)(g & 0xffffu), gy = (int)g >> 16;
+            gso += 4 * P.rw;
+            rso += P.stride;
+            xx[0] += __mul24(gx, gx); xx[1] += xx[0]; xx[2] += xx[1];
+            xy[0] += __mul24(gx, gy); xy[1] += xy[0]; xy[2] += xy[1];
+            yy[0] += __mul24(gy, gy); yy[1] += yy[0]; yy[2] += yy[1];
+            x[0] += gx; x[1] += x[0];
+            y[0] += gy; y[1] += y[0];
+            xr[0] += __mul24(gx, R); xr[1] += xr[0];
+            yr[0] += __mul24(gy, R); yr[1] += yr[0];
+            r1 += R;
+            r2 += __mul24(R, R);
+        };
+#pragma unroll 4
+        for (int r = 0; r < full; ++r) pixel();
+        if (rows > full) pixel();
+        // with j = rows - i for row i: sum j q and sum j (j + 1) / 2 q are the
+        // running sums' sums, and dy = end - j
+        const double dx = (double)e.dx, end = (double)e.dy + (double)rows;
+        auto fold3 = [&](const int (&q)[3], double* o) {
+            const double s0 = (double)q[0], s1 = (double)q[1], s2 = (double)q[2];
+            const double sy = end * s0 - s1;
+            o[0] += s0;
+            o[1] += dx * s0;
+            o[2] += sy;
+            o[3] += dx * dx * s0;
+            o[4] += dx * sy;
+            o[5] += end * (end * s0 - 2.0 * s1) + (2.0 * s2 - s1);
+        };
+        auto fold2 = [&](const int (&q)[2], double* o) {
+            const double s0 = (double)q[0];
+            o[0] += s0;
+            o[1] += dx * s0;
+            o[2] += end * s0 - (double)q[1];
+        };
+        fold3(xx, m + M_XX);
+        fold3(xy, m + M_XY);
+        fold3(yy, m + M_YY);
+        fold2(x, m + M_X);
+        fold2(y, m + M_Y);
+        fold2(xr, m + M_XR);
+        fold2(yr, m + M_YR);
+        m[M_R] += (double)r1;
+        m[M_RR] += (double)r2;
+    }
+    // the lanes' sum: eight moments at a time, lane hl takes moment hl % 8 of
+    // the lanes 8 (hl / 8) .. + 7
+#pragma unroll
+    for (int c = 0; c < kMoments / 8; ++c) {
+        wave_lds_sync();
+#pragma unroll
+        for (int v = 0; v < 8; ++v) red[v][hl] = m[8 * c + v];
+        wave_lds_sync();
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s += red[hl & 7][(hl & ~7) + i];
+        s += __shfl_xor(s, 8);
+        s += __shfl_xor(s, 16);
+        if constexpr (L == 64) s += __shfl_xor(s, 32);
+        if (hl < 8) mom[8 * c + hl] = s;
+    }
 }
 
-template <int L>
-__device__ __forceinline__ void ref_state_poi(const IcgnParams& P, int poi, int lane)
+// One POI's state (kRefStateUsed doubles) from its moments, in place.
+__device__ __forceinline__ void ref_finish(const IcgnParams& P, double* slot)
 {
-    const int hl = lane & (L - 1);
-    const int py = P.poi[2 * poi], px = P.poi[2 * poi + 1];
-    double* rs = P.refstate + (size_t)poi * kRefStateStride;
-    // subsets that leave the ROI are flagged by the iteration kernel; keep the
-    // state well defined and touch no memory outside the ROI
-    if (px - P.Sx < P.sx0 || py - P.Sy < P.sy0 || px + P.Sx >= P.sx0 + P.rw ||
-        py + P.Sy >= P.sy0 + P.rh) {
-        for (int i = hl; i < kRefStateStride; i += L) rs[i] = (i == RS_FLAG) ? (double)TWDIC_ICGN_OUT_OF_ROI : 0.0;
-        return;
+    constexpr int kPick[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};       // the moment of basis product (k, q)
+    double Lf[21], a[6], b[6];
+    int t = 0;
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+#pragma unroll
+        for (int q = 0; q <= k; ++q)
+            Lf[t++] = 0.25 * slot[(k < 3 ? M_XX : q < 3 ? M_XY : M_YY) + kPick[k % 3][q % 3]];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        a[k] = 0.5 * slot[(k < 3 ? M_X : M_Y) + k % 3];
+        b[k] = 0.5 * slot[(k < 3 ? M_XR : M_YR) + k % 3];
     }
-    double h[21], a[6], br[6];
-#pragma unroll
-    for (int i = 0; i < 21; ++i) h[i] = 0.0;
-#pragma unroll
-    for (int i = 0; i < 6; ++i) { a[i] = 0.0; br[i] = 0.0; }
-    long long sr = 0, srr = 0;
-    const int W = P.Wsub, s = P.s;
-    const int q64 = L / W, r64 = L - q64 * W;
-    int l = hl / W, m = hl - l * W;
-    for (int p = hl; p < s; p += L) {
-        int gy = py - P.Sy + l, gxp = px - P.Sx + m;
-        int R = P.ref[(size_t)gy * P.stride + gxp];
-        const uint32_t g = P.g2[(size_t)(gy - P.sy0) * P.rw + (gxp - P.sx0)];
-        double rx = 0.5 * (double)(int16_t)(g & 0xffffu), ry = 0.5 * (double)(int16_t)(g >> 16);
-        double dx = (double)(m - P.Sx), dy = (double)(l - P.Sy);
-        double sd[6] = {rx, rx * dx, rx * dy, ry, ry * dx, ry * dy};
-        int t = 0;
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-#pragma unroll
-            for (int q = 0; q <= k; ++q) h[t++] += sd[k] * sd[q];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) { a[k] += sd[k]; br[k] += sd[k] * (double)R; }
-        sr += R;
-        srr += (long long)R * R;
-        m += r64; l += q64;
-        if (m >= W) { m -= W; l += 1; }
-    }
-#pragma unroll
-    for (int i = 0; i < 21; ++i) h[i] = group_sum_d<L>(h[i]);
-#pragma unroll
-    for (int i = 0; i < 6; ++i) { a[i] = group_sum_d<L>(a[i]); br[i] = group_sum_d<L>(br[i]); }
-    double dsr = group_sum_d<L>((double)sr), dsrr = group_sum_d<L>((double)srr);  // exact (< 2^53)
-
+    const double sr = slot[M_R], srr = slot[M_RR];
     double mean, spread;
-    mean_spread(dsr, dsrr, (double)s, mean, spread);
+    mean_spread(sr, srr, (double)P.s, mean, spread);
     double flag = 0.0;
     // TW_paDIC_ICGN2D_CPU.cpp:580-595: zero mean or zero spread -> DarkSubset.
     // Both sums are exact integers, so the test is exact: all-zero or uniform.
-    if (dsr == 0.0 || dsrr * (double)s == dsr * dsr) flag = (double)TWDIC_ICGN_DARK_SUBSET;
-    double Lf[21];
-#pragma unroll
-    for (int i = 0; i < 21; ++i) Lf[i] = h[i];
+    if (sr == 0.0 || srr * (double)P.s == sr * sr) flag = (double)TWDIC_ICGN_DARK_SUBSET;
     if (flag == 0.0) {
         // Cholesky (spotrf 'L', TW_paDIC_ICGN2D_CPU.cpp:682,688-693) in FP64
+#pragma unroll
         for (int j = 0; j < 6; ++j) {
-            int jj = j * (j + 1) / 2;
+            const int jj = j * (j + 1) / 2;
             double d = Lf[jj + j];
+#pragma unroll
             for (int k = 0; k < j; ++k) d -= Lf[jj + k] * Lf[jj + k];
             if (!(d > 0.0)) { flag = (double)TWDIC_ICGN_SINGULAR_HESSIAN; break; }
             d = sqrt(d);
             Lf[jj + j] = d;
+#pragma unroll
             for (int i = j + 1; i < 6; ++i) {
-                int ii = i * (i + 1) / 2;
+                const int ii = i * (i + 1) / 2;
                 double v = Lf[ii + j];
+#pragma unroll
                 for (int k = 0; k < j; ++k) v -= Lf[ii + k] * Lf[jj + k];
                 Lf[ii + j] = v / d;
             }
         }
     }
-    if (hl == 0) {
 #pragma unroll
-        for (int i = 0; i < 21; ++i) rs[RS_L + i] = Lf[i];
+    for (int i = 0; i < 21; ++i) slot[RS_L + i] = Lf[i];
 #pragma unroll
-        for (int i = 0; i < 6; ++i) {
-            rs[RS_A + i] = a[i];
-            rs[RS_B + i] = centred(br[i], mean, a[i]);
-        }
-        rs[RS_NORM] = spread;
-        rs[RS_FLAG] = flag;
-        rs[RS_MEAN] = mean;
+    for (int i = 0; i < 6; ++i) {
+        slot[RS_A + i] = a[i];
+        slot[RS_B + i] = centred(b[i], mean, a[i]);
+    }
+    slot[RS_NORM] = spread;
+    slot[RS_FLAG] = flag;
+    slot[RS_MEAN] = mean;
 #pragma unroll
-        for (int i = 0; i < 6; ++i) rs[RS_RDIAG + i] = flag == 0.0 ? 1.0 / Lf[i * (i + 1) / 2 + i] : 0.0;
+    for (int i = 0; i < 6; ++i) slot[RS_RDIAG + i] = flag == 0.0 ? 1.0 / Lf[i * (i + 1) / 2 + i] : 0.0;
+}
+
+// The state of a subset that leaves the ROI, which the iteration kernel flags:
+// well defined, and no memory outside the ROI is read for it.
+__device__ __forceinline__ void ref_outside(double* slot)
+{
+    for (int i = 0; i < kRefStateUsed; ++i) slot[i] = i == RS_FLAG ? (double)TWDIC_ICGN_OUT_OF_ROI : 0.0;
+}
+
+}  // namespace
+
+// R rounds of 256 / L POIs per workgroup, then their factorisations together.
+template <int L, int R>
+__global__ __launch_bounds__(256) void k_ref_state(IcgnParams P, RefPlan plan)
+{
+    constexpr int G = 256 / L, Q = G * R;
+    __shared__ StripLane tab[RefPlan::kMax * L];
+    __shared__ double red[G][8][L + 1];
+    __shared__ double slots[Q][kMomentSlot];
+    const int t = threadIdx.x, first = blockIdx.x * Q;
+    fill_strips<L>(tab, plan, P, true, t, 256);
+    __syncthreads();
+#pragma unroll 1
+    for (int r = 0; r < R; ++r) {
+        const int slot = r * G + t / L, poi = first + slot;
+        if (poi >= P.n) break;
+        const int py = P.poi[2 * poi], px = P.poi[2 * poi + 1];
+        if (!subset_outside(P, px, py)) ref_moments<L>(P, plan.count, px, py, t & (L - 1), tab, red[t / L], slots[slot]);
+    }
+    __syncthreads();
+    if (t < Q && first + t < P.n) {
+        const int py = P.poi[2 * (first + t)], px = P.poi[2 * (first + t) + 1];
+        if (subset_outside(P, px, py))
+            ref_outside(slots[t]);
+        else
+            ref_finish(P, slots[t]);
+    }
+    __syncthreads();
+    for (int i = t; i < Q * kRefStateUsed; i += 256) {
+        const int slot = i / kRefStateUsed, j = i - slot * kRefStateUsed;
+        if (first + slot < P.n) P.refstate[(size_t)(first + slot) * kRefStateStride + j] = slots[slot][j];
     }
 }
 
-template <int L>
-__global__ __launch_bounds__(256) void k_ref_state(IcgnParams P)
+// Two rounds per workgroup (one factorisation pass for 16 POIs) where that
+// leaves the GPU full: 0.26 ms for 157,609 POIs, as with four; one round 0.30 ms,
+// eight 0.36 ms.  Smaller sets take one.
+hipError_t launch_ref_state(const IcgnParams& p, const RefPlan& plan, hipStream_t st)
 {
-    const int poi = blockIdx.x * (256 / L) + (int)(threadIdx.x / L);
-    if (poi >= P.n) return;
-    ref_state_poi<L>(P, poi, threadIdx.x & 63);
-}
-
-// Two POIs per wavefront from 4,096 POIs on, so the 35 group reductions are
-// issued once for both (their own crossover: the sums are exact, so the
-// width need not follow the iterations'); smaller sets one per wavefront,
-// half the pixel rounds for a GPU left partly idle.
-hipError_t launch_ref_state(const IcgnParams& p, hipStream_t st)
-{
-    if (p.n >= 4096)
-        hipLaunchKernelGGL(k_ref_state<32>, dim3((p.n + 7) / 8), dim3(256), 0, st, p);
+    if (p.n <= 0) return hipSuccess;
+    if (ref_lanes_for(p.n) == 64)
+        hipLaunchKernelGGL((k_ref_state<64, 1>), dim3((p.n + 3) / 4), dim3(256), 0, st, p, plan);
+    else if (p.n < 32768)
+        hipLaunchKernelGGL((k_ref_state<32, 1>), dim3((p.n + 7) / 8), dim3(256), 0, st, p, plan);
     else
-        hipLaunchKernelGGL(k_ref_state<64>, dim3((p.n + 3) / 4), dim3(256), 0, st, p);
+        hipLaunchKernelGGL((k_ref_state<32, 2>), dim3((p.n + 15) / 16), dim3(256), 0, st, p, plan);
     return hipGetLastError();
 }
 
-// Persistent form over (pair, POI) work items, one item per wavefront grab.
+// Persistent form over (pair, POI) work items, one item per wavefront grab, on
+// its pair's lanes (the whole wavefront, or its lower half).
 __global__ __launch_bounds__(256) void k_batch_ref_state(const PairDesc* __restrict__ pairs,
                                                          const int2* __restrict__ items, int total, int* counter)
 {
-    const int lane = threadIdx.x & 63;
+    __shared__ StripLane tabs[4][RefPlan::kMax * 64];
+    __shared__ double reds[4][8][64 + 1];
+    __shared__ double slots[4][kMomentSlot];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double* slot = slots[wave];
     for (;;) {
         int i = 0;
         if (lane == 0) i = atomicAdd(counter, 1);
         i = __builtin_amdgcn_readfirstlane(__shfl(i, 0));
         if (i >= total) break;
         const int2 it = items[i];
-        const IcgnParams P = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(it.x)].icgn;
-        ref_state_poi<64>(P, __builtin_amdgcn_readfirstlane(it.y), lane);
+        const int pair = __builtin_amdgcn_readfirstlane(it.x);
+        const IcgnParams P = const_pairs(pairs)[pair].icgn;
+        const RefPlan plan = const_pairs(pairs)[pair].ref;
+        const int poi = __builtin_amdgcn_readfirstlane(it.y), py = P.poi[2 * poi], px = P.poi[2 * poi + 1];
+        wave_lds_sync();
+        if (!subset_outside(P, px, py)) {
+            if (ref_lanes_for(P.n) == 64) {
+                fill_strips<64>(tabs[wave], plan, P, true, lane, 64);
+                wave_lds_sync();
+                ref_moments<64>(P, plan.count, px, py, lane, tabs[wave], reds[wave], slot);
+            } else {
+                fill_strips<32>(tabs[wave], plan, P, true, lane, 64);
+                wave_lds_sync();
+                if (lane < 32)
+                    ref_moments<32>(P, plan.count, px, py, lane, tabs[wave], reinterpret_cast<double (*)[33]>(reds[wave]),
+                                    slot);
+            }
+        }
+        wave_lds_sync();
+        if (lane == 0) {
+            if (subset_outside(P, px, py))
+                ref_outside(slot);
+            else
+                ref_finish(P, slot);
+        }
+        wave_lds_sync();
+        for (int j = lane; j < kRefStateUsed; j += 64) P.refstate[(size_t)poi * kRefStateStride + j] = slot[j];
     }
 }
 

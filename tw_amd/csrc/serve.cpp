@@ -143,6 +143,7 @@ struct twdic_server {
     std::map<std::tuple<uint64_t, int, int>, StateEntry*> states;
     uint64_t use_clock = 0;
     std::map<int, float2*> twiddles;               // per FFT window edge
+    std::map<int, SubsetWalks> walks;              // per subset half size
     std::deque<Job> queue;
     std::vector<Slot> slots;
     std::unordered_map<uint64_t, int> ticket_state;  // 0 pending, 1 done, -1 failed
@@ -362,10 +363,13 @@ bool admit(twdic_server* s, Slot& sl, Job& j)
     ip.Sx = ip.Sy = r.subset; ip.Wsub = ip.Hsub = 2 * r.subset + 1; ip.s = ip.Wsub * ip.Hsub;
     ip.max_iter = r.max_iter; ip.delta_p = r.delta_p;
     ip.g2 = d_g2; ip.lut = nullptr; ip.rp = d_rp; ip.refstate = d_state;
-    ip.poi = d_poi; ip.n = n; set_icgn_layout(ip, n);
+    ip.poi = d_poi; ip.n = n;
+    auto walks = s->walks.find(r.subset);
+    if (walks == s->walks.end()) walks = s->walks.emplace(r.subset, subset_walks(ip.Wsub, ip.Hsub)).first;
+    set_icgn_layout(ip, n, walks->second);
     ip.u = d_u; ip.v = d_v; ip.p6 = d_p6; ip.iters = d_it; ip.flags = d_fl; ip.dpnorm = nullptr;
     if (build) {
-        chk(launch_ref_state(ip, sl.st));
+        chk(launch_ref_state(ip, ref_plan(n, walks->second), sl.st));
         chk(hipEventRecord(e->ready, sl.st));
     } else {
         chk(hipStreamWaitEvent(sl.st, e->ready, 0));

@@ -202,7 +202,7 @@ IcgnParams icgn_params(twdic_ctx* c, const int32_t* poi, int n, float* u, float*
     p.rp = uses_plane(c) ? c->d_rp : nullptr;
     p.refstate = c->d_refstate;
     p.poi = poi; p.n = n;
-    set_icgn_layout(p, n);
+    set_icgn_layout(p, n, c->walks);
     p.u = u; p.v = v; p.p6 = p6; p.iters = iters; p.flags = flags; p.dpnorm = dpnorm;
     return p;
 }
@@ -263,7 +263,7 @@ twdic_status icgn_prepare(twdic_ctx* c, const int32_t* d_poi, int n, float* d_u,
     if (c->refstate_version != c->ref_version || c->refstate_poi != d_poi || c->refstate_n != n) {
         // per-reference state (RefAllSubetsNorm_Kernel + InverseHessian_Kernel,
         // TW_paDIC_cuICGN2D.cu:883-903), rebuilt when the reference or the POI set changed
-        TW_HIP(c, launch_ref_state(p, c->stream));
+        TW_HIP(c, launch_ref_state(p, ref_plan(p.n, c->walks), c->stream));
         c->refstate_version = c->ref_version;
         c->refstate_poi = d_poi;
         c->refstate_n = n;
@@ -345,6 +345,7 @@ twdic_status twdic_create(const twdic_config* cfg, int device, twdic_ctx** out)
     c->cfg = *cfg;
     c->device = device;
     num_poi(*cfg, &c->nx, &c->ny);
+    c->walks = subset_walks(2 * cfg->sx + 1, 2 * cfg->sy + 1);
     c->dstride = cfg->img_w;
     if (const char* v = std::getenv("TWDIC_FFTCC_VARIANT")) c->fftcc_variant = std::atoi(v);
     if (const char* v = std::getenv("TWDIC_ICGN_VARIANT")) c->icgn_variant = std::atoi(v);
@@ -585,7 +586,7 @@ twdic_status twdic_icgn_noalloc(twdic_ctx* c, const int32_t* d_poi, int n, float
     // field IC-GN reads), then the iterations read it, in stream order
     IcgnParams p = icgn_params(c, d_poi, n, d_u, d_v, d_p6, d_iters, d_flags, nullptr);
     p.refstate = state;
-    TW_HIP(c, launch_ref_state(p, c->stream));
+    TW_HIP(c, launch_ref_state(p, ref_plan(p.n, c->walks), c->stream));
     TW_HIP(c, launch_icgn(p, c->cfg.interp, c->icgn_variant, c->stream));
     return TWDIC_OK;
 }
@@ -680,7 +681,7 @@ twdic_status twdic_frame_replay(twdic_ctx* c)
     if (c->refstate_version != c->ref_version || c->refstate_poi != ip.poi || c->refstate_n != ip.n) {
         twdic_status st = ensure_ref_grads(c);
         if (st != TWDIC_OK) return st;
-        TW_HIP(c, launch_ref_state(ip, c->stream));
+        TW_HIP(c, launch_ref_state(ip, ref_plan(ip.n, c->walks), c->stream));
         c->refstate_version = c->ref_version;
         c->refstate_poi = ip.poi;
         c->refstate_n = ip.n;

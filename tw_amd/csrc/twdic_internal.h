@@ -38,51 +38,80 @@ constexpr int kRefStateUsed = 42;     // the doubles above that the iteration ke
 constexpr int kIcgnHalfWaveMin = 32768;
 inline int icgn_lanes_for(int n) { return n >= kIcgnHalfWaveMin ? 32 : 64; }
 
+// The reference state: two POIs per wavefront from 4,096 POIs on (its own
+// crossover: the sums are exact integers, so the width need not follow the
+// iterations'), smaller sets one per wavefront, half the rounds for a GPU left
+// partly idle.  A lane sums at most kRefRows rows at a time in 32 bits.
+__host__ __device__ inline int ref_lanes_for(int n) { return n >= 4096 ? 32 : 64; }
+constexpr int kRefRows = 56;
+
 // How the L lanes of a POI's group walk its subset: strips of `ncol` columns
 // from column `col`, each column cut into `segs` row ranges of equal length
 // (the first ones a row longer where they do not divide), one lane per column
 // and range, ncol segs <= L.
-constexpr int kMaxStrips = 6;
 struct Strip {
     int16_t col, ncol, segs;
 };
+template <int MAX>
 struct StripPlan {
+    static constexpr int kMax = MAX;
     int count;
-    Strip s[kMaxStrips];
+    Strip s[MAX];
 };
+typedef StripPlan<6> IcgnPlan;        // ranges of any length: at most ceil(121 / 32) strips are needed
+typedef StripPlan<13> RefPlan;        // ranges of at most kRefRows rows: ceil(121 / 10)
 
 // The strips of a W x H subset (1 <= W, H <= 121; L = 32 or 64) with the
-// fewest rounds, a strip costing one round besides its longest row range.
-inline StripPlan strip_plan(int W, int H, int L)
+// fewest rounds, a strip costing one round besides its longest row range, and
+// no row range longer than max_rows.
+template <class Plan>
+inline Plan strip_plan(int W, int H, int L, int max_rows)
 {
     constexpr int kMaxW = 128;
-    int cost[kMaxW], take[kMaxW];
-    cost[0] = 0;
+    int rounds[kMaxW], cost[kMaxW], take[kMaxW];
     auto segs = [&](int c) { return L / c < H ? L / c : H; };
+    int widest = 0;
+    for (int c = 1; c <= L && c <= W; ++c) {
+        rounds[c] = (H + segs(c) - 1) / segs(c);
+        if (rounds[c] <= max_rows) widest = c;
+    }
+    cost[0] = 0;
     for (int w = 1; w <= W; ++w) {
         cost[w] = 1 << 30;
-        for (int c = w < L ? w : L; c >= 1; --c) {
-            const int sg = segs(c), v = cost[w - c] + (H + sg - 1) / sg + 1;
+        for (int c = w < widest ? w : widest; c >= 1; --c) {
+            const int v = cost[w - c] + rounds[c] + 1;
             if (v < cost[w]) {
                 cost[w] = v;
                 take[w] = c;
             }
         }
     }
-    StripPlan p{};
+    Plan p{};
     int col = 0, w = W;
-    for (; w > 0 && p.count < kMaxStrips; w -= take[w]) {
+    for (; w > 0 && p.count < Plan::kMax; w -= take[w]) {
         p.s[p.count++] = {(int16_t)col, (int16_t)take[w], (int16_t)segs(take[w])};
         col += take[w];
     }
-    if (w > 0) {                       // more strips than the table holds: whole widths instead
+    if (w > 0) {                       // more strips than the table holds: the widest ones instead
         p.count = 0;
-        for (col = 0; col < W; col += L) {
-            const int c = W - col < L ? W - col : L;
+        for (col = 0; col < W; col += widest) {
+            const int c = W - col < widest ? W - col : widest;
             p.s[p.count++] = {(int16_t)col, (int16_t)c, (int16_t)segs(c)};
         }
     }
     return p;
+}
+
+// The walks of one subset size, by the lanes per POI (32, 64).
+struct SubsetWalks {
+    IcgnPlan icgn[2];
+    RefPlan ref[2];
+};
+
+inline SubsetWalks subset_walks(int W, int H)
+{
+    return {{strip_plan<IcgnPlan>(W, H, 32, H), strip_plan<IcgnPlan>(W, H, 64, H)},
+            {strip_plan<RefPlan>(W, H, 32, kRefRows), strip_plan<RefPlan>(W, H, 64, kRefRows)}};
 }
 
 // Mean and L2 spread of n samples from their exact-or-FP64 sums s1 = sum x,
@@ -99,6 +128,16 @@ __device__ __forceinline__ void mean_spread(double s1, double s2, double n, doub
 __device__ __forceinline__ double centred(double sdx, double mean, double a)
 {
     return __fma_rn(-mean, a, sdx);
+}
+
+// LDS written by lanes of a wavefront and then read by other lanes of it: its
+// LDS accesses complete in issue order; keep the compiler from moving them
+// across this point.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 struct FftccParams {
@@ -125,7 +164,7 @@ struct IcgnParams {
     int Sx, Sy, Wsub, Hsub, s;
     int max_iter;
     int lanes;                // lanes per POI: 32 or 64 (icgn_lanes_for of the set's POI count)
-    StripPlan strips;         // how those lanes walk the subset
+    IcgnPlan strips;          // how those lanes walk the subset
     double delta_p;           // the caller's float, widened: the loop test compares in FP64
     const uint32_t* g2;       // reference gradients (2Rx, 2Ry) as int16 pairs, ROI-relative
     const float* lut;         // target LUT [rh][rw][16]
@@ -147,13 +186,51 @@ struct IcgnParams {
 struct PairDesc {
     IcgnParams icgn;
     FftccParams fftcc;
+    RefPlan ref;              // how ref_lanes_for lanes walk the subset
 };
 
-// The lanes per POI and the walk of a set of n POIs, from its subset size.
-inline void set_icgn_layout(IcgnParams& p, int n)
+// The lanes per POI of a set of n POIs, and their walks of its subset.
+inline void set_icgn_layout(IcgnParams& p, int n, const SubsetWalks& w)
 {
     p.lanes = icgn_lanes_for(n);
-    p.strips = strip_plan(p.Wsub, p.Hsub, p.lanes);
+    p.strips = w.icgn[p.lanes == 64];
+}
+inline const RefPlan& ref_plan(int n, const SubsetWalks& w) { return w.ref[ref_lanes_for(n) == 64]; }
+
+// A lane's share of a strip (StripPlan): the exact float offsets of its first
+// pixel from the POI, that pixel's byte offset in the gradient plane from the
+// subset's corner, and, a byte each, its row count (0: the lane has no share),
+// the rows that every share of the strip has at least, and the strip's row
+// shares per column.  Every POI of a launch has the same subset and ROI width,
+// so one table in LDS serves a workgroup.
+//
+// The shares of a column are ranges of rows where the lane keeps a cell's rows
+// (row polynomials), which needs consecutive ones; otherwise the rows are dealt out in
+// turn, so that a wavefront reads neighbouring rows of the LUT or the image.
+struct StripLane {
+    float dx, dy;
+    uint32_t go;
+    uint32_t rows;
+};
+
+template <int L, class Plan>
+__device__ __forceinline__ void fill_strips(StripLane* tab, const Plan& plan, const IcgnParams& P, bool ranges,
+                                            int t0, int tstride)
+{
+    // constant strip indices: a run-time index would move the plan to scratch
+#pragma unroll
+    for (int k = 0; k < Plan::kMax; ++k) {
+        if (k >= plan.count) break;
+        const Strip s = plan.s[k];
+        const int base = P.Hsub / s.segs, rem = P.Hsub - base * s.segs;
+        for (int l = t0; l < L; l += tstride) {
+            const int seg = l / s.ncol, m = s.col + l - seg * s.ncol;
+            const int y = ranges ? seg * base + min(seg, rem) : seg;
+            const int rows = seg < s.segs ? base + (seg < rem ? 1 : 0) : 0;
+            tab[k * L + l] = {(float)(m - P.Sx), (float)(y - P.Sy), 4u * (uint32_t)(y * P.rw + m),
+                              (uint32_t)(rows | (base << 8) | (s.segs << 16))};
+        }
+    }
 }
 
 // Descriptors are never written while a batch kernel runs: reading them
@@ -219,7 +296,7 @@ inline size_t row_poly_bytes(int rw, int rh)
 // all_rp: every pair's descriptor has its row-polynomial plane
 hipError_t launch_batch_icgn_wg(const PairDesc* pairs, const int2* wg, int count, int lanes, int waves,
                                 bool xcd_ranges, bool all_rp, hipStream_t st);
-hipError_t launch_ref_state(const IcgnParams& p, hipStream_t st);
+hipError_t launch_ref_state(const IcgnParams& p, const RefPlan& plan, hipStream_t st);
 hipError_t launch_icgn(const IcgnParams& p, int interp, int variant, hipStream_t st);
 // persistent batch kernels: `blocks` workgroups drain a device work counter
 hipError_t launch_batch_icgn(const PairDesc* pairs, const int2* items, int total, int* counter, int chunk,
@@ -251,6 +328,7 @@ struct twdic_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     int nx = 0, ny = 0;
+    twdic::SubsetWalks walks{};       // of the configured subset
     int dstride = 0;                  // device image row stride (bytes)
     uint8_t* d_ref = nullptr;
     uint8_t* d_tar = nullptr;
