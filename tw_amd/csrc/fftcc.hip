@@ -1180,10 +1180,10 @@ __global__ __launch_bounds__(64) void k_batch_fftcc_mma(const PairDesc* __restri
 // N / 2 fits the 32 columns, so no column is packed; columns 0 and N / 2, their
 // own conjugates, count once.  Row k = 31 is empty: it carries the mask that
 // keeps rows b >= N from being candidates.  N <= 48 needs three K chunks instead
-// of four (112 MFMAs instead of 144) and 160 registers, so twelve wavefronts, three
-// per SIMD, hide each other's chains of dependent MFMAs and conversions, which
-// bound the engine: .53 ms for 155k POIs at N = 40, .75 ms at N = 56 (188
-// registers, two wavefronts per SIMD).
+// of four (112 MFMAs instead of 144) and fits 168 registers, so twelve wavefronts,
+// three per SIMD, hide each other's chains of dependent MFMAs and conversions,
+// which bound the engine: .48 ms for 155k POIs at N = 40, .71 ms at N = 56 and .73 ms
+// at N = 64 (two wavefronts per SIMD).
 // ===========================================================================
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
@@ -1203,7 +1203,7 @@ constexpr double kDftBoundN = 26.0;
 //   800     .016/.012  .016/.013  .016/.015  .016/.018  .016/.020  .016/.021
 //   1,200   .016/.014  .016/.016  .016/.019  .016/.024  .017/.026  .016/.027
 //   5,000   .025/.034  .023/.038  .025/.044  .03 /.065  .031/.072  .03 /.076
-//   155k    .53 /.69   .53 /.82   .56 /1.00  .73 /1.61  .75 /1.86  .77 /1.96
+//   155k    .47 /.69   .48 /.82   .51 /1.00  .69 /1.61  .71 /1.86  .72 /1.96
 inline bool dft_takes(int N, int n)
 {
     return N == 64 || (N > 48 && N <= 60) || (N > 32 && N <= 48 && n >= 1280);
@@ -1238,7 +1238,111 @@ struct DftWgSmem {
     uint8_t ex[WAVES][ROWS * (RP + TP)];
     float col0[FULL ? WAVES : 1][4][64];                // Re R^, Im R^, Re T^, Im T^ of column 0, by row j
     uint32_t xcol[FULL ? WAVES : 1][64];
+    static constexpr int KEPT = 32;                     // POIs whose outputs are formed together
+    int kept[WAVES][7][KEPT];                           // item, sums of R, T, R^2, T^2, sum R T at the peak, peak
 };
+
+// Where a window pair is (no padding bytes: those kept copies in memory).
+struct DftItem {
+    const uint8_t *ref, *tar;
+    int stride, py, px, inside;                         // inside: the windows lie in the image
+    __device__ __forceinline__ size_t row(int lane, int N) const
+    {
+        return (size_t)(py - N / 2 + lane) * stride + (px - N / 2);
+    }
+};
+
+__device__ __forceinline__ DftItem dft_item(const FftccParams& p, int poi)
+{
+    const int py = p.poi[2 * poi], px = p.poi[2 * poi + 1], h = p.N / 2;
+    return {p.ref, p.tar, p.stride, py, px, py >= h && px >= h && py + h <= p.img_h && px + h <= p.img_w};
+}
+
+// A window pair's rows in flight, CH lanes to a row, 16 bytes each, so that a
+// load instruction touches the lines of 64 / CH rows (with a lane per row the
+// lines of 64, four times over: the loads of eight wavefronts queued up in the
+// address unit, 0.81 ms per 157,609 POIs at N = 64 against 0.74 ms).  Lane l
+// holds piece l % CH of the rows k (64 / CH) + l / CH.  A row's last piece ends
+// with the row, so nothing outside it is read; words() moves it to its place.
+template <int CH, bool FULL>
+struct DftRows {
+    static constexpr int RL = 64 / CH, LOADS = (16 * CH + RL - 1) / RL;
+    uint32_t r[LOADS][4], t[LOADS][4];
+    __device__ __forceinline__ static int row(int k, int lane) { return RL * k + lane / CH; }
+    __device__ __forceinline__ static bool active(int k, int lane, int N)
+    {
+        return FULL || (row(k, lane) < N && lane < RL * CH);
+    }
+    // Any values, or zeros where load() may leave them: nothing has to be kept
+    // in these registers until then.
+    __device__ __forceinline__ void drop()
+    {
+#pragma unroll
+        for (int k = 0; k < LOADS; ++k)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                if constexpr (FULL) {
+                    asm("" : "=v"(r[k][w]));
+                    asm("" : "=v"(t[k][w]));
+                } else {
+                    r[k][w] = t[k][w] = 0u;
+                }
+            }
+    }
+    __device__ __forceinline__ void load(const DftItem& it, int N, int lane)
+    {
+        const int x = min(16 * (lane % CH), N - 16);
+#pragma unroll
+        for (int k = 0; k < LOADS; ++k)
+            if (active(k, lane, N)) {
+                const size_t o = it.row(row(k, lane), N) + x;
+                __builtin_memcpy(r[k], it.ref + o, 16);
+                __builtin_memcpy(t[k], it.tar + o, 16);
+            }
+    }
+    // The words of bytes 16 (lane % CH) .. + 15 of a row, zero beyond N: the last
+    // piece less the 16 CH - N bytes that belong to the one before.
+    __device__ __forceinline__ static void words(const uint32_t (&raw)[4], int N, int lane, uint32_t (&w)[4])
+    {
+        if constexpr (FULL) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = raw[i];
+        } else {
+            const int sh = lane % CH == CH - 1 ? 16 * CH - N : 0;
+            uint32_t m2 = (sh & 8) ? ~0u : 0u, m1 = (sh & 4) ? ~0u : 0u;
+            asm volatile("" : "+v"(m2), "+v"(m1));      // bitwise selects, as in load_row
+            uint32_t a[5], b[5];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = ((i < 2 ? raw[(i + 2) & 3] : 0u) & m2) | (raw[i] & ~m2);
+            a[4] = 0u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[i] = (a[i + 1] & m1) | (a[i] & ~m1);
+            b[4] = 0u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_alignbyte(b[i + 1], b[i], sh & 3);
+        }
+    }
+};
+
+// Sums over the wavefront of four values at once (as swap_add in icgn.hip:
+// pairs folded by permlane swaps, then row rotations), in scalars.
+__device__ __forceinline__ void dpp_sum4(int v[4])
+{
+    int w[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const auto s = __builtin_amdgcn_permlane32_swap((uint32_t)v[i], (uint32_t)v[i + 2], false, false);
+        w[i] = (int)(s[0] + s[1]);                      // lanes 0-31: v[i], 32-63: v[i + 2]
+    }
+    const auto s = __builtin_amdgcn_permlane16_swap((uint32_t)w[0], (uint32_t)w[1], false, false);
+    int x = (int)(s[0] + s[1]);                         // rows 0 .. 3: v[0], v[1], v[2], v[3]
+    x += __builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x124, 0xF, 0xF, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x122, 0xF, 0xF, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x121, 0xF, 0xF, true);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __builtin_amdgcn_readlane(x, 16 * i);
+}
 
 __device__ __forceinline__ f16x mfma16(h8 a, h8 b, f16x c)
 {
@@ -1315,104 +1419,85 @@ __device__ __forceinline__ h8 centred_h8(uint2 w, h2v off)
     return r;
 }
 
-template <int CH, bool FULL>
-__device__ __forceinline__ void fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int wave, int lane, const FftccParams& p,
-                                                   int poi)
+// The exact peak of one window pair whose rows are in `rows`; `next` is called
+// when they and most registers are free again, to load the following pair's.
+// Returns false for a flat window, else the four window sums, the exact sum of
+// R T at the peak and the peak's place 64 a + b.
+template <int CH, bool FULL, class Next>
+__device__ __forceinline__ bool fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int wave, int lane, int N, const DftItem& it,
+                                                   DftRows<CH, FULL>& rows, int (&sums)[4], int& bestI, int& peak,
+                                                   Next next)
 {
     using Sm = DftWgSmem<CH, FULL>;
     constexpr int WORDS = 4 * CH;
-    const int N = FULL ? 64 : p.N, NN = N * N;
-    const int m = lane & 31, h = lane >> 5;
-    const int py = p.poi[2 * poi], px = p.poi[2 * poi + 1];
-    if (py - N / 2 < 0 || px - N / 2 < 0 || py + N / 2 > p.img_h || px + N / 2 > p.img_w) {
-        if (lane == 0 && p.status) p.status[poi] = TWDIC_FFTCC_OUT;
-        return;
-    }
+    if constexpr (FULL) N = 64;
+    const int NN = N * N, m = lane & 31, h = lane >> 5;
     uint8_t* ex = sm.ex[wave];
     const uint8_t* erows = ex;                     // R row y at y RP, zero beyond N
     const uint8_t* etrows = ex + Sm::ROWS * Sm::RP;    // T row y at y TP, and again N bytes on
-    // -- window rows (lane = row) to LDS, exact integer sums -------------------
-    int sr = 0, st = 0, srr = 0, stt = 0;
-    if constexpr (FULL) {
-        const size_t o = (size_t)(py - N / 2 + lane) * p.stride + (px - N / 2);
-        uint32_t rw[16], tw[16];
-        __builtin_memcpy(rw, p.ref + o, 64);
-        __builtin_memcpy(tw, p.tar + o, 64);
+    // -- window rows to LDS, exact integer sums ---------------------------------
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            sr = (int)__builtin_amdgcn_udot4(rw[k], 0x01010101u, (uint32_t)sr, false);
-            st = (int)__builtin_amdgcn_udot4(tw[k], 0x01010101u, (uint32_t)st, false);
-            srr = (int)__builtin_amdgcn_udot4(rw[k], rw[k], (uint32_t)srr, false);
-            stt = (int)__builtin_amdgcn_udot4(tw[k], tw[k], (uint32_t)stt, false);
-        }
-        wave_lds_sync();                       // the previous POI's reads of this region are done
-        uint2* er = reinterpret_cast<uint2*>(ex + lane * Sm::RP);
-        uint2* et = reinterpret_cast<uint2*>(ex + Sm::ROWS * Sm::RP + lane * Sm::TP);
+    for (int i = 0; i < 4; ++i) sums[i] = 0;
+    {
+        using Rows = DftRows<CH, FULL>;
+        uint32_t rw[Rows::LOADS][4], tw[Rows::LOADS][4];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint2 a = make_uint2(rw[2 * k], rw[2 * k + 1]);
-            const uint2 b = make_uint2(tw[2 * k], tw[2 * k + 1]);
-            er[k] = a;
-            et[k] = b;
-            et[8 + k] = b;
-        }
-    } else {
-        uint32_t rw[WORDS] = {}, tw[WORDS] = {};
-        if (lane < N) {
-            const size_t o = (size_t)(py - N / 2 + lane) * p.stride + (px - N / 2);
-            load_row<WORDS>(p.ref + o, N, rw);
-            load_row<WORDS>(p.tar + o, N, tw);
-        }
+        for (int k = 0; k < Rows::LOADS; ++k) {
+            Rows::words(rows.r[k], N, lane, rw[k]);
+            Rows::words(rows.t[k], N, lane, tw[k]);
 #pragma unroll
-        for (int k = 0; k < WORDS; ++k) {
-            const int x = 4 * k;
-            const uint32_t keep = x + 4 <= N ? ~0u : x >= N ? 0u : 0xffffu;   // N is even
-            rw[k] &= keep;
-            tw[k] &= keep;
-            sr = (int)__builtin_amdgcn_udot4(rw[k], 0x01010101u, (uint32_t)sr, false);
-            st = (int)__builtin_amdgcn_udot4(tw[k], 0x01010101u, (uint32_t)st, false);
-            srr = (int)__builtin_amdgcn_udot4(rw[k], rw[k], (uint32_t)srr, false);
-            stt = (int)__builtin_amdgcn_udot4(tw[k], tw[k], (uint32_t)stt, false);
-        }
-        wave_lds_sync();                       // the previous POI's reads of this region are done
-        if (lane < N) {
-            uint2* er = reinterpret_cast<uint2*>(ex + lane * Sm::RP);
-            uint8_t* trow = ex + Sm::ROWS * Sm::RP + lane * Sm::TP;
-            uint2* et = reinterpret_cast<uint2*>(trow);
-#pragma unroll
-            for (int k = 0; k < WORDS / 2; ++k) {
-                er[k] = make_uint2(rw[2 * k], rw[2 * k + 1]);
-                et[k] = make_uint2(tw[2 * k], tw[2 * k + 1]);
-            }
-            // the T row again from byte N on (up to byte 2 N - 1 it is read)
-            uint32_t* t32 = reinterpret_cast<uint32_t*>(trow) + (N >> 2);
-            if ((N & 2) == 0) {
-#pragma unroll
-                for (int e = 0; e < WORDS; ++e) t32[e] = tw[e];
-            } else {                                       // N = 4 n + 2: bytes 0, 1 at N, then shifted words
-                *reinterpret_cast<uint16_t*>(trow + N) = (uint16_t)tw[0];
-#pragma unroll
-                for (int e = 0; e + 1 < WORDS; ++e) t32[1 + e] = __builtin_amdgcn_alignbyte(tw[e + 1], tw[e], 2);
+            for (int w = 0; w < 4; ++w) {
+                sums[0] = (int)__builtin_amdgcn_udot4(rw[k][w], 0x01010101u, (uint32_t)sums[0], false);
+                sums[1] = (int)__builtin_amdgcn_udot4(tw[k][w], 0x01010101u, (uint32_t)sums[1], false);
+                sums[2] = (int)__builtin_amdgcn_udot4(rw[k][w], rw[k][w], (uint32_t)sums[2], false);
+                sums[3] = (int)__builtin_amdgcn_udot4(tw[k][w], tw[k][w], (uint32_t)sums[3], false);
             }
         }
+        wave_lds_sync();                           // the previous POI's reads of this region are done
+        uint8_t* er = ex + (lane / CH) * Sm::RP + 16 * (lane % CH);
+        uint8_t* et = ex + Sm::ROWS * Sm::RP + (lane / CH) * Sm::TP + 16 * (lane % CH);
+#pragma unroll
+        for (int k = 0; k < Rows::LOADS; ++k)
+            if (Rows::active(k, lane, N)) {
+                uint2* e2 = reinterpret_cast<uint2*>(er + k * Rows::RL * Sm::RP);
+                uint2* t2 = reinterpret_cast<uint2*>(et + k * Rows::RL * Sm::TP);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    e2[e] = make_uint2(rw[k][2 * e], rw[k][2 * e + 1]);
+                    t2[e] = make_uint2(tw[k][2 * e], tw[k][2 * e + 1]);
+                }
+            }
+        // the T rows again from byte N on (up to byte 2 N - 1 they are read),
+        // over the zeros of the last piece
+#pragma unroll
+        for (int k = 0; k < Rows::LOADS; ++k)
+            if (Rows::active(k, lane, N)) {
+                uint8_t* again = et + k * Rows::RL * Sm::TP + N;
+                if constexpr (FULL) {
+                    reinterpret_cast<uint2*>(again)[0] = make_uint2(tw[k][0], tw[k][1]);
+                    reinterpret_cast<uint2*>(again)[1] = make_uint2(tw[k][2], tw[k][3]);
+                } else {
+                    __builtin_memcpy(again, tw[k], 16);
+                }
+            }
     }
-    sr = dpp_sum(sr); st = dpp_sum(st); srr = dpp_sum(srr); stt = dpp_sum(stt);
-    const long long Sr = sr, St = st, Srr = srr, Stt = stt;
-    if (Srr * NN == Sr * Sr || Stt * NN == St * St) {          // flat window (:271-275)
-        if (lane == 0 && p.status) p.status[poi] = TWDIC_FFTCC_FLAT;
-        return;
-    }
-    const int a = (int)((uint32_t)(sr + NN / 2) / (uint32_t)NN), b = (int)((uint32_t)(st + NN / 2) / (uint32_t)NN);   // rounded means
+    dpp_sum4(sums);
+    const int a = (int)((uint32_t)(sums[0] + NN / 2) / (uint32_t)NN);             // rounded means
+    const int b = (int)((uint32_t)(sums[1] + NN / 2) / (uint32_t)NN);
     const h2v oa = {(_Float16)(1024 + a), (_Float16)(1024 + a)};
     const h2v ob = {(_Float16)(1024 + b), (_Float16)(1024 + b)};
-    const double nr2 = (double)(Srr - 2LL * a * Sr + (long long)a * a * NN);     // ||r||^2, exact
-    const double nt2 = (double)(Stt - 2LL * b * St + (long long)b * b * NN);
-    const double rho = sqrt(nr2 * nt2);
-    int ex2;
-    (void)frexp((double)NN * rho, &ex2);
-    const float s = ldexpf(1.0f, 14 - ex2);                                      // s N^2 rho in [2^13, 2^14)
-    const double bound = FULL ? kDftBound : kDftBoundN * (double)NN / 4096.0;
-    const float tol = (float)(2.0 * 1.25 * bound * rho * (double)s / 65536.0);     // in C^ units (s 2^-16 N^2 C)
+    // ||r||^2, ||t||^2, exact below 2^31; zero for a uniform window, whose
+    // rounded mean is its value, and for no other: flat (:271-275)
+    const int nr2 = sums[2] - 2 * a * sums[0] + a * a * NN, nt2 = sums[3] - 2 * b * sums[1] + b * b * NN;
+    if (nr2 == 0 || nt2 == 0) {
+        next();
+        return false;
+    }
+    // the tolerance's factor 1.25 over the bound dwarfs the FP32 rounding here
+    const float rho = __builtin_amdgcn_sqrtf((float)nr2) * __builtin_amdgcn_sqrtf((float)nt2);
+    const float s = ldexpf(1.0f, 14 - __builtin_amdgcn_frexp_expf((float)NN * rho));   // s N^2 rho in [2^13, 2^14)
+    const float bound = FULL ? (float)kDftBound : (float)(kDftBoundN / 4096.0) * (float)NN;
+    const float tol = 2.5f / 65536.f * bound * rho * s;                          // in C^ units (s 2^-16 N^2 C)
     wave_lds_sync();
 
     const int wave_f = FULL ? wave : 0;
@@ -1593,20 +1678,24 @@ __device__ __forceinline__ void fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int 
         }
     uint64_t mask = ((uint64_t)mw[1] << 32) | mw[0];
 
-    // -- exact integer correlation at the candidates, in increasing index order ---
+    next();
+
+    // -- exact integer correlation at the candidates: the largest, of equal ones
+    //    the lowest index ------------------------------------------------------
     const uint32_t* rrow = reinterpret_cast<const uint32_t*>(erows + (FULL || lane < N ? lane : 0) * Sm::RP);
-    int bestI = -1, peak = -1;
-    for (;;) {
-        int mine = INT_MAX;
-        if (mask) {
-            const int bit = __builtin_ctzll(mask);
-            const int Nd = bit >> 5, Md = (bit >> 4) & 1, r = bit & 15;
-            mine = (32 * Nd + m) * 64 + 32 * Md + 8 * (r >> 2) + 4 * h + (r & 3);
-        }
-        const int k = dpp_min(mine);
-        if (k == INT_MAX) break;
+    bestI = -1;
+    peak = 0;
+    // a lane's lowest candidate as 64 a + b
+    auto lowest = [&]() {
+        const int bit = __builtin_ctzll(mask | (1ull << 63));
+        const int Nd = bit >> 5, Md = (bit >> 4) & 1, r = bit & 15;
+        return (32 * Nd + m) * 64 + 32 * Md + 8 * (r >> 2) + 4 * h + (r & 3);
+    };
+    for (unsigned long long lanes; (lanes = __ballot(mask != 0)) != 0;) {
+        const int from = __builtin_ctzll(lanes), k = __builtin_amdgcn_readlane(lowest(), from);
+        if (lane == from) mask &= mask - 1;
         const int kv = k >> 6, ku = k & 63, d = ku >> 2, sh = ku & 3;
-        int ty = lane + kv;                    // row (lane + kv) mod N
+        int ty = lane + kv;                        // row (lane + kv) mod N
         if constexpr (FULL)
             ty &= 63;
         else
@@ -1621,23 +1710,12 @@ __device__ __forceinline__ void fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int 
             w0 = w1;
         }
         const int I = dpp_sum(FULL || lane < N ? (int)acc : 0);
-        if (I > bestI) {
+        if (I > bestI || (I == bestI && k < peak)) {
             bestI = I;
             peak = k;
         }
-        if (mine == k) mask &= mask - 1;
     }
-    if (lane == 0) {
-        const double nr = (double)Srr - (double)Sr * (double)Sr / (double)NN;
-        const double nt = (double)Stt - (double)St * (double)St / (double)NN;
-        int iu = peak & 63, iv = peak >> 6;    // wrapped to the reference's (u, v) (:316-322)
-        if (iu > N / 2) iu -= N;
-        if (iv > N / 2) iv -= N;
-        p.u[poi] = (float)iu;
-        p.v[poi] = (float)iv;
-        p.zncc[poi] = (float)(((double)bestI - (double)Sr * (double)St / (double)NN) / sqrt(nr * nt));
-        if (p.status) p.status[poi] = TWDIC_FFTCC_OK;
-    }
+    return true;
 }
 
 // A workgroup's wavefronts share the DFT tables in LDS; workgroup b takes the
@@ -1706,38 +1784,125 @@ __device__ __forceinline__ int dft_range_index()
     return (G & 7) == 0 ? (b & 7) * (G >> 3) + (b >> 3) : b;
 }
 
+// A wavefront's share of the items [lo, hi): every WAVES-th.  The next item's
+// rows are loaded while the current one's candidates are evaluated (of 22,600
+// cycles per POI 4,100 went by waiting for its place and rows), and the
+// outputs, some 100 FP64 instructions, are formed for KEPT items at a time, a lane
+// each, instead of by one lane per item.  With the rows' loads in DftRows:
+// 0.81 -> 0.73 ms for 155k POIs at N = 64, 0.53 -> 0.48 ms at N = 40.  src.item(i) is the window pair of item i, src.params(i)
+// its outputs, src.poi(i) their index.
+template <int CH, bool FULL, class Source>
+__device__ __forceinline__ void fftcc_dft_run(DftWgSmem<CH, FULL>& sm, const Source& src, int N, int lo, int hi)
+{
+    using Sm = DftWgSmem<CH, FULL>;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    int (*kept)[Sm::KEPT] = sm.kept[wave];
+    int nkept = 0;
+    auto flush = [&]() {
+        wave_lds_sync();
+        if (lane < nkept) {
+            const int i = kept[0][lane], I = kept[5][lane], peak = kept[6][lane];
+            const double sr = kept[1][lane], st = kept[2][lane], srr = kept[3][lane], stt = kept[4][lane];
+            const FftccParams p = src.params(i);
+            const int poi = src.poi(i);
+            const double NN = (double)(N * N);
+            const double nr = srr - sr * sr / NN, nt = stt - st * st / NN;
+            int iu = peak & 63, iv = peak >> 6;    // wrapped to the reference's (u, v) (:316-322)
+            if (iu > N / 2) iu -= N;
+            if (iv > N / 2) iv -= N;
+            p.u[poi] = (float)iu;
+            p.v[poi] = (float)iv;
+            p.zncc[poi] = (float)(((double)I - sr * st / NN) / sqrt(nr * nt));
+            if (p.status) p.status[poi] = TWDIC_FFTCC_OK;
+        }
+        wave_lds_sync();
+        nkept = 0;
+    };
+    auto fail = [&](int i, int status) {
+        const FftccParams p = src.params(i);
+        if (lane == 0 && p.status) p.status[src.poi(i)] = (uint8_t)status;
+    };
+    int i = lo + wave;
+    if (i >= hi) return;
+    DftRows<CH, FULL> rows;
+    DftItem cur = src.item(i);
+    rows.drop();
+    if (cur.inside) rows.load(cur, N, lane);
+    for (;;) {
+        const int ni = i + Sm::WAVES;
+        DftItem nx = cur;
+        if (ni < hi) nx = src.item(ni);
+        auto next = [&]() {
+            rows.drop();
+            if (ni < hi && nx.inside) rows.load(nx, N, lane);
+        };
+        if (cur.inside) {
+            int sums[4], I, peak;
+            if (fftcc_dft_mfma_poi<CH, FULL>(sm, wave, lane, N, cur, rows, sums, I, peak, next)) {
+                if (lane == 0) {
+                    const int v[7] = {i, sums[0], sums[1], sums[2], sums[3], I, peak};
+#pragma unroll
+                    for (int f = 0; f < 7; ++f) kept[f][nkept] = v[f];
+                }
+                if (++nkept == Sm::KEPT) flush();
+            } else {
+                fail(i, TWDIC_FFTCC_FLAT);
+            }
+        } else {
+            next();
+            fail(i, TWDIC_FFTCC_OUT);
+        }
+        if (ni >= hi) break;
+        i = ni;
+        cur = nx;
+    }
+    flush();
+}
+
+struct DftSet {                                    // the POIs of one set
+    const FftccParams& p;
+    __device__ __forceinline__ DftItem item(int i) const { return dft_item(p, i); }
+    __device__ __forceinline__ const FftccParams& params(int) const { return p; }
+    __device__ __forceinline__ int poi(int i) const { return i; }
+};
+
+struct DftBatch {                                  // items (pair, POI) of a batch
+    const PairDesc* pairs;
+    const int2* items;
+    __device__ __forceinline__ DftItem item(int i) const
+    {
+        const int2 it = items[i];
+        return dft_item(const_pairs(pairs)[__builtin_amdgcn_readfirstlane(it.x)].fftcc,
+                        __builtin_amdgcn_readfirstlane(it.y));
+    }
+    __device__ __forceinline__ FftccParams params(int i) const { return const_pairs(pairs)[items[i].x].fftcc; }
+    __device__ __forceinline__ int poi(int i) const { return items[i].y; }
+};
+
 template <int CH, bool FULL>
 __global__ __launch_bounds__((64 * DftWgSmem<CH, FULL>::WAVES), 1) void k_fftcc_dft_mfma(FftccParams p)
 {
     __shared__ DftWgSmem<CH, FULL> sm;
     dft_tables_to_lds(sm, p.tw, p.N);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = dft_range_index();
     const int lo = (int)((long long)g * p.n / gridDim.x);
     const int hi = (int)((long long)(g + 1) * p.n / gridDim.x);
-    for (int poi = lo + wave; poi < hi; poi += DftWgSmem<CH, FULL>::WAVES) fftcc_dft_mfma_poi(sm, wave, lane, p, poi);
+    fftcc_dft_run<CH, FULL>(sm, DftSet{p}, FULL ? 64 : p.N, lo, hi);
 }
 
 // Batched form over items (pair, POI) of pairs that share N: the same ranges
-// per workgroup, each wavefront reading its item's pair descriptor.
+// per workgroup, each item with its pair's descriptor.
 template <int CH, bool FULL>
 __global__ __launch_bounds__((64 * DftWgSmem<CH, FULL>::WAVES), 1) void k_batch_fftcc_dft_mfma(
     const PairDesc* __restrict__ pairs, const int2* __restrict__ items, int count)
 {
     __shared__ DftWgSmem<CH, FULL> sm;
-    {
-        const FftccParams p = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(items[0].x)].fftcc;
-        dft_tables_to_lds(sm, p.tw, p.N);
-    }
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const FftccParams p = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(items[0].x)].fftcc;
+    dft_tables_to_lds(sm, p.tw, p.N);
     const int g = dft_range_index();
     const int lo = (int)((long long)g * count / gridDim.x);
     const int hi = (int)((long long)(g + 1) * count / gridDim.x);
-    for (int i = lo + wave; i < hi; i += DftWgSmem<CH, FULL>::WAVES) {
-        const int2 it = items[i];
-        const FftccParams p = const_pairs(pairs)[__builtin_amdgcn_readfirstlane(it.x)].fftcc;
-        fftcc_dft_mfma_poi(sm, wave, lane, p, __builtin_amdgcn_readfirstlane(it.y));
-    }
+    fftcc_dft_run<CH, FULL>(sm, DftBatch{pairs, items}, FULL ? 64 : p.N, lo, hi);
 }
 
 // workgroups for n POIs: one per compute unit (each holds one), fewer for
