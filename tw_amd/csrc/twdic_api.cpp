@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -89,6 +91,55 @@ twdic_status check_spans(twdic_ctx* c, const char* call, std::initializer_list<N
         twdic_status s_ = check_spans((ctx), (call), {__VA_ARGS__});       \
         if (s_ != TWDIC_OK) return s_;                                     \
     } while (0)
+
+// A small device-to-host copy through the context's pinned buffer, behind the
+// stream's work like any other; false: not taken, nothing was done.  Taken for
+// device memory of the context's own device going to memory that is no device
+// memory, outside a capture (a captured copy is the runtime's to refuse), one
+// at a time.  Up to 16 KiB, the size up to which the runtime stages its copies:
+// 22.5 us by the runtime, 9.4 us here for 25 bytes, 10.8 for 4 KiB, 17.9 for
+// 16 KiB; from 16.4 KB on the runtime's direct copy takes 10.4 us.
+bool download_small(twdic_ctx* c, void* dst, const void* src, size_t bytes, hipError_t* result)
+{
+    if (!c->h_down || bytes > kDownBytes) return false;
+    int device = -1;
+    hipPointerAttribute_t a{};
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipGetDevice(&device) != hipSuccess || device != c->device) return false;
+    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
+    if (hipPointerGetAttributes(&a, src) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (a.type != hipMemoryTypeDevice || a.device != c->device) return false;
+    size_t span = 0;
+    if (device_span(dst, &span)) return false;
+    if (c->down_busy.test_and_set(std::memory_order_acquire)) return false;
+    struct Release {
+        std::atomic_flag& f;
+        ~Release() { f.clear(std::memory_order_release); }
+    } release{c->down_busy};
+    auto* flag = reinterpret_cast<std::atomic<uint32_t>*>(c->h_down + kDownBytes);
+    const uint32_t seq = ++c->down_seq;
+    if (launch_to_host(src, c->d_down, bytes, reinterpret_cast<uint32_t*>(c->d_down + kDownBytes), seq, c->stream) !=
+        hipSuccess)
+        return false;
+    // the flag as long as the wait is short; behind longer work the runtime's
+    // wait, which also returns the stream's errors
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    bool here = false;
+    do {
+        for (int i = 0; i < 32 && !here; ++i) here = flag->load(std::memory_order_acquire) == seq;
+    } while (!here && std::chrono::steady_clock::now() < until);
+    if (!here) {
+        *result = hipStreamSynchronize(c->stream);
+        if (*result != hipSuccess) return true;
+        if (flag->load(std::memory_order_acquire) != seq) return false;
+    }
+    std::memcpy(dst, c->h_down, bytes);
+    *result = hipSuccess;
+    return true;
+}
 
 // Fftcc2D::recomputeNumPOI (TW_paDIC_FFTCC2D.cpp:88-94): float division,
 // floor, truncation (a negative count, as the reference computes it, marks
@@ -386,6 +437,17 @@ twdic_status twdic_create(const twdic_config* cfg, int device, twdic_ctx** out)
         if ((e = hipEventCreate(&c->ev[i])) != hipSuccess) bail(e, "hipEventCreate");
     for (int i = 0; i <= twdic_ctx::kMaxFrameChunks && st == TWDIC_OK; ++i)
         if ((e = hipEventCreateWithFlags(&c->pev[i], hipEventDisableTiming)) != hipSuccess) bail(e, "hipEventCreate");
+    // without it (no error) small downloads go the way of large ones
+    if (st == TWDIC_OK) {
+        if (hipHostMalloc((void**)&c->h_down, kDownBytes + 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+            hipHostGetDevicePointer((void**)&c->d_down, c->h_down, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            if (c->h_down) (void)hipHostFree(c->h_down);
+            c->h_down = nullptr;
+        } else {
+            std::memset(c->h_down, 0, kDownBytes + 64);
+        }
+    }
     if (st == TWDIC_OK) {
         // twiddles exp(-2 pi i e / N), rounded from double
         float2 tw[kMaxFftN];
@@ -417,6 +479,7 @@ twdic_status twdic_destroy(twdic_ctx* c)
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
+    if (c->h_down) (void)hipHostFree(c->h_down);
     for (auto& ev : c->ev)
         if (ev) (void)hipEventDestroy(ev);
     for (auto& ev : c->pev)
@@ -841,6 +904,11 @@ twdic_status twdic_memcpy(twdic_ctx* c, void* dst, const void* src, size_t bytes
     hipMemcpyKind k = kind == 0 ? hipMemcpyHostToDevice : kind == 1 ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
     if (kind < 0 || kind > 2) return fail(c, TWDIC_EINVAL, "memcpy kind");
     TW_SPANS(c, "twdic_memcpy", {kind != 1 ? dst : nullptr, bytes, "dst"}, {kind != 0 ? src : nullptr, bytes, "src"});
+    hipError_t small;
+    if (kind == 1 && download_small(c, dst, src, bytes, &small)) {
+        TW_HIP(c, small);
+        return TWDIC_OK;
+    }
     TW_HIP(c, hipMemcpyAsync(dst, src, bytes, k, c->stream));
     if (kind != 2) TW_HIP(c, hipStreamSynchronize(c->stream));
     return TWDIC_OK;

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -248,6 +249,10 @@ __device__ __forceinline__ ConstPairDescPtr const_pairs(const PairDesc* p)
 }
 
 // Kernel launch wrappers (return hipError_t of the launch).
+// `bytes` (at most kDownBytes) from device memory to the pinned buffer `out`,
+// then seq into *flag.
+constexpr size_t kDownBytes = 16384;
+hipError_t launch_to_host(const void* src, void* out, size_t bytes, uint32_t* flag, uint32_t seq, hipStream_t st);
 hipError_t launch_gradients(const uint8_t* img, int stride, int sx0, int sy0, int rw, int rh,
                             float* gx, float* gy, float* gxy, uint32_t* g2, hipStream_t st);
 hipError_t launch_bspline_lut(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float* lut,
@@ -360,6 +365,12 @@ struct twdic_ctx {
     int icgn_variant = 5;             // occupancy target of the IC-GN kernel (0: compiler's choice)
     uint8_t* h_stage = nullptr;       // pinned staging for host images
     size_t h_stage_bytes = 0;
+    // small downloads (twdic_memcpy): a pinned buffer, its device address, and
+    // the sequence number that follows its kDownBytes bytes
+    uint8_t* h_down = nullptr;
+    uint8_t* d_down = nullptr;
+    uint32_t down_seq = 0;
+    std::atomic_flag down_busy = ATOMIC_FLAG_INIT;
     hipEvent_t ev[16] = {};
     // frame pipeline: FFT-CC of POI chunk i + 1 (on `stream`) overlaps IC-GN of
     // chunk i (on `stream2`)
