@@ -36,9 +36,16 @@ FP32_PEAK_TFLOPS = 157.3
 FP32_UNPACKED_PEAK_TFLOPS = 78.6    # without packed FP32 (v_pk_fma_f32), which the kernels here do not use
 INT8_MFMA_PEAK_TOPS = 5000.0
 FP16_MFMA_PEAK_TFLOPS = 2500.0
-# fp16 DFT engine (N = 64): 144 v_mfma_f32_32x32x16_f16 of 32 x 32 x 16 x 2
-# flops per POI, the half-spectrum DFT-by-matrix product with no padding
-DFT_MFMA_FLOPS_PER_POI = 144 * 32 * 32 * 16 * 2
+# fp16 DFT engine: v_mfma_f32_32x32x16_f16 of 32 x 32 x 16 x 2 flops, 144 per POI
+# (112 for N <= 48), the half-spectrum DFT-by-matrix product as it is issued
+DFT_MFMA_FLOPS = 32 * 32 * 16 * 2
+
+
+def dft_mfmas_per_poi(N: int, n: int) -> int:
+    """MFMAs per POI where the fp16 DFT engine takes the set, else 0."""
+    if N == 64 or 48 < N <= 60:
+        return 144
+    return 112 if 32 < N <= 48 and n >= 1280 else 0
 
 
 def measured_traffic() -> dict:
@@ -481,10 +488,10 @@ def main():
 
     # Roofline of each kernel from its measured launch time; the dominant
     # (longer) one is reported as "roofline".  Work conventions:
-    #   FFT-CC, default engine for N = 64: fp16 DFTs as matrix products,
-    #   DFT_MFMA_FLOPS_PER_POI against the dense fp16 MFMA peak (the exact
+    #   FFT-CC, fp16 DFT engine: fp16 DFTs as matrix products,
+    #   dft_mfmas_per_poi against the dense fp16 MFMA peak (the exact
     #   integer re-evaluation of the few near-maximal shifts is not counted);
-    #   the integer engine (other N): the whole integer correlation surface,
+    #   the integer engine (other sets): the whole integer correlation surface,
     #   2 N^4 int8 operations per POI, against the dense int8 MFMA peak; the
     #   FFT formulation's F_cc(N) = 3 * 2.5 N^2 log2(N^2) + 6 N (N/2 + 1) +
     #   7 N^2 (two forward and one inverse N x N transform, spectrum product,
@@ -498,11 +505,11 @@ def main():
     fft_ms = float(np.mean(t_fft))
     f_cc = 3 * 2.5 * N * N * np.log2(N * N) + 6 * N * (N // 2 + 1) + 7 * N * N
     variant = os.environ.get("TWDIC_FFTCC_VARIANT", "9")
-    dft = variant == "9" and N == 64
+    dft = dft_mfmas_per_poi(N, n) if variant == "9" else 0
     mma = variant not in ("2", "3", "4") and not dft
     kern = {
         "k_fftcc": {"ms": fft_ms, "flops": f_cc * n, "int8_ops": 2.0 * N ** 4 * n if mma else None,
-                    "fp16_flops": float(DFT_MFMA_FLOPS_PER_POI) * n if dft else None,
+                    "fp16_flops": float(dft * DFT_MFMA_FLOPS) * n if dft else None,
                     # both images read once, POI in, u/v/ZNCC out
                     "bytes": 2 * W * H + n * (8 + 12)},
         "k_icgn": {"ms": icgn_ms, "flops": 66.0 * s * kbar * n,
