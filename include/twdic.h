@@ -61,7 +61,7 @@ enum {
                                Catmull-Rom, which equals the LUT polynomial built
                                from central-difference derivatives) from the
                                target rows' cubic coefficients: 16 bytes per ROI
-                               pixel (exact in FP32), built once
+                               pixel (exact in fp16), built once
                                per target (every call once TWDIC_BUF_TAR has been
                                handed out), instead of the 64-byte LUT */
     TWDIC_INTERP_BSPLINE = 2 /* ICGN2DInterpolationFLag::BicubicSpline: the cubic

@@ -269,7 +269,8 @@ __device__ __forceinline__ float interp_fused_s(const TargetBuf& B, int ix, int 
 
 // The target's row polynomials (launch_row_poly) as a buffer resource whose
 // base is the entry of row -1, column 0: row iy - 1 of cell (ix, iy) is at
-// byte offset 16 (iy rw + ix), the rows below it 16 rw further each.  The
+// byte offset 16 (iy rw + ix) with row iy in the 8 bytes behind it, the rows
+// below 16 rw further each.  The
 // host passes the plane only when every such offset is below 2^32.
 struct RowPolyBuf {
     __amdgpu_buffer_rsrc_t r;
@@ -291,11 +292,24 @@ __device__ __forceinline__ int row_poly_offset(const RowPolyBuf& B, int ix, int 
     return (int)__umul24((uint32_t)iy, (uint32_t)B.pitch) + 16 * ix;
 }
 
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
 // the row polynomial at byte offset o, `rows` rows further down
-__device__ __forceinline__ f32x4 load_row_poly(const RowPolyBuf& B, int o, int rows)
+__device__ __forceinline__ h4 load_row_poly(const RowPolyBuf& B, int o, int rows)
 {
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(B.r, o, rows * B.pitch, 0));
+    return __builtin_bit_cast(h4, __builtin_amdgcn_raw_buffer_load_b64(B.r, o, rows * B.pitch, 0));
 }
+
+// the row polynomials there and one row below it
+__device__ __forceinline__ h8 load_row_polys(const RowPolyBuf& B, int o, int rows)
+{
+    return __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(B.r, o, rows * B.pitch, 0));
+}
+
+__device__ __forceinline__ h4 lower(h8 v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3); }
+__device__ __forceinline__ h4 upper(h8 v) { return __builtin_shufflevector(v, v, 4, 5, 6, 7); }
+__device__ __forceinline__ f32x4 widen(h4 v) { return __builtin_convertvector(v, f32x4); }
 
 // One row's cubic at t from its stored coefficients c0, c1/2, c2/2, c3/2:
 // c0 + t (c1/2 + t (c2/2 + t c3/2)).  Every intermediate is exactly half the
@@ -309,6 +323,12 @@ __device__ __forceinline__ float row_poly(f32x4 c, float t)
     const float s = fmaf(t, fmaf(t, c.w, c.z), c.y);
     asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r) : "v"(t), "v"(s), "v"(c.x));
     return r;
+}
+
+// the same from the halves: mixed-precision FMAs take them as exact operands
+__device__ __forceinline__ float row_poly(h4 c, float t)
+{
+    return fmaf(t, fmaf(t, fmaf(t, (float)c.w, (float)c.z), (float)c.y), (float)c.x);
 }
 
 // Bicubic value from the cubics of the four rows iy - 1 .. iy + 2 at tx: the
@@ -455,24 +475,34 @@ __device__ __forceinline__ void kahan_pixel(float ks[8], float kc[8], float T, u
 // The bicubic passes over the row polynomials (ROLL) also keep the four rows
 // of the current cell in registers: in a column the next pixel's cell is the
 // one below unless a cell border runs between them, so a pixel loads one row
-// instead of four, and as its place is known beforehand, a pixel ahead.  The
-// fractional parts are then the coordinates less the expected cell's corner,
-// and one unsigned compare of both tells whether the pixel lies in it.  Their
-// integer pass (GROUP) issues the loads of eight rows together: with one row's
-// at a time a lone wavefront waited for memory once a row, 14,000 cycles for
-// 31x31 pixels where the groups take 6,100 (the kernel 28.2 -> 24.2 us for 25
-// POIs, 118 -> 115 us for 11k, 1.13 -> 1.11 ms for 157k); in B-spline mode,
+// (8 bytes, widened once for its four uses) instead of two entries, and as its
+// place is known beforehand, a pixel ahead.  The fractional parts are then the
+// coordinates less the expected cell's corner, and one unsigned compare of both
+// tells whether the pixel lies in it.  With KEEP
+// unset a pixel's two entries are loaded directly.
+// Their integer pass (GROUP) issues the loads of eight rows together: with one
+// row's at a time a lone wavefront waited for memory once a row, 14,000 cycles
+// for 31x31 pixels where the groups take 6,100 (the kernel 28.2 -> 24.2 us for
+// 20 POIs, 118 -> 115 us for 11k, 1.13 -> 1.11 ms for 157k); in B-spline mode,
 // whose lanes are dealt rows in turn, it is no gain (0.398 -> 0.413 ms for 28k
 // POIs).
 //
-// Bound by VALU issue: 84 % of the slots on the 2048^2 frame (157,609 POIs of
-// 41x41).  There a walk in row-major order from a table of pixel offsets took
-// 1.35 ms (58 VALU instructions per bicubic pixel, of them 12 mixed-precision
-// ones of 1.5 slots, 26 per integer pixel), walking columns 1.20 ms (47 and
-// 16; two rows per trip 1.27 ms), keeping the rows 1.07 ms (48, all of one
-// slot); 14k POIs on whole wavefronts 0.153, 0.139, 0.123 ms.  W1 dy and W4 dy
-// from an LDS table (45 instructions) changed nothing.
-template <int L, int INTERP, bool INT, bool CHECK, bool RP, bool K32 = false>
+// Bound by VALU issue (a row-major walk from a table of pixel offsets: 58 VALU
+// instructions per bicubic pixel, 12 of them mixed-precision ones of 1.5 slots,
+// 26 per integer pixel; walking columns 47 and 16; keeping the rows 52, all of
+// one slot).  104k POIs of 41x41, ms:
+//   strain of the field   row-major   columns   rows kept   rows kept, FP32 plane
+//   0                     0.95        0.87      0.78        0.71
+//   0.2 %                 0.97        0.89      0.85        0.79
+//   0.4 %                 0.98        0.90      0.88        0.83
+//   0.7 %                 0.99        0.90      0.94        0.93
+//   1 %                   1.02        0.92      0.99        1.02
+//   4 % (POIs astray)     7.75        7.71      8.69        11.4
+// hence the rule in subset_pass.  With one FP32 row per 16 bytes (no widening, 48
+// instructions) a cell takes four loads instead of two whenever its rows are not
+// at hand, so a batch of 64 mixed pairs took 249 ms (row-major 228, these 202).
+// W1 dy and W4 dy from an LDS table changed nothing.
+template <int L, int INTERP, bool INT, bool CHECK, bool RP, bool K32 = false, bool KEEP = false>
 __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py, const float Wm[6], int lane,
                                             double acc[8], const StripLane* tab)
 {
@@ -481,7 +511,7 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     // the sums are scaled back at the end, exactly
     constexpr bool SCALED = !INT && INTERP == TWDIC_INTERP_FUSED && !RP;
     constexpr bool ROWS = RP && INTERP != TWDIC_INTERP_BSPLINE;      // the target's rows as polynomials
-    constexpr bool ROLL = ROWS && !INT && !CHECK && !K32;
+    constexpr bool ROLL = KEEP && ROWS && !INT && !CHECK && !K32;
     constexpr bool GROUP = ROWS && INT && !CHECK && !K32;
     constexpr int kNoPixel = 0x7fffffff;          // past every image (target_buf: records fit an int)
     const int sx0 = P.sx0, sy0 = P.sy0, rw = P.rw, rh = P.rh;
@@ -556,12 +586,11 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                 T = interp_planes(P.rp, (size_t)rw * rh, (uint32_t)((iy - sy0) * rw + (ix - sx0)), tx, ty);
             } else if constexpr (RP) {
                 const int o = row_poly_offset(rb, ix, iy);
-                const f32x4 q0 = load_row_poly(rb, o, 0), q1 = load_row_poly(rb, o, 1), q2 = load_row_poly(rb, o, 2),
-                            q3 = load_row_poly(rb, o, 3);
+                const h8 a = load_row_polys(rb, o, 0), b = load_row_polys(rb, o, 2);
                 if constexpr (INTERP == TWDIC_INTERP_LUT)
-                    T = lut_cubic(q0, q1, q2, q3, tx, ty);
+                    T = lut_cubic(widen(lower(a)), widen(upper(a)), widen(lower(b)), widen(upper(b)), tx, ty);
                 else
-                    T = column_cubic(row_poly(q0, tx), row_poly(q1, tx), row_poly(q2, tx), row_poly(q3, tx), ty);
+                    T = column_cubic(row_poly(lower(a), tx), row_poly(upper(a), tx), row_poly(lower(b), tx), row_poly(upper(b), tx), ty);
             } else if (INTERP == TWDIC_INTERP_FUSED) {
                 T = interp_fused_s(tb, ix, iy, tx, ty);
             } else {
@@ -602,8 +631,14 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                 int o = row_poly_offset(rb, (int)wx, (int)wy);
                 float fx = (float)(int)wx, fy = (float)(int)wy;
                 f32x4 q[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) q[i] = load_row_poly(rb, o, i);
+                h4 fresh;
+                {
+                    const h8 a = load_row_polys(rb, o, 0), b = load_row_polys(rb, o, 2);
+                    q[0] = widen(lower(a));
+                    q[1] = widen(upper(a));
+                    q[2] = widen(lower(b));
+                    fresh = upper(b);
+                }
                 uint32_t g = gradient(go, 0);
                 auto next = [&](auto k) {
                     constexpr int K = decltype(k)::value;
@@ -617,18 +652,23 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                         tx = wx - fx;
                         ty = wy - fy;
                         o = row_poly_offset(rb, ix, iy);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) q[(K + i) & 3] = load_row_poly(rb, o, i);
+                        const h8 a = load_row_polys(rb, o, 0), b = load_row_polys(rb, o, 2);
+                        q[K] = widen(lower(a));
+                        q[(K + 1) & 3] = widen(upper(a));
+                        q[(K + 2) & 3] = widen(lower(b));
+                        fresh = upper(b);
                     }
+                    q[(K + 3) & 3] = widen(fresh);
+                    asm volatile("" : "+v"(q[(K + 3) & 3]));
                     so += 4 * rw;
                     const uint32_t gn = gradient(go, so);
                     float T;
                     if constexpr (INTERP == TWDIC_INTERP_LUT) {
                         T = lut_cubic(q[K], q[(K + 1) & 3], q[(K + 2) & 3], q[(K + 3) & 3], tx, ty);
-                        q[K] = load_row_poly(rb, o, 4);
+                        fresh = load_row_poly(rb, o, 4);
                     } else {
                         const float R0 = row_poly(q[K], tx);
-                        q[K] = load_row_poly(rb, o, 4);
+                        fresh = load_row_poly(rb, o, 4);
                         T = column_cubic(R0, row_poly(q[(K + 1) & 3], tx), row_poly(q[(K + 2) & 3], tx),
                                          row_poly(q[(K + 3) & 3], tx), ty);
                     }
@@ -744,7 +784,16 @@ __device__ __forceinline__ bool subset_pass(const IcgnParams& P, int px, int py,
     const bool safe = cx - rx >= (float)(P.sx0 + 1) && cx + rx < (float)(P.sx0 + P.rw - 2) &&
                       cy - ry >= (float)(P.sy0 + 1) && cy + ry < (float)(P.sy0 + P.rh - 2);
     // both halves take the same loop: the per-pixel tests run unless every
-    // active lane's POI is safe
+    // active lane's POI is safe.
+    if constexpr (RP && INTERP != TWDIC_INTERP_BSPLINE && !INT && !K32) {
+        // |W4 - 1| + |W1| is how often a lane's next pixel is in another cell than the
+        // one below.  At 0.006 half the rows of 64 lanes hold such a pixel and both
+        // forms take the same (0.002 strain: 0.85 against 0.89 ms, 0.004: 0.88 and
+        // 0.90, 0.007: 0.94 and 0.90; the table above)
+        constexpr float kGentle = 0.006f;
+        const bool gentle = fabsf(Wm[4] - 1.f) + fabsf(Wm[1]) < kGentle;
+        if (__all(safe && gentle)) return subset_loop<L, INTERP, INT, false, RP, K32, true>(P, px, py, Wm, lane, acc, tab);
+    }
     if (__all(safe)) return subset_loop<L, INTERP, INT, false, RP, K32>(P, px, py, Wm, lane, acc, tab);
     return subset_loop<L, INTERP, INT, true, RP, K32>(P, px, py, Wm, lane, acc, tab);
 }

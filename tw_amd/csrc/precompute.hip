@@ -237,27 +237,36 @@ hipError_t launch_bicubic_lut(const uint8_t* tar, int stride, int sx0, int sy0, 
 // and x + 1, its cubic through p0..p3 = T(y, x-1 .. x+2) is
 //   R(t) = c0 + t/2 (c1 + t (c2 + t c3)),
 //   c0 = p1, c1 = p2 - p0, c2 = 2 p0 - 5 p1 + 4 p2 - p3, c3 = 3 (p1 - p2) + p3 - p0,
-// integers of magnitude at most 1530.  Stored as c0, c1/2, c2/2, c3/2 in FP32
+// integers of magnitude at most 1530.  Stored as c0, c1/2, c2/2, c3/2 in fp16
 // (exactly), the cubic is c0 + t (c1/2 + t (c2/2 + t c3/2)).  Entry (x, j) holds
-// the four coefficients (16 bytes) of row y = sy0 - 1 + j for cell column
+// the coefficients (8 bytes each) of rows y = sy0 - 1 + j and y + 1 for cell column
 // sx0 + x, x < rw, j <= rh + 1; the last column (never an interior cell) is
-// zero.  A cell's four neighbourhood rows are the entries (x, j) .. (x, j + 3).
+// zero.  A cell's four neighbourhood rows are the entries (x, j) and (x, j + 2),
+// and a single row the first half of its entry.
 // ---------------------------------------------------------------------------
-// Entry (x, j) from the target row's dword at columns sx0 + x - 1 ..
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
+// Entry (x, j) from the target rows' dwords at columns sx0 + x - 1 ..
 // sx0 + x + 2: for x < rw - 1 it lies in the image (the ROI keeps a one-pixel
 // frame); the buffer's range check would read anything past its last row as
 // zero.  The target resource's base is the image, records (sy0 + rh + 1) rows.
 __device__ __forceinline__ void row_poly_entry(__amdgpu_buffer_rsrc_t img, int stride, int sx0, int sy0, int rw,
                                                int x, int j, float4* __restrict__ rp)
 {
-    float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
+    h8 e = {};
     if (x < rw - 1) {
-        const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(img, (sy0 - 1 + j) * stride + (sx0 - 1 + x), 0, 0);
-        const int p0 = (int)(w & 255u), p1 = (int)((w >> 8) & 255u), p2 = (int)((w >> 16) & 255u), p3 = (int)(w >> 24);
-        e = make_float4((float)p1, 0.5f * (float)(p2 - p0), 0.5f * (float)(2 * p0 - 5 * p1 + 4 * p2 - p3),
-                        0.5f * (float)(3 * (p1 - p2) + p3 - p0));
+        const int o = (sy0 - 1 + j) * stride + (sx0 - 1 + x);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(img, o, r * stride, 0);
+            const int p0 = (int)(w & 255u), p1 = (int)((w >> 8) & 255u), p2 = (int)((w >> 16) & 255u), p3 = (int)(w >> 24);
+            e[4 * r] = (_Float16)(float)p1;
+            e[4 * r + 1] = (_Float16)(0.5f * (float)(p2 - p0));
+            e[4 * r + 2] = (_Float16)(0.5f * (float)(2 * p0 - 5 * p1 + 4 * p2 - p3));
+            e[4 * r + 3] = (_Float16)(0.5f * (float)(3 * (p1 - p2) + p3 - p0));
+        }
     }
-    rp[(size_t)j * rw + x] = e;
+    rp[(size_t)j * rw + x] = __builtin_bit_cast(float4, e);
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_poly_src(const uint8_t* tar, int stride, int sy0, int rh)

@@ -5,7 +5,7 @@
 // buffer over the link and then raises a sequence number beside them, which the
 // host polls (twdic_memcpy).  Bound by the launch and one link round trip: 9.4 us
 // for 25 bytes and 10.8 us for 4 KiB, where the runtime's copy and wait took
-// 22.5 us; six results of 25 POIs with their frame 186 -> 118 us.
+// 22.5 us; six results of 20 POIs with their frame 186 -> 118 us.
 #include "twdic_internal.h"
 
 namespace twdic {
