@@ -735,7 +735,12 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                 }
                 walked = r;
             } else {
-#pragma unroll 1
+                // direct cells, whole wavefronts: two rows per trip, as a lone wavefront
+                // waits for each one's loads (9,409 POIs: 1 % strain 0.138 -> 0.125 ms, POIs
+                // astray 1.03 -> 0.92; four rows 0.16 and 1.08); with halves, whose
+                // wavefronts hide it, one (two: 1.20 -> 1.27 ms for 157k POIs)
+                constexpr int U = ROWS && !INT && L == 64 ? 2 : 1;
+#pragma unroll U
                 for (int r = 0; r < full; ++r) {
                     pixel(cx, cy, e.dx, dy, go, so);
                     dy += (float)step;
