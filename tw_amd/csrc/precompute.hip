@@ -316,6 +316,71 @@ hipError_t launch_batch_row_poly(const PairDesc* pairs, int npairs, int max_rh, 
 }
 
 // ---------------------------------------------------------------------------
+// The LUT from the layouts IC-GN reads instead of it, once per context: when the
+// LUT is handed out, its cells must be those of the target IC-GN last ran on,
+// which the image buffer need no longer hold.  Once: a launch recorded into a
+// graph does nothing where another has done it (done).  Bound by the 64 bytes
+// written per cell.
+// ---------------------------------------------------------------------------
+
+// a[k][l], the coefficient of y^k x^l, is a small-integer combination of the row
+// coefficients, exact in FP32 (multiples of 1/4 below 2^14), as k_bicubic_lut's
+// sums are, so the two write the same numbers.
+__global__ __launch_bounds__(256) void k_lut_of_rows(const float4* __restrict__ rp, int rw, int rh,
+                                                     float4* __restrict__ lut, const int* done)
+{
+    if (*done) return;
+    const int x = blockIdx.x * 64 + (threadIdx.x & 63), y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (x >= rw || y >= rh) return;
+    float a[4][4] = {};
+    if (x < rw - 1 && y < rh - 1) {               // the last row and column are zero
+        // rows y - 1, y and y + 1, y + 2
+        const h8 e0 = __builtin_bit_cast(h8, rp[(size_t)y * rw + x]);
+        const h8 e2 = __builtin_bit_cast(h8, rp[(size_t)(y + 2) * rw + x]);
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const float q0 = (float)e0[l], q1 = (float)e0[4 + l], q2 = (float)e2[l], q3 = (float)e2[4 + l];
+            a[0][l] = q1;
+            a[1][l] = 0.5f * (q2 - q0);
+            a[2][l] = 0.5f * (2.f * q0 - 5.f * q1 + 4.f * q2 - q3);
+            a[3][l] = 0.5f * (3.f * (q1 - q2) + (q3 - q0));
+        }
+    }
+    float4* out = lut + 4 * ((size_t)y * rw + x);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) out[k] = make_float4(a[k][0], a[k][1], a[k][2], a[k][3]);
+}
+
+__global__ __launch_bounds__(256) void k_lut_of_planes(const float4* __restrict__ planes, int rw, int rh,
+                                                       float4* __restrict__ lut, const int* done)
+{
+    if (*done) return;
+    const int x = blockIdx.x * 64 + (threadIdx.x & 63), y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (x >= rw || y >= rh) return;
+    const size_t cell = (size_t)y * rw + x, cells = (size_t)rw * rh;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) lut[4 * cell + k] = planes[k * cells + cell];
+}
+
+__global__ void k_set(int* flag) { *flag = 1; }
+
+hipError_t launch_lut_of_rows(const float4* rp, int rw, int rh, float* lut, int* done, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_lut_of_rows, dim3((rw + 63) / 64, (rh + 3) / 4), dim3(256), 0, st, rp, rw, rh,
+                       reinterpret_cast<float4*>(lut), done);
+    hipLaunchKernelGGL(k_set, dim3(1), dim3(1), 0, st, done);
+    return hipGetLastError();
+}
+
+hipError_t launch_lut_of_planes(const float4* planes, int rw, int rh, float* lut, int* done, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_lut_of_planes, dim3((rw + 63) / 64, (rh + 3) / 4), dim3(256), 0, st, planes, rw, rh,
+                       reinterpret_cast<float4*>(lut), done);
+    hipLaunchKernelGGL(k_set, dim3(1), dim3(1), 0, st, done);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Per-reference state, one POI per group of L lanes (a wavefront, or a
 // half-wavefront for large POI sets; built once per reference and POI set; the
 // reference rebuilds it on m_isRefImgUpdated, TW_paDIC_cuICGN2D.cu:883-903).

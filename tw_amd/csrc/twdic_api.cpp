@@ -233,7 +233,7 @@ twdic_status ensure_ref_grads(twdic_ctx* c)
 // Whether IC-GN reads the target from d_rp: always in the fused mode (row
 // polynomials), in the LUT and B-spline modes as long as nobody can see the
 // LUT itself (bicubic cells follow exactly from the row polynomials, icgn.hip
-// lut_cubic; the B-spline coefficients are kept as planes).  No row
+// lut_cubic; the B-spline coefficients are kept as planes; use_lut).  No row
 // polynomials: ROIs past 2^28 pixels.
 bool uses_plane(const twdic_ctx* c)
 {
@@ -281,9 +281,68 @@ hipError_t launch_target_interp(twdic_ctx* c, hipStream_t st)
     return hipSuccess;
 }
 
+bool stream_capturing(const twdic_ctx* c)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(c->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
+// A build of d_rp was enqueued: in the LUT modes it, and not d_lut, now holds the
+// table that IC-GN runs on.
+void plane_built(twdic_ctx* c)
+{
+    c->tar_rp_valid = true;
+    c->lut_behind = c->cfg.interp != TWDIC_INTERP_FUSED;
+}
+
+// d_lut from d_rp, if that is still to be done (use_lut).  Under a capture it is
+// recorded, and stays to be done for every other graph and for the next call
+// outside: whichever runs first does it, by the flag on the device.
+twdic_status settle_lut(twdic_ctx* c)
+{
+    if (!c->lut_pending) return TWDIC_OK;
+    const twdic_config& g = c->cfg;
+    TW_HIP(c, g.interp == TWDIC_INTERP_BSPLINE
+                  ? launch_lut_of_planes(c->d_rp, g.roi_w, g.roi_h, c->d_lut, c->d_lut_done, c->stream)
+                  : launch_lut_of_rows(c->d_rp, g.roi_w, g.roi_h, c->d_lut, c->d_lut_done, c->stream));
+    c->lut_pending = stream_capturing(c);
+    return TWDIC_OK;
+}
+
+// From here on the LUT modes build and read d_lut: it is handed out, or a call
+// is being captured by the caller, whose graph then runs without this code
+// knowing.  d_lut first becomes what it would be had it been built all along: the
+// table of the target IC-GN last ran on, from d_rp, since the image may have
+// changed since.
+twdic_status use_lut(twdic_ctx* c)
+{
+    if (c->cfg.interp == TWDIC_INTERP_FUSED) return TWDIC_OK;
+    if (!c->lut_exposed) {
+        c->lut_exposed = true;
+        c->lut_pending = c->lut_behind;
+        c->tar_pre_valid = c->tar_pre_valid || c->tar_rp_valid;
+    }
+    return settle_lut(c);
+}
+
+// Before a call that builds or reads the table.
+twdic_status lut_ready(twdic_ctx* c)
+{
+    const bool lut = c->lut_exposed || (c->cfg.interp != TWDIC_INTERP_FUSED && stream_capturing(c));
+    return lut ? use_lut(c) : TWDIC_OK;
+}
+
 twdic_status target_interp_prepare(twdic_ctx* c)
 {
-    bool& valid = c->cfg.interp == TWDIC_INTERP_FUSED || uses_plane(c) ? c->tar_rp_valid : c->tar_pre_valid;
+    const twdic_status st = lut_ready(c);
+    if (st != TWDIC_OK) return st;
+    if (uses_plane(c)) {
+        if (c->tar_rp_valid && !c->tar_exposed) return TWDIC_OK;
+        TW_HIP(c, launch_target_interp(c, c->stream));
+        plane_built(c);
+        return TWDIC_OK;
+    }
+    bool& valid = c->cfg.interp == TWDIC_INTERP_FUSED ? c->tar_rp_valid : c->tar_pre_valid;
     if (valid && !c->tar_exposed) return TWDIC_OK;
     TW_HIP(c, launch_target_interp(c, c->stream));
     valid = true;
@@ -419,7 +478,7 @@ twdic_status twdic_create(const twdic_config* cfg, int device, twdic_ctx** out)
         {(void**)&c->d_rx, roi * 4}, {(void**)&c->d_ry, roi * 4},
         {(void**)&c->d_tx, roi * 4}, {(void**)&c->d_ty, roi * 4}, {(void**)&c->d_txy, roi * 4},
         {(void**)&c->d_lut, roi * 64}, {(void**)&c->d_fft_tw, sizeof(float2) * kMaxFftN},
-        {(void**)&c->d_g2, roi * 4},
+        {(void**)&c->d_g2, roi * 4}, {(void**)&c->d_lut_done, sizeof(int)},
     };
     for (auto& a : allocs) {
         if (st != TWDIC_OK) break;
@@ -475,7 +534,7 @@ twdic_status twdic_destroy(twdic_ctx* c)
     if (c->stream2) (void)hipStreamSynchronize(c->stream2);
     drop_graph(c);
     void* bufs[] = {c->d_ref, c->d_tar, c->d_rx, c->d_ry, c->d_tx, c->d_ty, c->d_txy, c->d_lut,
-                    c->d_fft_tw, c->d_refstate, c->d_g2, c->d_rp};
+                    c->d_fft_tw, c->d_refstate, c->d_g2, c->d_rp, c->d_lut_done};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
@@ -498,6 +557,8 @@ const char* twdic_last_error(const twdic_ctx* c)
 twdic_status twdic_sync(twdic_ctx* c)
 {
     if (!c) return TWDIC_EINVAL;
+    const twdic_status st = settle_lut(c);
+    if (st != TWDIC_OK) return st;
     TW_HIP(c, hipStreamSynchronize(c->stream));
     return TWDIC_OK;
 }
@@ -556,6 +617,8 @@ twdic_status twdic_precompute_target(twdic_ctx* c)
     if (!c->tar_loaded) return fail(c, TWDIC_EINVAL, "target image not set");
     twdic_status st = ensure_ref_grads(c);
     if (st != TWDIC_OK) return st;
+    st = lut_ready(c);
+    if (st != TWDIC_OK) return st;
     const twdic_config& g = c->cfg;
     TW_HIP(c, launch_gradients(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_tx, c->d_ty,
                                c->d_txy, nullptr, c->stream));
@@ -564,6 +627,7 @@ twdic_status twdic_precompute_target(twdic_ctx* c)
     else
         TW_HIP(c, launch_bicubic_lut(c->d_tar, c->dstride, g.roi_x, g.roi_y, g.roi_w, g.roi_h, c->d_lut, c->stream));
     c->tar_pre_valid = true;
+    c->lut_behind = false;
     return TWDIC_OK;
 }
 
@@ -749,16 +813,21 @@ twdic_status twdic_frame_replay(twdic_ctx* c)
         c->refstate_poi = ip.poi;
         c->refstate_n = ip.n;
     }
-    // a graph captured before the LUT was handed out builds the rows or planes:
-    // the LUT is kept up beside it
+    // a graph captured before the LUT was in use builds the rows or planes: the
+    // LUT is kept up beside it
     const bool plane = ip.rp != nullptr;
-    if (plane && c->cfg.interp != TWDIC_INTERP_FUSED && c->lut_exposed) {
+    if (plane && c->lut_exposed) {
+        const twdic_status st = settle_lut(c);
+        if (st != TWDIC_OK) return st;
         TW_HIP(c, launch_target_interp(c, c->stream));
         c->tar_pre_valid = true;
     }
     TW_HIP(c, hipGraphLaunch(c->graph_exec, c->stream));
-    // the graph rebuilt the LUT, or the rows or planes
-    (c->cfg.interp == TWDIC_INTERP_FUSED || plane ? c->tar_rp_valid : c->tar_pre_valid) = true;
+    // the graph rebuilt the rows or planes, or the LUT
+    if (plane && !c->lut_exposed)
+        plane_built(c);
+    else
+        (c->cfg.interp == TWDIC_INTERP_FUSED ? c->tar_rp_valid : c->tar_pre_valid) = true;
     return TWDIC_OK;
 }
 
@@ -780,13 +849,9 @@ twdic_status twdic_get_buffer(twdic_ctx* c, int which, void** d_ptr, size_t* byt
     case TWDIC_BUF_TAR: p = c->d_tar; b = img; c->tar_exposed = true; break;
     default: return fail(c, TWDIC_EINVAL, "unknown buffer");
     }
-    if (which == TWDIC_BUF_LUT && c->cfg.interp != TWDIC_INTERP_FUSED && !c->lut_exposed) {
-        c->lut_exposed = true;
-        // the LUT of the target IC-GN last ran on, if that is still the current one
-        if (c->tar_rp_valid && !c->tar_pre_valid) {
-            TW_HIP(c, launch_target_interp(c, c->stream));
-            c->tar_pre_valid = true;
-        }
+    if (which == TWDIC_BUF_LUT) {
+        const twdic_status st = use_lut(c);
+        if (st != TWDIC_OK) return st;
     }
     if (which == TWDIC_BUF_RX || which == TWDIC_BUF_RY) {
         twdic_status st = ensure_ref_grads(c);
@@ -904,6 +969,8 @@ twdic_status twdic_memcpy(twdic_ctx* c, void* dst, const void* src, size_t bytes
     hipMemcpyKind k = kind == 0 ? hipMemcpyHostToDevice : kind == 1 ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
     if (kind < 0 || kind > 2) return fail(c, TWDIC_EINVAL, "memcpy kind");
     TW_SPANS(c, "twdic_memcpy", {kind != 1 ? dst : nullptr, bytes, "dst"}, {kind != 0 ? src : nullptr, bytes, "src"});
+    const twdic_status st = settle_lut(c);
+    if (st != TWDIC_OK) return st;
     hipError_t small;
     if (kind == 1 && download_small(c, dst, src, bytes, &small)) {
         TW_HIP(c, small);

@@ -257,6 +257,10 @@ hipError_t launch_gradients(const uint8_t* img, int stride, int sx0, int sy0, in
                             float* gx, float* gy, float* gxy, uint32_t* g2, hipStream_t st);
 hipError_t launch_bspline_lut(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float* lut,
                               hipStream_t st);
+// the LUT as its own kernels write it, from the row polynomials, or from the
+// B-spline planes, bit for bit; nothing once *done is set, which it then is
+hipError_t launch_lut_of_rows(const float4* rp, int rw, int rh, float* lut, int* done, hipStream_t st);
+hipError_t launch_lut_of_planes(const float4* planes, int rw, int rh, float* lut, int* done, hipStream_t st);
 // the same coefficients as planes, float4[4][rh][rw]
 hipError_t launch_bspline_planes(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* planes,
                                  hipStream_t st);
@@ -351,7 +355,11 @@ struct twdic_ctx {
     bool tar_pre_valid = false;       // Tx/Ty/Txy/LUT match d_tar
     bool tar_rp_valid = false;        // d_rp matches d_tar
     bool tar_exposed = false;         // d_tar was handed out: it may change without twdic_set_target
-    bool lut_exposed = false;         // d_lut was handed out: the LUT modes keep it up and read it
+    bool lut_exposed = false;         // the LUT modes keep d_lut up and read it: it was handed out, or the
+                                      // caller captured a call into a graph of its own
+    bool lut_behind = false;          // d_rp holds the table of a later build than d_lut's
+    bool lut_pending = false;         // d_lut is still to be made from d_rp, unless *d_lut_done
+    int* d_lut_done = nullptr;
     uint64_t ref_version = 0;
     // per-reference POI state cache key
     double* d_refstate = nullptr;
