@@ -247,8 +247,8 @@ __device__ __forceinline__ TargetBuf target_buf(const IcgnParams& P)
 {
     const int stride = P.stride;
     const uint8_t* base = P.tar - stride - 1;
-    const int records = (P.sy0 + P.rh + 3) * stride;
-    return {__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, records, 0x00020000), stride};
+    const uint32_t records = target_records(P.sy0, P.rh, stride);
+    return {__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)records, 0x00020000), stride};
 }
 
 __device__ __forceinline__ int target_offset(const TargetBuf& B, int ix, int iy)
@@ -513,7 +513,6 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     constexpr bool ROWS = RP && INTERP != TWDIC_INTERP_BSPLINE;      // the target's rows as polynomials
     constexpr bool ROLL = KEEP && ROWS && !INT && !CHECK && !K32;
     constexpr bool GROUP = ROWS && INT && !CHECK && !K32;
-    constexpr int kNoPixel = 0x7fffffff;          // past every image (target_buf: records fit an int)
     const int sx0 = P.sx0, sy0 = P.sy0, rw = P.rw, rh = P.rh;
     const TargetBuf tb = target_buf(P);
     const __amdgpu_buffer_rsrc_t g2r =
@@ -712,7 +711,7 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                         float wx, wy;
                         warp(cx, cy, dy + (float)i, wx, wy);
                         int o = target_offset(tb, (int)wx, (int)wy);
-                        if (MASK) o = r + i < rows ? o : kNoPixel;
+                        if (MASK) o = r + i < rows ? o : (int)kNoOffset;
                         t[i] = __builtin_amdgcn_raw_buffer_load_b8(tb.r, o, tb.stride + 1, 0);      // :629
                         g[i] = gradient(go, so + 4 * rw * i);
                     }

@@ -248,6 +248,18 @@ __device__ __forceinline__ ConstPairDescPtr const_pairs(const PairDesc* p)
     return (ConstPairDescPtr)p;
 }
 
+// The bytes that IC-GN's target loads may reach, from the pixel (-1, -1) on: the
+// rows of the ROI and what its last cells' neighbourhoods add, at most the
+// image's 2^31 bytes and three rows of 65,535 more, which an int need not hold.
+__host__ __device__ inline uint32_t target_records(int sy0, int rh, int stride)
+{
+    return (uint32_t)(sy0 + rh + 3) * (uint32_t)stride;
+}
+
+// A byte offset past every such range, also with a row of a scalar offset added:
+// a load there returns zero.
+constexpr uint32_t kNoOffset = 0xC0000000u;
+
 // Kernel launch wrappers (return hipError_t of the launch).
 // `bytes` (at most kDownBytes) from device memory to the pinned buffer `out`,
 // then seq into *flag.
