@@ -1468,7 +1468,8 @@ __device__ __forceinline__ bool fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int 
                 }
             }
         // the T rows again from byte N on (up to byte 2 N - 1 they are read),
-        // over the zeros of the last piece
+        // over the zeros of the last piece, which another lane has stored
+        if constexpr (!FULL) wave_lds_sync();
 #pragma unroll
         for (int k = 0; k < Rows::LOADS; ++k)
             if (Rows::active(k, lane, N)) {
