@@ -283,7 +283,7 @@ __device__ __forceinline__ RowPolyBuf row_poly_buf(const IcgnParams& P)
 {
     const uint32_t lead = 16u * ((uint32_t)P.sy0 * (uint32_t)P.rw + (uint32_t)P.sx0);
     const uint8_t* base = reinterpret_cast<const uint8_t*>(P.rp) - lead;
-    const int records = (int)(lead + 16u * (uint32_t)(P.rh + 2) * (uint32_t)P.rw);
+    const int records = (int)(lead + 16u * (uint32_t)(P.rh + 1) * (uint32_t)P.rw);
     return {__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, records, 0x00020000), 16 * P.rw};
 }
 
@@ -295,10 +295,10 @@ __device__ __forceinline__ int row_poly_offset(const RowPolyBuf& B, int ix, int 
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
-// the row polynomial at byte offset o, `rows` rows further down
-__device__ __forceinline__ h4 load_row_poly(const RowPolyBuf& B, int o, int rows)
+// the second row polynomial of the entry at byte offset o, `rows` rows further down
+__device__ __forceinline__ h4 load_lower_row(const RowPolyBuf& B, int o, int rows)
 {
-    return __builtin_bit_cast(h4, __builtin_amdgcn_raw_buffer_load_b64(B.r, o, rows * B.pitch, 0));
+    return __builtin_bit_cast(h4, __builtin_amdgcn_raw_buffer_load_b64(B.r, o + 8, rows * B.pitch, 0));
 }
 
 // the row polynomials there and one row below it
@@ -664,10 +664,10 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                     float T;
                     if constexpr (INTERP == TWDIC_INTERP_LUT) {
                         T = lut_cubic(q[K], q[(K + 1) & 3], q[(K + 2) & 3], q[(K + 3) & 3], tx, ty);
-                        fresh = load_row_poly(rb, o, 4);
+                        fresh = load_lower_row(rb, o, 3);
                     } else {
                         const float R0 = row_poly(q[K], tx);
-                        fresh = load_row_poly(rb, o, 4);
+                        fresh = load_lower_row(rb, o, 3);
                         T = column_cubic(R0, row_poly(q[(K + 1) & 3], tx), row_poly(q[(K + 2) & 3], tx),
                                          row_poly(q[(K + 3) & 3], tx), ty);
                     }

@@ -240,9 +240,8 @@ hipError_t launch_bicubic_lut(const uint8_t* tar, int stride, int sx0, int sy0, 
 // integers of magnitude at most 1530.  Stored as c0, c1/2, c2/2, c3/2 in fp16
 // (exactly), the cubic is c0 + t (c1/2 + t (c2/2 + t c3/2)).  Entry (x, j) holds
 // the coefficients (8 bytes each) of rows y = sy0 - 1 + j and y + 1 for cell column
-// sx0 + x, x < rw, j <= rh + 1; the last column (never an interior cell) is
-// zero.  A cell's four neighbourhood rows are the entries (x, j) and (x, j + 2),
-// and a single row the first half of its entry.
+// sx0 + x, x < rw, j <= rh; the last column (never an interior cell) is
+// zero.  A cell's four neighbourhood rows are the entries (x, j) and (x, j + 2).
 // ---------------------------------------------------------------------------
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
@@ -282,13 +281,13 @@ __global__ __launch_bounds__(256) void k_row_poly(const uint8_t* __restrict__ ta
     const __amdgpu_buffer_rsrc_t img = row_poly_src(tar, stride, sy0, rh);
     const int x = blockIdx.x * 256 + threadIdx.x;
     if (x >= rw) return;
-    for (int j = blockIdx.y; j <= rh + 1; j += gridDim.y) row_poly_entry(img, stride, sx0, sy0, rw, x, j, rp);
+    for (int j = blockIdx.y; j <= rh; j += gridDim.y) row_poly_entry(img, stride, sx0, sy0, rw, x, j, rp);
 }
 
 hipError_t launch_row_poly(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* rp,
                            hipStream_t st)
 {
-    const dim3 grid((rw + 255) / 256, std::min(rh + 2, 65535));
+    const dim3 grid((rw + 255) / 256, std::min(rh + 1, 65535));
     hipLaunchKernelGGL(k_row_poly, grid, dim3(256), 0, st, tar, stride, sx0, sy0, rw, rh, rp);
     return hipGetLastError();
 }
@@ -302,7 +301,7 @@ __global__ __launch_bounds__(256) void k_batch_row_poly(const PairDesc* __restri
     const IcgnParams P = const_pairs(pairs)[blockIdx.y].icgn;
     if (P.rp == nullptr) return;
     const __amdgpu_buffer_rsrc_t img = row_poly_src(P.tar, P.stride, P.sy0, P.rh);
-    for (int j = blockIdx.x; j <= P.rh + 1; j += gridDim.x)
+    for (int j = blockIdx.x; j <= P.rh; j += gridDim.x)
         for (int x = threadIdx.x; x < P.rw; x += 256)
             row_poly_entry(img, P.stride, P.sx0, P.sy0, P.rw, x, j, const_cast<float4*>(P.rp));
 }
@@ -310,7 +309,7 @@ __global__ __launch_bounds__(256) void k_batch_row_poly(const PairDesc* __restri
 hipError_t launch_batch_row_poly(const PairDesc* pairs, int npairs, int max_rh, hipStream_t st)
 {
     if (npairs <= 0) return hipSuccess;
-    const int blocks = std::max(1, std::min(max_rh + 2, 1024));
+    const int blocks = std::max(1, std::min(max_rh + 1, 1024));
     hipLaunchKernelGGL(k_batch_row_poly, dim3(blocks, npairs), dim3(256), 0, st, pairs);
     return hipGetLastError();
 }

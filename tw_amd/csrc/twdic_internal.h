@@ -169,7 +169,7 @@ struct IcgnParams {
     double delta_p;           // the caller's float, widened: the loop test compares in FP64
     const uint32_t* g2;       // reference gradients (2Rx, 2Ry) as int16 pairs, ROI-relative
     const float* lut;         // target LUT [rh][rw][16]
-    const float4* rp;         // target row polynomials [rh + 2][rw] (fused, LUT modes) or B-spline planes
+    const float4* rp;         // target row polynomials [rh + 1][rw] (fused, LUT modes) or B-spline planes
                               // [4][rh][rw]; null: from the image bytes or the LUT
     double* refstate;         // kRefStateStride doubles per POI
     const int32_t* poi;
@@ -276,7 +276,7 @@ hipError_t launch_lut_of_planes(const float4* planes, int rw, int rh, float* lut
 // the same coefficients as planes, float4[4][rh][rw]
 hipError_t launch_bspline_planes(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* planes,
                                  hipStream_t st);
-// Catmull-Rom row polynomials of the target, (rh + 2) x rw entries of 16 bytes
+// Catmull-Rom row polynomials of the target, (rh + 1) x rw entries of 16 bytes
 hipError_t launch_row_poly(const uint8_t* tar, int stride, int sx0, int sy0, int rw, int rh, float4* rp,
                            hipStream_t st);
 // the same for every pair of a batch with a plane (descriptor icgn.rp set);
@@ -311,7 +311,7 @@ inline bool row_poly_fits(int sx0, int sy0, int rw, int rh)
 }
 inline size_t row_poly_bytes(int rw, int rh)
 {
-    return 16ull * (size_t)rw * (size_t)(rh + 2);
+    return 16ull * (size_t)rw * (size_t)(rh + 1);
 }
 // waves: occupancy target 5 or 6; xcd_ranges: contiguous per-XCD item ranges;
 // all_rp: every pair's descriptor has its row-polynomial plane
