@@ -291,7 +291,7 @@ bool stream_capturing(const twdic_ctx* c)
 // table that IC-GN runs on.
 void plane_built(twdic_ctx* c)
 {
-    c->tar_rp_valid = true;
+    c->tar_rp_valid = c->rp_built = true;
     c->lut_behind = c->cfg.interp != TWDIC_INTERP_FUSED;
 }
 
@@ -321,6 +321,11 @@ twdic_status use_lut(twdic_ctx* c)
         c->lut_exposed = true;
         c->lut_pending = c->lut_behind;
         c->tar_pre_valid = c->tar_pre_valid || c->tar_rp_valid;
+        // never built: nothing reads it, and no graph will
+        if (c->d_rp && !c->rp_built && !stream_capturing(c)) {
+            TW_HIP(c, hipFree(c->d_rp));
+            c->d_rp = nullptr;
+        }
     }
     return settle_lut(c);
 }
@@ -487,11 +492,19 @@ twdic_status twdic_create(const twdic_config* cfg, int device, twdic_ctx** out)
     }
     // fused and LUT modes: the target's row polynomials (16 bytes per ROI pixel);
     // without them (ROIs past 2^28 pixels) IC-GN reads the image bytes or the LUT.
-    // B-spline mode: the coefficient planes (64 bytes per ROI pixel).
+    // B-spline mode: the coefficient planes (64 bytes per ROI pixel).  Beside a
+    // LUT they are only the faster layout: memory that holds the LUT but not them
+    // is no error.
     const size_t rp = cfg->interp == TWDIC_INTERP_BSPLINE ? roi * 64
                       : row_poly_fits(cfg->roi_x, cfg->roi_y, cfg->roi_w, cfg->roi_h)
                           ? row_poly_bytes(cfg->roi_w, cfg->roi_h) : 0;
-    if (st == TWDIC_OK && rp && (e = hipMalloc((void**)&c->d_rp, rp)) != hipSuccess) bail(e, "hipMalloc");
+    if (st == TWDIC_OK && rp && (e = hipMalloc((void**)&c->d_rp, rp)) != hipSuccess) {
+        c->d_rp = nullptr;
+        if (cfg->interp == TWDIC_INTERP_FUSED)
+            bail(e, "hipMalloc");
+        else
+            (void)hipGetLastError();
+    }
     for (int i = 0; i < 16 && st == TWDIC_OK; ++i)
         if ((e = hipEventCreate(&c->ev[i])) != hipSuccess) bail(e, "hipEventCreate");
     for (int i = 0; i <= twdic_ctx::kMaxFrameChunks && st == TWDIC_OK; ++i)

@@ -359,13 +359,14 @@ struct twdic_ctx {
     float* d_ty = nullptr;
     float* d_txy = nullptr;
     float* d_lut = nullptr;
-    float4* d_rp = nullptr;           // target row polynomials (fused interpolation)
+    float4* d_rp = nullptr;           // target row polynomials or B-spline planes (null: not kept)
     uint32_t* d_g2 = nullptr;         // packed (2Rx, 2Ry) int16 pairs
     float2* d_fft_tw = nullptr;
     bool ref_loaded = false, tar_loaded = false;
     bool ref_grads_valid = false;     // Rx/Ry match d_ref
     bool tar_pre_valid = false;       // Tx/Ty/Txy/LUT match d_tar
     bool tar_rp_valid = false;        // d_rp matches d_tar
+    bool rp_built = false;            // d_rp was built at some time
     bool tar_exposed = false;         // d_tar was handed out: it may change without twdic_set_target
     bool lut_exposed = false;         // the LUT modes keep d_lut up and read it: it was handed out, or the
                                       // caller captured a call into a graph of its own
