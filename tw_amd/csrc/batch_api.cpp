@@ -61,8 +61,9 @@ struct twdic_batch {
     int lanes = 4;                    // TWDIC_BATCH_STREAMS (1..4)
     // flat form: one launch per stage and kernel form over all pairs
     bool flat = true;                 // TWDIC_BATCH_FORM=direct selects the direct form
-    struct WindowItems {              // FFT-CC items (pair, POI) of the pairs with window edge N
+    struct WindowItems {              // FFT-CC items (pair, POI) of one launch (launch_batch_fftcc_mma)
         int N;
+        bool dft;
         int2* d;
         int64_t n;
     };
@@ -265,13 +266,13 @@ twdic_status run_direct(twdic_batch* b, bool fftcc, bool icgn)
     return TWDIC_OK;
 }
 
-// Flat form: FFT-CC per window edge, then IC-GN per lane
+// Flat form: FFT-CC per engine and window edge or kernel, then IC-GN per lane
 // count, each one launch over the items of every pair on the batch stream.  The
 // same per-POI device code as the single-context kernels.
 twdic_status enqueue_flat(twdic_batch* b, bool fftcc, bool icgn)
 {
     if (fftcc)
-        for (const auto& m : b->mitems) TB_HIP(b, launch_batch_fftcc_mma(b->d_desc, m.d, (int)m.n, m.N, b->stream));
+        for (const auto& m : b->mitems) TB_HIP(b, launch_batch_fftcc_mma(b->d_desc, m.d, (int)m.n, m.N, m.dft, b->stream));
     if (icgn) TB_HIP(b, launch_batch_row_poly(b->d_desc, (int)b->pairs.size(), b->max_rh, b->stream));
     if (icgn)
         for (int t = 0; t < 2; ++t)
@@ -411,22 +412,33 @@ twdic_status set_pairs_impl(twdic_batch* b, const twdic_pair* pairs, int npairs)
         }
     }
     if (total) TB_HIP(b, hipMemcpy(b->d_items, items.data(), sizeof(int2) * total, hipMemcpyHostToDevice));
-    // flat form: FFT-CC items per window edge, IC-GN items of 256 / lanes POIs of one pair
-    std::map<int, std::vector<int2>> mitems;
+    // flat form: FFT-CC items per launch, IC-GN items of 256 / lanes POIs of one pair
+    std::map<int, int64_t> edge_pois;                     // POIs per window edge
+    for (const auto& p : b->pairs) edge_pois[p.fft_n] += p.n;
+    auto dft_edge = [&](int N, bool beside) {
+        const int n = (int)std::min<int64_t>(edge_pois[N], INT32_MAX);
+        return beside ? dft_takes_beside(N, n) : dft_takes(N, n);
+    };
+    std::map<int, int> rest;                              // edges per integer kernel that do not leave it for the DFT engine
+    for (const auto& [N, n] : edge_pois)
+        if (n > 0 && !dft_edge(N, true)) ++rest[mma_form(N)];
+    std::map<std::pair<bool, int>, std::vector<int2>> mitems;
     std::vector<int2> wg[2];
     for (int i = 0; i < npairs; ++i) {
         const twdic_pair& p = b->pairs[i];
-        auto& mi = mitems[p.fft_n];
+        // an edge that would have its integer kernel to itself is as in a single context
+        const bool dft = dft_edge(p.fft_n, true) || (rest[mma_form(p.fft_n)] == 1 && dft_edge(p.fft_n, false));
+        auto& mi = mitems[{dft, dft ? p.fft_n : mma_form(p.fft_n)}];
         for (int k = 0; k < p.n; ++k) mi.push_back(make_int2(i, k));
         const int lanes = icgn_lanes_for(p.n), per_wg = 256 / lanes;
         auto& w = wg[lanes == 64 ? 1 : 0];
         for (int k = 0; k < p.n; k += per_wg) w.push_back(make_int2(i, k));
     }
-    for (const auto& [N, list] : mitems) {
+    for (const auto& [key, list] : mitems) {
         if (list.empty()) continue;
         if (list.size() > (size_t)INT32_MAX)
-            return bfail(b, TWDIC_EINVAL, "more than 2^31 - 1 POIs in one FFT-CC window edge");
-        b->mitems.push_back({N, nullptr, (int64_t)list.size()});
+            return bfail(b, TWDIC_EINVAL, "more than 2^31 - 1 POIs in one FFT-CC launch");
+        b->mitems.push_back({key.second, key.first, nullptr, (int64_t)list.size()});
         int2*& d = b->mitems.back().d;
         TB_HIP(b, alloc((void**)&d, sizeof(int2) * list.size()));
         TB_HIP(b, hipMemcpy(d, list.data(), sizeof(int2) * list.size(), hipMemcpyHostToDevice));

@@ -1193,22 +1193,6 @@ constexpr double kDftBound = 22.0;        // N^2 |C^ - C| / (||r|| ||t||) at N =
 // the same over N^2 / 4096 for every even 32 < N <= 60 (largest at N = 54: 25.9)
 constexpr double kDftBoundN = 26.0;
 
-// The POI sets the engine takes (both engines give the same results): N = 64,
-// the even 48 < N <= 60, and 32 < N <= 48 from the count on at which it is the
-// faster one: it starts with its tables, 3 us more than the integer engine for
-// one POI.  (N = 62 leaves the spectrum no free row, see fftcc_dft_mfma_poi.)
-// Against the integer engine, 2048^2 speckle, ms:
-//   N       34         40         48         50         56         60
-//   25      .013/.011  .014/.012  .015/.013  .015/.016  .015/.017  .015/.018
-//   800     .016/.012  .016/.013  .016/.015  .016/.018  .016/.020  .016/.021
-//   1,200   .016/.014  .016/.016  .016/.019  .016/.024  .017/.026  .016/.027
-//   5,000   .025/.034  .023/.038  .025/.044  .03 /.065  .031/.072  .03 /.076
-//   155k    .47 /.69   .48 /.82   .51 /1.00  .69 /1.61  .71 /1.86  .72 /1.96
-inline bool dft_takes(int N, int n)
-{
-    return N == 64 || (N > 48 && N <= 60) || (N > 32 && N <= 48 && n >= 1280);
-}
-
 // F in fp16 as MFMA operands, [table][part][tile][K chunk][lane], lane = 32 h + m,
 // parts re, im, -im:
 //   table 0: F[16 c + 8 h + q][32 t + m]                 (B operand, K in natural order);
@@ -1933,14 +1917,15 @@ void launch_batch_dft(const PairDesc* pairs, const int2* items, int count, hipSt
 
 }  // namespace
 
-hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int N, hipStream_t st)
+hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int N, bool dft,
+                                  hipStream_t st)
 {
     if (count <= 0) return hipSuccess;
-    if (N == 64)
+    if (dft && N == 64)
         launch_batch_dft<4, true>(pairs, items, count, st);
-    else if (dft_takes(N, count) && N > 48)
+    else if (dft && N > 48)
         launch_batch_dft<4, false>(pairs, items, count, st);
-    else if (dft_takes(N, count))
+    else if (dft)
         launch_batch_dft<3, false>(pairs, items, count, st);
     else if (N > 48)
         hipLaunchKernelGGL((k_batch_fftcc_mma<64, false, 32>), dim3(count), dim3(64), 0, st, pairs, items);
@@ -1951,8 +1936,6 @@ hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int 
     return hipGetLastError();
 }
 
-// variant: occupancy target of the register engine (waves per SIMD the
-// compiler budgets registers for): 2 (no spills), 3 or 4.
 hipError_t launch_fftcc(const FftccParams& p, int variant, hipStream_t st)
 {
     if (p.n <= 0) return hipSuccess;

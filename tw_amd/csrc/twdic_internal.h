@@ -296,9 +296,39 @@ constexpr int kFftccMma = 8;
 constexpr int kFftccDftMfma = 9;
 hipError_t dft_tables_init(int device);
 hipError_t launch_fftcc(const FftccParams& p, int variant, hipStream_t st);
-// batched form: the matrix-core kernels over items (pair, POI) of pairs that
-// share the window edge N
-hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int N, hipStream_t st);
+// The POI sets the matrix-core DFT engine takes in place of the integer one (both
+// give the same results): N = 64,
+// the even 48 < N <= 60, and 32 < N <= 48 from the count on at which it is the
+// faster one: it starts with its tables, 3 us more than the integer engine for
+// one POI.  (N = 62 leaves the spectrum no free row, fftcc_dft_mfma_poi.)
+// Against the integer engine, 2048^2 speckle, ms:
+//   N       34         40         48         50         56         60
+//   25      .013/.011  .014/.012  .015/.013  .015/.016  .015/.017  .015/.018
+//   800     .016/.012  .016/.013  .016/.015  .016/.018  .016/.020  .016/.021
+//   1,200   .016/.014  .016/.016  .016/.019  .016/.024  .017/.026  .016/.027
+//   5,000   .025/.034  .023/.038  .025/.044  .03 /.065  .031/.072  .03 /.076
+//   155k    .47 /.69   .48 /.82   .51 /1.00  .69 /1.61  .71 /1.86  .72 /1.96
+inline bool dft_takes(int N, int n)
+{
+    return N == 64 || (N > 48 && N <= 60) || (N > 32 && N <= 48 && n >= 1280);
+}
+
+// In a flat batch the window edges of one integer kernel (mma_form) share its
+// launch, while the DFT engine needs a launch per edge, 14 us before its first
+// POIs are through.  Beside other edges it is therefore taken from higher counts
+// on.  Batches of one pair per edge with their IC-GN, us, launches of their own /
+// one together:
+//   POIs per pair   900       1,296     1,764     3,721     7,056
+//   50 .. 60        194/173   219/224   231/272   372/483   600/859
+//   34 .. 48                            298/257   433/447   707/783
+inline bool dft_takes_beside(int N, int n) { return dft_takes(N, n) && (N == 64 || n >= (N > 48 ? 1200 : 3200)); }
+// the integer kernel of a window edge, by the largest edge it serves
+inline int mma_form(int N) { return N <= 32 ? 32 : N <= 48 ? 48 : 64; }
+
+// batched form: the matrix-core kernels over items (pair, POI): of pairs that
+// share the window edge N, by the DFT engine (dft), or whose edges have the
+// integer kernel of N
+hipError_t launch_batch_fftcc_mma(const PairDesc* pairs, const int2* items, int count, int N, bool dft, hipStream_t st);
 // batched form: IC-GN (fused interpolation) over workgroup items (pair, first
 // POI), 256 / lanes POIs of one pair per workgroup, every listed pair with
 // that many lanes per POI.
