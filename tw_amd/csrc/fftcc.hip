@@ -1171,7 +1171,7 @@ __global__ __launch_bounds__(64) void k_batch_fftcc_mma(const PairDesc* __restri
 //   maximum is evaluated exactly in integers, in increasing index order,
 //   keeping the first strict maximum: the exact argmax with the CPU path's
 //   lowest-index tie-break.  (Speckle windows leave about two such shifts; a
-//   window of pure noise a handful; the count is not capped.)
+//   window of pure noise a handful; at N = 64 the count is not capped.)
 //   A workgroup of eight wavefronts, one POI each, shares the fp16 tables in
 //   LDS; the window bytes stay in LDS for the exact stage.
 //
@@ -1403,83 +1403,247 @@ __device__ __forceinline__ h8 centred_h8(uint2 w, h2v off)
     return r;
 }
 
+// One window pair's rows (DftRows) to the wavefront's LDS: R row y at y RP, zero
+// beyond N, T row y at y TP and again N bytes on; and the exact integer sums of
+// R, T, R^2, T^2.
+template <int CH, bool FULL>
+__device__ __forceinline__ void dft_window(DftWgSmem<CH, FULL>& sm, int wave, int lane, int N,
+                                           const DftRows<CH, FULL>& rows, int (&sums)[4])
+{
+    using Sm = DftWgSmem<CH, FULL>;
+    uint8_t* ex = sm.ex[wave];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sums[i] = 0;
+    using Rows = DftRows<CH, FULL>;
+    uint32_t rw[Rows::LOADS][4], tw[Rows::LOADS][4];
+#pragma unroll
+    for (int k = 0; k < Rows::LOADS; ++k) {
+        Rows::words(rows.r[k], N, lane, rw[k]);
+        Rows::words(rows.t[k], N, lane, tw[k]);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            sums[0] = (int)__builtin_amdgcn_udot4(rw[k][w], 0x01010101u, (uint32_t)sums[0], false);
+            sums[1] = (int)__builtin_amdgcn_udot4(tw[k][w], 0x01010101u, (uint32_t)sums[1], false);
+            sums[2] = (int)__builtin_amdgcn_udot4(rw[k][w], rw[k][w], (uint32_t)sums[2], false);
+            sums[3] = (int)__builtin_amdgcn_udot4(tw[k][w], tw[k][w], (uint32_t)sums[3], false);
+        }
+    }
+    wave_lds_sync();                           // the previous POI's reads of this region are done
+    uint8_t* er = ex + (lane / CH) * Sm::RP + 16 * (lane % CH);
+    uint8_t* et = ex + Sm::ROWS * Sm::RP + (lane / CH) * Sm::TP + 16 * (lane % CH);
+#pragma unroll
+    for (int k = 0; k < Rows::LOADS; ++k)
+        if (Rows::active(k, lane, N)) {
+            uint2* e2 = reinterpret_cast<uint2*>(er + k * Rows::RL * Sm::RP);
+            uint2* t2 = reinterpret_cast<uint2*>(et + k * Rows::RL * Sm::TP);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                e2[e] = make_uint2(rw[k][2 * e], rw[k][2 * e + 1]);
+                t2[e] = make_uint2(tw[k][2 * e], tw[k][2 * e + 1]);
+            }
+        }
+    // the T rows again from byte N on (up to byte 2 N - 1 they are read),
+    // over the zeros of the last piece, which another lane has stored
+    if constexpr (!FULL) wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < Rows::LOADS; ++k)
+        if (Rows::active(k, lane, N)) {
+            uint8_t* again = et + k * Rows::RL * Sm::TP + N;
+            if constexpr (FULL) {
+                reinterpret_cast<uint2*>(again)[0] = make_uint2(tw[k][0], tw[k][1]);
+                reinterpret_cast<uint2*>(again)[1] = make_uint2(tw[k][2], tw[k][3]);
+            } else {
+                __builtin_memcpy(again, tw[k], 16);
+            }
+        }
+    dpp_sum4(sums);
+}
+
+// The rounded means a, b of R and T and ||R - a||^2, ||T - b||^2, exact below 2^31:
+// zero for a uniform window, whose rounded mean is its value, and for no other.
+struct DftNorms {
+    int a, b, r2, t2;
+    __device__ __forceinline__ DftNorms(const int (&sums)[4], int NN)
+        : a((int)((uint32_t)(sums[0] + NN / 2) / (uint32_t)NN)),
+          b((int)((uint32_t)(sums[1] + NN / 2) / (uint32_t)NN)),
+          r2(sums[2] - 2 * a * sums[0] + a * a * NN), t2(sums[3] - 2 * b * sums[1] + b * b * NN)
+    {
+    }
+    __device__ __forceinline__ bool flat() const { return r2 == 0 || t2 == 0; }       // (:271-275)
+};
+
+// Below N = 64 a window pair that leaves more than N shifts in question (it is
+// periodic, or nearly so, in both directions) has its whole integer surface formed
+// instead, in a time that does not depend on the image.  With more than N / 2 (a
+// texture that varies in one direction only gives N) the wavefront's next pairs, its
+// neighbours, go there at once: one pair, and when the DFTs then find another
+// such, 3, 7, ... kDftDirectRun.  Of 32,761 POIs at N = 40 the DFTs take 0.114 ms,
+// each candidate 0.0057 and the integer surface 0.25, i.e. 24 candidates more than
+// the DFTs and 44 alone; at N = 56 0.165, 0.0081, 0.45: 35 and 55.
+constexpr int kDftDirectRun = 31;
+
+// The exact peak of the window pair in the wavefront's LDS rows from the integer
+// surface, as k_fftcc_mma forms it (48 x 48 in 16 x 16 tiles for CH = 3, 64 x 64 in
+// 32 x 32 ones): lane (m, g) holds bytes 16 g .. 16 g + 15 of a K chunk.  The rows
+// are turned signed in place first (reference bytes from N on stay zero).  With
+// two or three wavefronts per SIMD the waits for LDS show, so both operands of a
+// row are loaded while the products of the one before run.  32,761 POIs of a
+// grating of period 4: 0.256 ms at N = 40 (all 400 candidates: 2.3; the integer
+// kernel, with more wavefronts, 0.20), 0.46 ms at N = 56 (784: 6.3; 0.36).
+template <int CH>
+__device__ __forceinline__ void mma_direct(DftWgSmem<CH, false>& sm, int wave, int lane, int N, const int (&sums)[4],
+                                           int& bestI, int& peak)
+{
+    using Sm = DftWgSmem<CH, false>;
+    constexpr int TE = CH == 3 ? 16 : 32, T = CH == 3 ? 3 : 2, KC = CH == 3 ? 1 : 2, NB = 3, REGS = TE * TE / 64;
+    typedef int acc_t __attribute__((ext_vector_type(REGS)));
+    uint8_t *rows = sm.ex[wave], *trows = rows + Sm::ROWS * Sm::RP;
+    wave_lds_sync();
+    constexpr int RQ = Sm::RP / 8, RN = Sm::ROWS * RQ, TN = Sm::ROWS * Sm::TP / 8;
+#pragma unroll
+    for (int k = 0; k < (RN + 63) / 64; ++k) {
+        const int i = 64 * k + lane, x = 8 * (i % RQ);
+        if (i < RN) {
+            uint2* q = reinterpret_cast<uint2*>(rows) + i;
+            auto flip = [&](int at) { return at + 4 <= N ? 0x80808080u : at >= N ? 0u : 0x8080u; };     // N is even
+            *q = make_uint2(q->x ^ flip(x), q->y ^ flip(x + 4));
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < (TN + 63) / 64; ++k) {
+        const int i = 64 * k + lane;
+        if (i < TN) {
+            uint2* q = reinterpret_cast<uint2*>(trows) + i;
+            *q = make_uint2(q->x ^ 0x80808080u, q->y ^ 0x80808080u);
+        }
+    }
+    wave_lds_sync();
+
+    const int m = lane % TE, g = lane / TE;
+    // bytes 48 .. 63 of a 48-byte row: the zeros of the half spectrum's unused column 31
+    const bool pad = CH == 3 && g == 3;
+    const int step = pad ? 0 : Sm::RP, wrap = N * Sm::RP, end = pad ? INT_MAX : wrap;
+    int ra[T], bd[NB], bs[NB];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const int kv = TE * t + m;       // reference row (y' - kv) mod N
+        ra[t] = pad ? (int)(reinterpret_cast<const uint8_t*>(&sm.ta[0][0][31]) - rows)
+                    : (kv > 0 && kv < N ? N - kv : 0) * Sm::RP + 16 * g;
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int o = TE * j + 16 * g + m;
+        bd[j] = o >> 2;
+        bs[j] = o & 3;
+    }
+    acc_t acc[T][T];
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int t2 = 0; t2 < T; ++t2) acc[t][t2] = acc_t{};
+    v4i A[2][KC][T];
+    uint32_t raw[NB][5];
+    auto fetch_b = [&](int y) {
+        const uint32_t* trow = reinterpret_cast<const uint32_t*>(trows + y * Sm::TP);
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int i = 0; i < 5; ++i) raw[j][i] = trow[bd[j] + i];
+    };
+    auto fetch_a = [&](v4i (&d)[KC][T]) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+#pragma unroll
+            for (int xc = 0; xc < KC; ++xc) {
+                const uint2* p = reinterpret_cast<const uint2*>(rows + ra[t] + 32 * xc);
+                const uint2 a = p[0], b = p[1];
+                d[xc][t] = v4i{(int)a.x, (int)a.y, (int)b.x, (int)b.y};
+            }
+            ra[t] += step;
+            if (ra[t] >= end) ra[t] -= wrap;
+        }
+    };
+    auto row = [&](const v4i (&cur)[KC][T], v4i (&next)[KC][T], int y) {
+        v4i B[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) B[j][i] = (int)__builtin_amdgcn_alignbyte(raw[j][i + 1], raw[j][i], bs[j]);
+        fetch_b(min(y + 1, N - 1));
+        fetch_a(next);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int xc = 0; xc < KC; ++xc)
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int t2 = 0; t2 < T; ++t2) {
+                    if constexpr (CH == 3)
+                        acc[t][t2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur[xc][t], B[xc + t2], acc[t][t2], 0, 0, 0);
+                    else
+                        acc[t][t2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur[xc][t], B[xc + t2], acc[t][t2], 0, 0, 0);
+                }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    fetch_b(0);
+    fetch_a(A[0]);
+    for (int y = 0; y < N; y += 2) {      // N is even
+        row(A[0], A[1], y);
+        row(A[1], A[0], y + 1);
+    }
+    // the largest, of equal ones the lowest place 64 kv + ku: a lane's are visited
+    // in increasing order
+    int best = INT_MIN;
+    peak = INT_MAX;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < REGS; ++r)
+#pragma unroll
+            for (int t2 = 0; t2 < T; ++t2) {
+                const int kv = TE * t + 8 * (r >> 2) + 4 * g + (r & 3), ku = TE * t2 + m, v = acc[t][t2][r];
+                // N > TE (T - 1): only the last tiles reach beyond the window
+                const bool take = (t < T - 1 || kv < N) && (t2 < T - 1 || ku < N) && v > best;
+                best = take ? v : best;
+                peak = take ? 64 * kv + ku : peak;
+            }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const int ov = __shfl_xor(best, o), ok = __shfl_xor(peak, o);
+        const bool take = ov > best || (ov == best && ok < peak);
+        best = take ? ov : best;
+        peak = take ? ok : peak;
+    }
+    bestI = best + 128 * (sums[0] + sums[1]) - 16384 * N * N;
+}
+
 // The exact peak of one window pair whose rows are in `rows`; `next` is called
 // when they and most registers are free again, to load the following pair's.
-// Returns false for a flat window, else the four window sums, the exact sum of
-// R T at the peak and the peak's place 64 a + b.
+// Gives the four window sums, the number of candidates and, but for a flat window or
+// one with too many of them (DFT_MANY), the exact sum of R T at the peak and the
+// peak's place 64 a + b.
+enum { DFT_PEAK, DFT_FLAT, DFT_MANY };
 template <int CH, bool FULL, class Next>
-__device__ __forceinline__ bool fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int wave, int lane, int N, const DftItem& it,
-                                                   DftRows<CH, FULL>& rows, int (&sums)[4], int& bestI, int& peak,
-                                                   Next next)
+__device__ __forceinline__ int fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int wave, int lane, int N,
+                                                  DftRows<CH, FULL>& rows, int (&sums)[4], int& many, int& bestI,
+                                                  int& peak, Next next)
 {
     using Sm = DftWgSmem<CH, FULL>;
     constexpr int WORDS = 4 * CH;
     if constexpr (FULL) N = 64;
     const int NN = N * N, m = lane & 31, h = lane >> 5;
-    uint8_t* ex = sm.ex[wave];
-    const uint8_t* erows = ex;                     // R row y at y RP, zero beyond N
-    const uint8_t* etrows = ex + Sm::ROWS * Sm::RP;    // T row y at y TP, and again N bytes on
-    // -- window rows to LDS, exact integer sums ---------------------------------
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sums[i] = 0;
-    {
-        using Rows = DftRows<CH, FULL>;
-        uint32_t rw[Rows::LOADS][4], tw[Rows::LOADS][4];
-#pragma unroll
-        for (int k = 0; k < Rows::LOADS; ++k) {
-            Rows::words(rows.r[k], N, lane, rw[k]);
-            Rows::words(rows.t[k], N, lane, tw[k]);
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                sums[0] = (int)__builtin_amdgcn_udot4(rw[k][w], 0x01010101u, (uint32_t)sums[0], false);
-                sums[1] = (int)__builtin_amdgcn_udot4(tw[k][w], 0x01010101u, (uint32_t)sums[1], false);
-                sums[2] = (int)__builtin_amdgcn_udot4(rw[k][w], rw[k][w], (uint32_t)sums[2], false);
-                sums[3] = (int)__builtin_amdgcn_udot4(tw[k][w], tw[k][w], (uint32_t)sums[3], false);
-            }
-        }
-        wave_lds_sync();                           // the previous POI's reads of this region are done
-        uint8_t* er = ex + (lane / CH) * Sm::RP + 16 * (lane % CH);
-        uint8_t* et = ex + Sm::ROWS * Sm::RP + (lane / CH) * Sm::TP + 16 * (lane % CH);
-#pragma unroll
-        for (int k = 0; k < Rows::LOADS; ++k)
-            if (Rows::active(k, lane, N)) {
-                uint2* e2 = reinterpret_cast<uint2*>(er + k * Rows::RL * Sm::RP);
-                uint2* t2 = reinterpret_cast<uint2*>(et + k * Rows::RL * Sm::TP);
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    e2[e] = make_uint2(rw[k][2 * e], rw[k][2 * e + 1]);
-                    t2[e] = make_uint2(tw[k][2 * e], tw[k][2 * e + 1]);
-                }
-            }
-        // the T rows again from byte N on (up to byte 2 N - 1 they are read),
-        // over the zeros of the last piece, which another lane has stored
-        if constexpr (!FULL) wave_lds_sync();
-#pragma unroll
-        for (int k = 0; k < Rows::LOADS; ++k)
-            if (Rows::active(k, lane, N)) {
-                uint8_t* again = et + k * Rows::RL * Sm::TP + N;
-                if constexpr (FULL) {
-                    reinterpret_cast<uint2*>(again)[0] = make_uint2(tw[k][0], tw[k][1]);
-                    reinterpret_cast<uint2*>(again)[1] = make_uint2(tw[k][2], tw[k][3]);
-                } else {
-                    __builtin_memcpy(again, tw[k], 16);
-                }
-            }
-    }
-    dpp_sum4(sums);
-    const int a = (int)((uint32_t)(sums[0] + NN / 2) / (uint32_t)NN);             // rounded means
-    const int b = (int)((uint32_t)(sums[1] + NN / 2) / (uint32_t)NN);
-    const h2v oa = {(_Float16)(1024 + a), (_Float16)(1024 + a)};
-    const h2v ob = {(_Float16)(1024 + b), (_Float16)(1024 + b)};
-    // ||r||^2, ||t||^2, exact below 2^31; zero for a uniform window, whose
-    // rounded mean is its value, and for no other: flat (:271-275)
-    const int nr2 = sums[2] - 2 * a * sums[0] + a * a * NN, nt2 = sums[3] - 2 * b * sums[1] + b * b * NN;
-    if (nr2 == 0 || nt2 == 0) {
+    const uint8_t* erows = sm.ex[wave];
+    const uint8_t* etrows = erows + Sm::ROWS * Sm::RP;
+    dft_window(sm, wave, lane, N, rows, sums);
+    const DftNorms norm(sums, NN);
+    if (norm.flat()) {
         next();
-        return false;
+        return DFT_FLAT;
     }
+    const h2v oa = {(_Float16)(1024 + norm.a), (_Float16)(1024 + norm.a)};
+    const h2v ob = {(_Float16)(1024 + norm.b), (_Float16)(1024 + norm.b)};
     // the tolerance's factor 1.25 over the bound dwarfs the FP32 rounding here
-    const float rho = __builtin_amdgcn_sqrtf((float)nr2) * __builtin_amdgcn_sqrtf((float)nt2);
+    const float rho = __builtin_amdgcn_sqrtf((float)norm.r2) * __builtin_amdgcn_sqrtf((float)norm.t2);
     const float s = ldexpf(1.0f, 14 - __builtin_amdgcn_frexp_expf((float)NN * rho));   // s N^2 rho in [2^13, 2^14)
     const float bound = FULL ? (float)kDftBound : (float)(kDftBoundN / 4096.0) * (float)NN;
     const float tol = 2.5f / 65536.f * bound * rho * s;                          // in C^ units (s 2^-16 N^2 C)
@@ -1664,6 +1828,10 @@ __device__ __forceinline__ bool fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int 
     uint64_t mask = ((uint64_t)mw[1] << 32) | mw[0];
 
     next();
+    if constexpr (!FULL) {
+        many = dpp_sum(__popcll(mask));
+        if (many > N) return DFT_MANY;
+    }
 
     // -- exact integer correlation at the candidates: the largest, of equal ones
     //    the lowest index ------------------------------------------------------
@@ -1686,21 +1854,23 @@ __device__ __forceinline__ bool fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int 
         else
             ty = lane >= N ? 0 : ty >= N ? ty - N : ty;
         const uint32_t* trow = reinterpret_cast<const uint32_t*>(etrows + ty * Sm::TP);
-        uint32_t acc = 0;
-        uint32_t w0 = trow[d];
+        // all words first: read and used one by one, each waits for LDS
+        uint32_t acc = 0, tw[WORDS + 1], rw[WORDS];
 #pragma unroll
-        for (int j = 0; j < WORDS; ++j) {
-            const uint32_t w1 = trow[d + j + 1];
-            acc = __builtin_amdgcn_udot4(rrow[j], __builtin_amdgcn_alignbyte(w1, w0, sh), acc, false);
-            w0 = w1;
-        }
+        for (int j = 0; j <= WORDS; ++j) tw[j] = trow[d + j];
+#pragma unroll
+        for (int j = 0; j < WORDS; ++j) rw[j] = rrow[j];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < WORDS; ++j)
+            acc = __builtin_amdgcn_udot4(rw[j], __builtin_amdgcn_alignbyte(tw[j + 1], tw[j], sh), acc, false);
         const int I = dpp_sum(FULL || lane < N ? (int)acc : 0);
         if (I > bestI || (I == bestI && k < peak)) {
             bestI = I;
             peak = k;
         }
     }
-    return true;
+    return DFT_PEAK;
 }
 
 // A workgroup's wavefronts share the DFT tables in LDS; workgroup b takes the
@@ -1807,39 +1977,75 @@ __device__ __forceinline__ void fftcc_dft_run(DftWgSmem<CH, FULL>& sm, const Sou
         const FftccParams p = src.params(i);
         if (lane == 0 && p.status) p.status[src.poi(i)] = (uint8_t)status;
     };
-    int i = lo + wave;
-    if (i >= hi) return;
-    DftRows<CH, FULL> rows;
-    DftItem cur = src.item(i);
-    rows.drop();
-    if (cur.inside) rows.load(cur, N, lane);
-    for (;;) {
-        const int ni = i + Sm::WAVES;
-        DftItem nx = cur;
-        if (ni < hi) nx = src.item(ni);
-        auto next = [&]() {
-            rows.drop();
-            if (ni < hi && nx.inside) rows.load(nx, N, lane);
-        };
-        if (cur.inside) {
-            int sums[4], I, peak;
-            if (fftcc_dft_mfma_poi<CH, FULL>(sm, wave, lane, N, cur, rows, sums, I, peak, next)) {
-                if (lane == 0) {
-                    const int v[7] = {i, sums[0], sums[1], sums[2], sums[3], I, peak};
+    auto keep = [&](int i, const int (&sums)[4], int I, int peak) {
+        if (lane == 0) {
+            const int v[7] = {i, sums[0], sums[1], sums[2], sums[3], I, peak};
 #pragma unroll
-                    for (int f = 0; f < 7; ++f) kept[f][nkept] = v[f];
-                }
-                if (++nkept == Sm::KEPT) flush();
-            } else {
-                fail(i, TWDIC_FFTCC_FLAT);
-            }
-        } else {
-            next();
-            fail(i, TWDIC_FFTCC_OUT);
+            for (int f = 0; f < 7; ++f) kept[f][nkept] = v[f];
         }
-        if (ni >= hi) break;
-        i = ni;
-        cur = nx;
+        if (++nkept == Sm::KEPT) flush();
+    };
+    int i = lo + wave, run = 0;
+    while (i < hi) {
+        DftRows<CH, FULL> rows;
+        DftItem cur = src.item(i);
+        rows.drop();
+        if (cur.inside) rows.load(cur, N, lane);
+        int direct = 0;                       // items from i on that are mma_direct's
+        for (;;) {
+            const int ni = i + Sm::WAVES;
+            DftItem nx = cur;
+            if (ni < hi) nx = src.item(ni);
+            auto next = [&]() {
+                rows.drop();
+                if (ni < hi && nx.inside) rows.load(nx, N, lane);
+            };
+            if (cur.inside) {
+                int sums[4], many = 0, I, peak;
+                const int r = fftcc_dft_mfma_poi<CH, FULL>(sm, wave, lane, N, rows, sums, many, I, peak, next);
+                if (r == DFT_PEAK)
+                    keep(i, sums, I, peak);
+                else if (r == DFT_FLAT)
+                    fail(i, TWDIC_FFTCC_FLAT);
+                if constexpr (!FULL) {
+                    if (2 * many > N) {
+                        run = min(2 * run + 1, kDftDirectRun);
+                        direct = run + (r == DFT_MANY ? 1 : 0);
+                        if (r != DFT_MANY) i = ni;
+                        break;
+                    }
+                    run = 0;
+                }
+            } else {
+                next();
+                fail(i, TWDIC_FFTCC_OUT);
+            }
+            i = ni;
+            if (i >= hi) break;
+            cur = nx;
+        }
+        if constexpr (!FULL) {
+            // in a loop of its own, whose registers the one above does not give up
+            for (; direct > 0 && i < hi; --direct, i += Sm::WAVES) {
+                int l = lane;
+                asm volatile("" : "+v"(l));      // (as that would: nothing that follows from the lane is kept)
+                const DftItem it = src.item(i);
+                if (!it.inside) {
+                    fail(i, TWDIC_FFTCC_OUT);
+                    continue;
+                }
+                rows.drop();
+                rows.load(it, N, l);
+                int sums[4], I, peak;
+                dft_window(sm, wave, l, N, rows, sums);
+                if (DftNorms(sums, N * N).flat()) {
+                    fail(i, TWDIC_FFTCC_FLAT);
+                } else {
+                    mma_direct<CH>(sm, wave, l, N, sums, I, peak);
+                    keep(i, sums, I, peak);
+                }
+            }
+        }
     }
     flush();
 }
