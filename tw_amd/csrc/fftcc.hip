@@ -1473,11 +1473,11 @@ struct DftNorms {
 };
 
 // Below N = 64 a window pair that leaves more than N shifts in question (it is
-// periodic, or nearly so, in both directions) has its whole integer surface formed
-// instead, in a time that does not depend on the image.  With more than N / 2 (a
-// texture that varies in one direction only gives N) the wavefront's next pairs, its
-// neighbours, go there at once: one pair, and when the DFTs then find another
-// such, 3, 7, ... kDftDirectRun.  Of 32,761 POIs at N = 40 the DFTs take 0.114 ms,
+// periodic, or nearly so) has its whole integer surface formed instead, in a time
+// that does not depend on the image, and so have the wavefront's next
+// kDftDirectRun pairs, its neighbours.  After one with more than N / 2 (a texture
+// that varies in one direction only gives N) the next pair goes there at once, and
+// when the DFTs then find another such, the next 3, 7, ... kDftDirectRun.  Of 32,761 POIs at N = 40 the DFTs take 0.114 ms,
 // each candidate 0.0057 and the integer surface 0.25, i.e. 24 candidates more than
 // the DFTs and 44 alone; at N = 56 0.165, 0.0081, 0.45: 35 and 55.
 constexpr int kDftDirectRun = 31;
@@ -1488,7 +1488,7 @@ constexpr int kDftDirectRun = 31;
 // are turned signed in place first (reference bytes from N on stay zero).  With
 // two or three wavefronts per SIMD the waits for LDS show, so both operands of a
 // row are loaded while the products of the one before run.  32,761 POIs of a
-// grating of period 4: 0.256 ms at N = 40 (all 400 candidates: 2.3; the integer
+// grating of period 4: 0.260 ms at N = 40 (all 400 candidates: 2.3; the integer
 // kernel, with more wavefronts, 0.20), 0.46 ms at N = 56 (784: 6.3; 0.36).
 template <int CH>
 __device__ __forceinline__ void mma_direct(DftWgSmem<CH, false>& sm, int wave, int lane, int N, const int (&sums)[4],
@@ -1619,8 +1619,8 @@ __device__ __forceinline__ void mma_direct(DftWgSmem<CH, false>& sm, int wave, i
 
 // The exact peak of one window pair whose rows are in `rows`; `next` is called
 // when they and most registers are free again, to load the following pair's.
-// Gives the four window sums, the number of candidates and, but for a flat window or
-// one with too many of them (DFT_MANY), the exact sum of R T at the peak and the
+// Gives the four window sums, the number of candidates (DFT_MANY: the first N, and
+// no peak) and, but for a flat window, the exact sum of R T at the peak and the
 // peak's place 64 a + b.
 enum { DFT_PEAK, DFT_FLAT, DFT_MANY };
 template <int CH, bool FULL, class Next>
@@ -1636,6 +1636,7 @@ __device__ __forceinline__ int fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int w
     const uint8_t* etrows = erows + Sm::ROWS * Sm::RP;
     dft_window(sm, wave, lane, N, rows, sums);
     const DftNorms norm(sums, NN);
+    many = 0;
     if (norm.flat()) {
         next();
         return DFT_FLAT;
@@ -1828,10 +1829,6 @@ __device__ __forceinline__ int fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int w
     uint64_t mask = ((uint64_t)mw[1] << 32) | mw[0];
 
     next();
-    if constexpr (!FULL) {
-        many = dpp_sum(__popcll(mask));
-        if (many > N) return DFT_MANY;
-    }
 
     // -- exact integer correlation at the candidates: the largest, of equal ones
     //    the lowest index ------------------------------------------------------
@@ -1845,6 +1842,7 @@ __device__ __forceinline__ int fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int w
         return (32 * Nd + m) * 64 + 32 * Md + 8 * (r >> 2) + 4 * h + (r & 3);
     };
     for (unsigned long long lanes; (lanes = __ballot(mask != 0)) != 0;) {
+        if (++many > N && !FULL) return DFT_MANY;
         const int from = __builtin_ctzll(lanes), k = __builtin_amdgcn_readlane(lowest(), from);
         if (lane == from) mask &= mask - 1;
         const int kv = k >> 6, ku = k & 63, d = ku >> 2, sh = ku & 3;
@@ -2001,7 +1999,7 @@ __device__ __forceinline__ void fftcc_dft_run(DftWgSmem<CH, FULL>& sm, const Sou
                 if (ni < hi && nx.inside) rows.load(nx, N, lane);
             };
             if (cur.inside) {
-                int sums[4], many = 0, I, peak;
+                int sums[4], many, I, peak;
                 const int r = fftcc_dft_mfma_poi<CH, FULL>(sm, wave, lane, N, rows, sums, many, I, peak, next);
                 if (r == DFT_PEAK)
                     keep(i, sums, I, peak);
@@ -2009,7 +2007,7 @@ __device__ __forceinline__ void fftcc_dft_run(DftWgSmem<CH, FULL>& sm, const Sou
                     fail(i, TWDIC_FFTCC_FLAT);
                 if constexpr (!FULL) {
                     if (2 * many > N) {
-                        run = min(2 * run + 1, kDftDirectRun);
+                        run = r == DFT_MANY ? kDftDirectRun : min(2 * run + 1, kDftDirectRun);
                         direct = run + (r == DFT_MANY ? 1 : 0);
                         if (r != DFT_MANY) i = ni;
                         break;
