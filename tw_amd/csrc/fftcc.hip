@@ -1360,10 +1360,6 @@ __device__ __forceinline__ int dpp_sum(int v)
 {
     return wave_reduce_dpp(v, [](int x, int y) { return x + y; });
 }
-__device__ __forceinline__ int dpp_min(int v)
-{
-    return wave_reduce_dpp(v, [](int x, int y) { return min(x, y); });
-}
 __device__ __forceinline__ float dpp_max(float v)
 {
     return __int_as_float(wave_reduce_dpp(__float_as_int(v), [](int x, int y) {
@@ -1643,11 +1639,19 @@ __device__ __forceinline__ int fftcc_dft_mfma_poi(DftWgSmem<CH, FULL>& sm, int w
     }
     const h2v oa = {(_Float16)(1024 + norm.a), (_Float16)(1024 + norm.a)};
     const h2v ob = {(_Float16)(1024 + norm.b), (_Float16)(1024 + norm.b)};
-    // the tolerance's factor 1.25 over the bound dwarfs the FP32 rounding here
-    const float rho = __builtin_amdgcn_sqrtf((float)norm.r2) * __builtin_amdgcn_sqrtf((float)norm.t2);
-    const float s = ldexpf(1.0f, 14 - __builtin_amdgcn_frexp_expf((float)NN * rho));   // s N^2 rho in [2^13, 2^14)
-    const float bound = FULL ? (float)kDftBound : (float)(kDftBoundN / 4096.0) * (float)NN;
-    const float tol = 2.5f / 65536.f * bound * rho * s;                          // in C^ units (s 2^-16 N^2 C)
+    // s: a power of two, s N^2 ||r|| ||t|| in [2^13, 2^14); the tolerance in C^ units
+    // (s 2^-16 N^2 C).  Below N = 64 in FP32, whose rounding the factor 1.25 over the
+    // bound dwarfs (in FP64 0.534 -> 0.543 ms for 155k POIs at N = 40)
+    float s, tol;
+    if constexpr (FULL) {
+        const double rho = sqrt((double)norm.r2 * (double)norm.t2);
+        s = ldexpf(1.0f, 14 - __builtin_amdgcn_frexp_exp(4096.0 * rho));
+        tol = (float)(2.0 * 1.25 * kDftBound * rho * (double)s / 65536.0);
+    } else {
+        const float rho = __builtin_amdgcn_sqrtf((float)norm.r2) * __builtin_amdgcn_sqrtf((float)norm.t2);
+        s = ldexpf(1.0f, 14 - __builtin_amdgcn_frexp_expf((float)NN * rho));
+        tol = 2.5f / 65536.f * (float)(kDftBoundN / 4096.0) * (float)NN * rho * s;
+    }
     wave_lds_sync();
 
     const int wave_f = FULL ? wave : 0;
