@@ -470,7 +470,11 @@ __device__ __forceinline__ void kahan_pixel(float ks[8], float kc[8], float T, u
 // after row i: Abel's summation by parts; rows that are STEP apart scale it).  S runs on from strip to strip;
 // what it held when a strip began is taken out again (a1, a2 below).  Where T
 // is integer-valued every term is an integer below 2^53, so these sums stay
-// exact there, as direct ones would be.
+// exact there, as direct ones would be.  Elsewhere the running sums are up to
+// twice as large as the direct ones and take two operations per pixel for the
+// direct one, so their rounding is bounded by four times the direct sums'; for
+// subsets of 21x21 to 121x121 the update then differs from the exact one by less
+// than a thousandth of the FP32 rounding that dp gets.
 //
 // The bicubic passes over the row polynomials (ROLL) also keep the four rows
 // of the current cell in registers: in a column the next pixel's cell is the
@@ -737,8 +741,9 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
                 // direct cells, whole wavefronts: two rows per trip, as a lone wavefront
                 // waits for each one's loads (9,409 POIs: 1 % strain 0.138 -> 0.125 ms, POIs
                 // astray 1.03 -> 0.92; four rows 0.16 and 1.08); with halves, whose
-                // wavefronts hide it, one (two: 1.20 -> 1.27 ms for 157k POIs)
-                constexpr int U = ROWS && !INT && L == 64 ? 2 : 1;
+                // wavefronts hide it, one (two: 1.20 -> 1.27 ms for 157k POIs); one, too, of
+                // lut_cubic's, which the compiler finds too long to repeat
+                constexpr int U = ROWS && INTERP != TWDIC_INTERP_LUT && !INT && L == 64 ? 2 : 1;
 #pragma unroll U
                 for (int r = 0; r < full; ++r) {
                     pixel(cx, cy, e.dx, dy, go, so);
