@@ -900,6 +900,9 @@ __device__ __forceinline__ void icgn_poi_t(const IcgnParams& P, int poi, int lan
     if ((lane & (L - 1)) == 0) {
         float Pp[6];
         params_of(Wm, Pp);
+        // the places anew: kept from the loads of u and v on, they spilled (95 MB of
+        // a 157k-POI launch's traffic)
+        if constexpr (L == 32) asm volatile("" : "+v"(poi));
         P.u[poi] = Pp[0];
         P.v[poi] = Pp[3];
         if (P.p6) {
