@@ -270,7 +270,9 @@ twdic_status twdic_strain_ls(twdic_ctx* ctx, const float* d_field, int nx, int n
  * (Rx, Ry) and target (Tx, Ty, Txy), ROI-relative row-major fp32; the target
  * bicubic LUT, [roi_h][roi_w][16] fp32 with element 4k+l multiplying y^k x^l
  * (same order as the CPU LUT, TW_utils.cpp:673-688; the last ROI row and
- * column are zero).  Target buffers are (re)computed by twdic_precompute_target. */
+ * column are zero).  Target buffers are (re)computed by twdic_precompute_target.
+ * In the LUT and B-spline modes the LUT is the one of the target IC-GN last ran
+ * on, and IC-GN reads it once it has been handed out. */
 enum { TWDIC_BUF_RX = 0, TWDIC_BUF_RY = 1, TWDIC_BUF_TX = 2, TWDIC_BUF_TY = 3,
        TWDIC_BUF_TXY = 4, TWDIC_BUF_LUT = 5, TWDIC_BUF_REF = 6, TWDIC_BUF_TAR = 7 };
 twdic_status twdic_get_buffer(twdic_ctx* ctx, int which, void** d_ptr, size_t* bytes);

@@ -1182,8 +1182,8 @@ __global__ __launch_bounds__(64) void k_batch_fftcc_mma(const PairDesc* __restri
 // keeps rows b >= N from being candidates.  N <= 48 needs three K chunks instead
 // of four (112 MFMAs instead of 144) and fits 168 registers, so twelve wavefronts,
 // three per SIMD, hide each other's chains of dependent MFMAs and conversions,
-// which bound the engine: .48 ms for 155k POIs at N = 40, .71 ms at N = 56 and .73 ms
-// at N = 64 (two wavefronts per SIMD).
+// which bound the engine: .48 ms for 157k POIs at N = 40, .71 ms at N = 56 and .73 ms
+// at N = 64 (two wavefronts per SIMD; on a slower card up to 8 % more).
 // ===========================================================================
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
@@ -1245,7 +1245,7 @@ __device__ __forceinline__ DftItem dft_item(const FftccParams& p, int poi)
 // A window pair's rows in flight, CH lanes to a row, 16 bytes each, so that a
 // load instruction touches the lines of 64 / CH rows (with a lane per row the
 // lines of 64, four times over: the loads of eight wavefronts queued up in the
-// address unit, 0.81 ms per 157,609 POIs at N = 64 against 0.74 ms).  Lane l
+// address unit, 0.81 ms for 157k POIs at N = 64 against 0.73 ms).  Lane l
 // holds piece l % CH of the rows k (64 / CH) + l / CH.  A row's last piece ends
 // with the row, so nothing outside it is read; words() moves it to its place.
 template <int CH, bool FULL>
@@ -1946,7 +1946,7 @@ __device__ __forceinline__ int dft_range_index()
 // cycles per POI 4,100 went by waiting for its place and rows), and the
 // outputs, some 100 FP64 instructions, are formed for KEPT items at a time, a lane
 // each, instead of by one lane per item.  With the rows' loads in DftRows:
-// 0.81 -> 0.73 ms for 155k POIs at N = 64, 0.53 -> 0.48 ms at N = 40.  src.item(i) is the window pair of item i, src.params(i)
+// 0.81 -> 0.73 ms for 157k POIs at N = 64, 0.53 -> 0.48 ms at N = 40.  src.item(i) is the window pair of item i, src.params(i)
 // its outputs, src.poi(i) their index.
 template <int CH, bool FULL, class Source>
 __device__ __forceinline__ void fftcc_dft_run(DftWgSmem<CH, FULL>& sm, const Source& src, int N, int lo, int hi)

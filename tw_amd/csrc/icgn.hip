@@ -486,10 +486,10 @@ __device__ __forceinline__ void kahan_pixel(float ks[8], float kc[8], float T, u
 // unset a pixel's two entries are loaded directly.
 // Their integer pass (GROUP) issues the loads of eight rows together: with one
 // row's at a time a lone wavefront waited for memory once a row, 14,000 cycles
-// for 31x31 pixels where the groups take 6,100 (the kernel 28.2 -> 24.2 us for
-// 20 POIs, 118 -> 115 us for 11k, 1.13 -> 1.11 ms for 157k); in B-spline mode,
-// whose lanes are dealt rows in turn, it is no gain (0.398 -> 0.413 ms for 28k
-// POIs).
+// for 31x31 pixels where the groups take 6,100 (the kernel by itself 28.9 -> 27.7 us
+// for 20 POIs, 115.8 -> 114.2 us for 11k, 1.126 -> 1.119 ms for 157k); in B-spline
+// mode, whose lanes are dealt rows in turn, it is no gain (0.398 -> 0.413 ms for
+// 28k POIs).
 //
 // Bound by VALU issue (a row-major walk from a table of pixel offsets: 58 VALU
 // instructions per bicubic pixel, 12 of them mixed-precision ones of 1.5 slots,
