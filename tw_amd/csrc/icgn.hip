@@ -520,7 +520,7 @@ __device__ __forceinline__ bool subset_loop(const IcgnParams& P, int px, int py,
     const int sx0 = P.sx0, sy0 = P.sy0, rw = P.rw, rh = P.rh;
     const TargetBuf tb = target_buf(P);
     const __amdgpu_buffer_rsrc_t g2r =
-        __builtin_amdgcn_make_buffer_rsrc((void*)P.g2, (short)0, 4 * rw * rh, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)P.g2, (short)0, (int)(4u * (uint32_t)rw * (uint32_t)rh), 0x00020000);
     const RowPolyBuf rb = ROWS ? row_poly_buf(P) : RowPolyBuf{};
     const float fpx = (float)px, fpy = (float)py;
     double st = 0.0, stt = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0, b0 = 0.0, b1 = 0.0, b2 = 0.0;

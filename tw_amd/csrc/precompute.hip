@@ -423,7 +423,8 @@ __device__ __forceinline__ void ref_moments(const IcgnParams& P, int nstrips, in
     const __amdgpu_buffer_rsrc_t imgr =
         __builtin_amdgcn_make_buffer_rsrc((void*)P.ref, (short)0, P.stride * (P.sy0 + P.rh), 0x00020000);
     const __amdgpu_buffer_rsrc_t g2r =
-        __builtin_amdgcn_make_buffer_rsrc((void*)P.g2, (short)0, 4 * P.rw * P.rh, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)P.g2, (short)0, (int)(4u * (uint32_t)P.rw * (uint32_t)P.rh),
+                                          0x00020000);
     const uint32_t gcorner = 4u * (uint32_t)((py - P.Sy - P.sy0) * P.rw + (px - P.Sx - P.sx0));
     double m[kMoments];
 #pragma unroll

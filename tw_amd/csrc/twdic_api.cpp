@@ -323,7 +323,12 @@ twdic_status use_lut(twdic_ctx* c)
         c->tar_pre_valid = c->tar_pre_valid || c->tar_rp_valid;
         // never built: nothing reads it, and no graph will
         if (c->d_rp && !c->rp_built && !stream_capturing(c)) {
-            TW_HIP(c, hipFree(c->d_rp));
+            // in the mode that disturbs no other thread's capture
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            const hipError_t e = hipFree(c->d_rp);
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            TW_HIP(c, e);
             c->d_rp = nullptr;
         }
     }
